@@ -139,8 +139,8 @@ def same_sample_precision(eng, bas, prec):
 
 def kernel_name(key):
     if key[0] == "shell":
-        _, lu, ll, clb, red = key
-        return f"k_eri_shell{'_red' if red else ''}<{lu}, {ll}, {clb}>"
+        _, lu, ll, p, _ = key
+        return f"k_eri_quartet<{lu}, {ll}, {p - 1}>"
     _, a, b = key
     return f"k_eri_class<{a}, {b}>" if a < 5 else "k_eri_generic"
 
@@ -162,8 +162,8 @@ def roofline_eri(res):
     Schwarz phase run side by side on the library's five streams and are
     timed together (HIP events around the fork and join on the library's
     stream).  Algorithmic FP64 flops (Boys values and R table once per
-    primitive quartet, Hermite contractions per component over its nonzero
-    Hermite coefficients, as counted by the library) over the phase time; a
+    primitive quartet, one multiply-add per scaled Hermite term, as counted by
+    the library) over the phase time; a
     "launch" is one phase's set of buckets."""
     st = res["eri_stats"]
     flops = sum(v["flops"] for v in st.values())
@@ -179,8 +179,8 @@ def roofline_eri(res):
             break
         traffic += t * d["launches"]
     return {"bound": "fp64-valu",
-            "kernel": "k_eri_shell<LU, LL, B> / k_eri_shell_red<LU, LL, B> (the buckets of a "
-                      "Schwarz phase, side by side on five streams)",
+            "kernel": "k_eri_quartet<LU, LL, PASS> (the buckets of a Schwarz phase, side by "
+                      "side on five streams)",
             "achieved": achieved, "peak": PEAK_FP64, "unit": "TFLOP/s",
             "frac": achieved / PEAK_FP64,
             "traffic": traffic / max(1, nset) if traffic is not None else None,

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64) void k_primpairs(BasisE B, const int *pair_i, c
     for (int e0 = 0; e0 < cap; e0 += 64) {
         int e = e0 + lane;
         bool keep = false;
-        double p = 0, Pc[3] = {0, 0, 0}, coef = 0;
+        double p = 0, Pc[3] = {0, 0, 0}, coef = 0, ea = 0, eb = 0;
         int a = 0, b = 0;
         if (e < cap) {
             a = e / ngk;
@@ -117,6 +117,8 @@ __global__ __launch_bounds__(64) void k_primpairs(BasisE B, const int *pair_i, c
                     keep = true;
                     for (int d = 0; d < 3; d++) Pc[d] = (al * A[d] + be * Bc[d]) * pinv;
                     coef = (di[a] * dk[b]) * fk;
+                    ea = al;
+                    eb = be;
                 }
             }
         }
@@ -131,6 +133,8 @@ __global__ __launch_bounds__(64) void k_primpairs(BasisE B, const int *pair_i, c
         pp.Py[at] = Pc[1];
         pp.Pz[at] = Pc[2];
         pp.c[at] = coef;
+        pp.al[at] = ea;
+        pp.be[at] = eb;
         // Hermite expansion, summed over the r^2 variants
         double ip2 = 0.5 / p;
         double E1[3][kEA][kEA][kET];
@@ -430,6 +434,8 @@ static PP pp_view(zv_context *c)
     pp.Py = base + 3 * T;
     pp.Pz = base + 4 * T;
     pp.c = base + 5 * T;
+    pp.al = base + 6 * T;
+    pp.be = base + 7 * T;
     pp.E = (double *)c->b_ppE.p;
     char *m = (char *)c->b_ppcnt.p;
     int64_t *d_off = (int64_t *)m;
@@ -448,9 +454,9 @@ static int ensure_primpairs(zv_context *c, PP &pp)
     int np = c->npair;
     ZV_CHECK(ensure_boys_table(c));
     pp.btab = (const double *)c->b_btab.p;
-    // layout inside b_pp: 6 planes of pp_total doubles; b_ppE: e_total doubles;
+    // layout inside b_pp: 8 planes of pp_total doubles; b_ppE: e_total doubles;
     // b_ppcnt: cnt[np] ints, off[np], eoff[np] int64, cap[np], L[np] ints
-    ZV_CHECK(zv_ensure(c, c->b_pp, sizeof(double) * 6 * (size_t)c->pp_total));
+    ZV_CHECK(zv_ensure(c, c->b_pp, sizeof(double) * 8 * (size_t)c->pp_total));
     ZV_CHECK(zv_ensure(c, c->b_ppE, sizeof(double) * (size_t)c->e_total));
     size_t meta = sizeof(int) * np * 3 + sizeof(int64_t) * np * 2 + 64;
     ZV_CHECK(zv_ensure(c, c->b_ppcnt, meta));
@@ -462,6 +468,8 @@ static int ensure_primpairs(zv_context *c, PP &pp)
     pp.Py = base + 3 * T;
     pp.Pz = base + 4 * T;
     pp.c = base + 5 * T;
+    pp.al = base + 6 * T;
+    pp.be = base + 7 * T;
     pp.E = (double *)c->b_ppE.p;
     char *m = (char *)c->b_ppcnt.p;
     int64_t *d_off = (int64_t *)m;

@@ -1,34 +1,51 @@
-// Shell-blocked analytic ERIs: the reference's gauss_ijkl
+// Shell-quartet analytic ERIs: the reference's gauss_ijkl
 // (src/gauss_ijkl.F90:51-154) for all Cartesian components of a shell
 // quartet at once, inside its Schwarz driver (src/two_e_slater.F90:230-273).
 //
 // The AOs of one shell (e.g. the six 3D functions of an atom) share center,
 // Gaussian exponents and contraction coefficients, so all AO pairs of a
 // shell pair share the primitive-pair data p, P, c_ab and the reference's
-// cuts; only the Hermite coefficients E differ.  For a shell quartet (U|L)
-// one primitive quartet (a, c) needs one Boys evaluation and one R table:
+// cuts; only the Hermite coefficients E differ, and they depend on the
+// primitive pair through three numbers only: 1/2p, x = beta/p and 1 - x
+// (P - A = x (B - A), P - B = -(1 - x)(B - A)).  For a shell pair of order L
 //
-//   (u|l) += c_a c_c pref(a,c) sum_hu E^u_hu(a) X^l_hu(a,c),
-//   X^l_hu(a,c) = sum_hl (-1)^(t+u+v of hl) E^l_hl(c) R_{hu+hl}(a,c)
+//   E^u_h(a) = sum_{n, m} G^u_{nm,h} sigma_nm(a),
+//   sigma_nm = (1/2p)^n x^m (1 - x)^(L-n-m),  0 <= n <= L, 0 <= m <= L - n,
 //
-// for every component u of U and l of L.
+// with G^u fixed by the AOs' powers and B - A.  A fit of 20 Gaussians per AO
+// gives up to 160,000 primitive quartets (a, c) per shell quartet, so the
+// contraction over them runs first, on the sigma alone:
 //
-// Work item of one wavefront: a shell quartet, a range of lane-side
-// components, a range of uniform-side components (up to 64 in the reduction
-// mode, at most kDirectMaxU in the direct mode) and a slice of the
-// uniform-side primitive pairs.  Lanes own lane-side primitive pairs (their
-// E in registers, reloaded per lane component); the uniform primitive pairs
-// are walked in the inner loop through an AoS copy ([a][component][h]) read
-// with scalar loads, so each uniform E value is one SGPR operand shared by
-// the 64 lanes.  Per-lane sums over the uniform components live in LDS;
-// each item writes its partial sums, and one scatter kernel adds the slices,
-// applies the Schwarz test per component quartet and writes triangle order.
+//   Z[nm, n'm', r] = sum_a sum_c w_nm(a) w'_n'm'(c) R_r(a, c) / sqrt(p + q),
+//   (u|l) = C sum G^u_{nm,hu} (-1)^|hl| G^l_{n'm',hl} Z[nm, n'm', hu + hl],
 //
-// E^l of one lane component is nonzero only on a pattern of Hermite indices
-// fixed by the AOs' Cartesian powers (HermPatterns); the classes listed in
-// kShellSparse read the pattern's rows of a compacted copy of E and run the
-// X contraction over them only, the same terms in the same order minus
-// exact zeros.
+// w = c_ab sigma / p, C the reference's 2 pi^(5/2).  Per primitive quartet
+// there is one Boys evaluation, one R table and at most one multiply-add per
+// (nm, r) with |r| <= n + L_l, for any number of components: a p x p | p x p
+// quartet (81 integrals) costs the 35-entry R table and 105 multiply-adds.
+// Powers of x and 1 - x are kept apart (every sigma of the same n has total
+// degree L - n, lower degrees raised by (x + 1 - x)^k), so the expansion adds
+// no cancellation to that of E itself.
+//
+// A wavefront owns a work item (a shell quartet or a slice of it) and runs
+// 4 uniform-side times 16 lane-side primitive pairs per step: lane
+// a_local * 16 + c_local.  The sum over a is v_mfma_f64_4x4x4 with R as the A
+// operand (its rows the 16 c in four blocks of 4, its inner index the 4 a)
+// and the weights as B (columns: 4 of the sigma), which keeps 4 sigma x 16 c
+// sums in one register pair per lane; rows that need one sigma (the top
+// order) take a plain multiply-add, which costs a third of the matrix
+// instruction.  After the last step of a chunk of 16 c, the accumulators are
+// the B operand of the same instruction with the lane weights as A, which
+// sums over c; the four blocks are folded with row rotations and added to Z
+// in LDS.  Z is transformed to the components once per item.
+//
+// Bound: FP64 issue.  The matrix instruction and FP64 vector instructions
+// share the pipe (alternating them adds their times: 16.4 and 5.4 cycles), so
+// the matrix form buys registers, not flops; there is no memory access in the
+// loop but the next step's rows.  Before, each lane contracted R with the E of
+// its components (passes of 1-4 components, Boys and R redone per pass, lane
+// data reloaded per uniform pair): kernel time of the 110-AO random molecule
+// 0.55 -> 0.27 s, of a 128-AO hydrocarbon 1.20 -> 0.42 s.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -36,6 +53,7 @@
 #include <numeric>
 #include <thread>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "eri_device.h"
@@ -45,555 +63,559 @@ using namespace zveri;
 
 namespace {
 
-struct SPD {
-    const int *comp;      // AO pair index of each component
-    const int *coff;      // first component of each shell pair (nsp + 1)
-    const int64_t *puoff; // AoS primitive data offset (doubles) per shell pair
-    const int64_t *euoff; // AoS E offset (doubles) per shell pair
-    const double *pu;     // [a][8]: p, 1/p, Px, Py, Pz, c, 0, 0
-    const double *eu;     // [a][component][h]  (scalar reads, direct mode)
-    const double *eu2;    // [a][h][component]  (lane-per-component reads, reduction mode)
-    const int *cpat;      // per component: Hermite pattern index | nonzero count << 8
-    const double *ec;     // lane-side E: the pattern's nonzero rows, offsets and stride of E
-};
-
-struct ShellItem {
-    int su, sl;   // shell pairs on the uniform and the lane side
-    int a0, a1;   // uniform primitive-pair slice
-    int cl0, cl1; // lane-side components
-    int cu0, nu;  // uniform-side components cu0 .. cu0 + nu - 1
-    int64_t part; // partial sums of this item: [nu][cl1 - cl0]
-};
-
-struct ShellGroup {
-    int su, sl, cu0, nu, cl0, nl, ns, pad; // ns slices of [nu][nl] partials from part on
-    int64_t part;
-};
-
-// Uniform components of a direct-mode item: the planner sends ranges of
-// kDirectMaxU + 1 or more uniform components to the reduction mode, so a
-// direct item holds a whole shell pair of at most this many components or
-// the short tail of a longer one (checked on the host before each launch).
-// The direct kernel's LDS accumulators are sized for it.
-constexpr int kDirectMaxU = 3;
-
-// AoS copies of a shell pair's primitive data and E (one block per shell pair)
-__global__ __launch_bounds__(256) void k_shellpairs(PP pp, SPD sd, double *pu, double *eu,
-                                                    double *eu2)
+// ------------------------------------------------------------------ sigma
+constexpr int nsig(int L) { return (L + 1) * (L + 2) / 2; }
+// sigma index s: n descending, m ascending, so that "n >= nmin" is a prefix
+constexpr int sig_depth(int s)
 {
-    const int s = blockIdx.x;
-    const int c0 = sd.coff[s], nc = sd.coff[s + 1] - c0;
-    const int rep = sd.comp[c0];
-    const int np = pp.cnt[rep];
-    const int H = hcount(pp.L[rep]);
-    const int64_t off = pp.off[rep];
-    double *dp = pu + sd.puoff[s];
-    for (int t = threadIdx.x; t < np * 8; t += blockDim.x) {
-        const int64_t at = off + (t >> 3);
-        double v = 0.0;
-        switch (t & 7) {
-        case 0: v = pp.p[at]; break;
-        case 1: v = pp.ip[at]; break;
-        case 2: v = pp.Px[at]; break;
-        case 3: v = pp.Py[at]; break;
-        case 4: v = pp.Pz[at]; break;
-        case 5: v = pp.c[at]; break;
-        default: break;
+    int d = 0;
+    while ((d + 1) * (d + 2) / 2 <= s) d++;
+    return d;
+}
+constexpr int sig_n(int L, int s) { return L - sig_depth(s); }
+constexpr int sig_index(int L, int n, int m) { return (L - n) * (L - n + 1) / 2 + m; }
+// sigmas with n >= nmin
+constexpr int sig_prefix(int L, int nmin)
+{
+    if (nmin <= 0) return nsig(L);
+    if (nmin > L) return 0;
+    return (L - nmin + 1) * (L - nmin + 2) / 2;
+}
+constexpr int hco(int L) { return L < 0 ? 0 : hcount(L); }
+constexpr int horder(int h)
+{
+    int s = 0;
+    while (hcount(s) <= h) s++;
+    return s;
+}
+
+// Row of one primitive pair: p, Px, Py, Pz, then its weights in sigma order,
+// zero-padded to whole groups of four (one B operand each); an even length
+// keeps rows 16-byte aligned.
+constexpr int kRow[5] = {6, 8, 12, 16, 20};
+constexpr int ngroup(int L) { return (nsig(L) + 3) / 4; }
+// primitive pairs of a shell pair are padded with zero-weight rows to
+// multiples of kLaneC, the lane-side chunk; kStepA per step on the uniform side
+constexpr int kLaneC = 16, kStepA = 4;
+
+// Expansion entries j = (sigma, h) of order L: the h with s = |h| <= n and
+// k = n - s, s + 2k <= L.
+constexpr int kNgMax = 98;
+struct GTable {
+    int n = 0;
+    int off[15] = {}, h0[15] = {}; // per sigma: first entry, first h
+    int sig[kNgMax] = {}, h[kNgMax] = {};
+};
+constexpr GTable make_gtable(int L)
+{
+    GTable g;
+    for (int s = 0; s < nsig(L); s++) {
+        const int n = sig_n(L, s);
+        const int lo = 2 * n - L > 0 ? 2 * n - L : 0;
+        g.off[s] = g.n;
+        g.h0[s] = hco(lo - 1);
+        for (int h = hco(lo - 1); h < hco(n); h++) {
+            g.sig[g.n] = s;
+            g.h[g.n] = h;
+            g.n++;
         }
-        dp[t] = v;
     }
-    double *de = eu + sd.euoff[s], *de2 = eu2 + sd.euoff[s];
-    const int64_t tot = (int64_t)np * nc * H;
-    for (int64_t t = threadIdx.x; t < tot; t += blockDim.x) {
-        const int h = (int)(t % H);
-        const int64_t r = t / H;
-        const int cu = (int)(r % nc);
-        const int a = (int)(r / nc);
-        const int P = sd.comp[c0 + cu];
-        const double v = pp.E[pp.eoff[P] + (int64_t)h * pp.cap[P] + a];
-        de[t] = v;
-        de2[((int64_t)a * H + h) * nc + cu] = v;
-    }
+    return g;
+}
+struct GTables {
+    GTable t[5];
+    constexpr GTables() : t() { for (int L = 0; L < 5; L++) t[L] = make_gtable(L); }
+};
+constexpr GTables kG{};
+static_assert(kG.t[4].n == kNgMax, "expansion entries");
+
+// ------------------------------------------------------------------ passes
+// A class (LU, LL), LU <= LL, whose accumulators and R table do not fit in
+// the registers (256 of each kind per wave) runs in passes, each a kernel of its own over the same
+// primitive quartets: the rows r of order rho0..rho1 and the sigma groups
+// [g0, g1).  The passes of a quartet write partial sums that the scatter adds.
+struct Pass {
+    int rho0, rho1, g0, g1;
+};
+constexpr int kPassMax = 4;
+constexpr int npass(int LU, int LL)
+{
+    if (LU == 4) return 4;
+    if (LU == 3) return 2;
+    return 1;
+}
+constexpr Pass pass_of(int LU, int LL, int p)
+{
+    const int ng = ngroup(LU);
+    if (LU == 4)
+        return p == 0 ? Pass{0, 5, 0, 2} : p == 1 ? Pass{0, 5, 2, 4} : p == 2 ? Pass{6, 7, 0, 4}
+                                                                           : Pass{8, 8, 0, 1};
+    if (LU == 3 && LL == 3) return p == 0 ? Pass{0, 6, 0, 1} : Pass{0, 4, 1, 3};
+    if (LU == 3) return p == 0 ? Pass{0, 5, 0, 3} : Pass{6, 7, 0, 1};
+    return Pass{0, LU + LL, 0, ng};
 }
 
-// Lane-side E without its structural zeros: per component (AO pair), the
-// rows of the nonzero Hermite indices of its pattern, in ascending order, at
-// the pair's E offset with the same row stride (one block per component).
-__global__ __launch_bounds__(256) void k_compact_e(PP pp, SPD sd, double *ec)
+// Accumulators and Z values of a pass.  A (row, group) entry with one
+// needed sigma is one per-lane sum (sigma >= 0), otherwise one matrix tile.
+// Needed are the sigma with n >= rho - LL (the lane side has |hl| <= LL), and
+// with them the lane sigma with n' >= rho - n.
+constexpr int kAccMax = 160, kZMax = 400;
+struct Slots {
+    int n = 0;
+    int r[kAccMax] = {}, g[kAccMax] = {}, sig[kAccMax] = {}; // sig -1: matrix tile
+    int z0[kAccMax] = {}, nz[kAccMax] = {};                  // Z tiles: first, count (groups g')
+    int ztot = 0;
+    int zslot[kZMax] = {}, zg[kZMax] = {};
+};
+constexpr Slots make_slots(int LU, int LL, Pass ps)
 {
-    const int q = blockIdx.x;
-    const int P = sd.comp[q];
-    const int L = pp.L[P];
-    if (L > ZV_LMAX_T) return;
-    const int pid = sd.cpat[q] & 0xff, nz = sd.cpat[q] >> 8;
-    const int n = pp.cnt[P], cap = pp.cap[P];
-    const int64_t eo = pp.eoff[P];
-    for (int t = threadIdx.x; t < nz * n; t += blockDim.x) {
-        const int k = t / n, a = t - k * n;
-        ec[eo + (int64_t)k * cap + a] = pp.E[eo + (int64_t)kHP.h[L][pid][k] * cap + a];
-    }
-}
-
-// Calls f(std::integral_constant<int, p>) for the runtime pattern index p of
-// order LL (a chain of uniform compares), so the body sees the pattern's
-// nonzero Hermite indices as constants.
-template <int LL, int I = 0, class F> __device__ __forceinline__ void pat_dispatch(int p, F &&f)
-{
-    if constexpr (I < kHP.n[LL]) {
-        if (p == I)
-            f(std::integral_constant<int, I>{});
-        else
-            pat_dispatch<LL, I + 1>(p, f);
-    }
-}
-
-// X[hu] over one lane component: the sum over the nonzero Hermite indices
-// hl of its pattern pat, in ascending order, of (-1)^(t+u+v of hl) sc(E[k])
-// R_{hu+hl}, E[k] the k-th nonzero coefficient; with INIT the first term
-// sets X (hl = 0, even), else every term is added.  The skipped terms are
-// exact zeros, so X equals the sum over all indices.
-template <int LU, int LL, bool INIT, int NZ, class Sc>
-__device__ __forceinline__ void lane_contract(int pat, const double (&E)[NZ], const double *R,
-                                              double (&X)[hcount(LU)], Sc sc)
-{
-    constexpr int HU = hcount(LU);
-    auto term = [&](int k, int hl) {
-        const double ek = sc(E[k]);
-        const double e = ((kH.t[hl] + kH.u[hl] + kH.v[hl]) & 1) ? -ek : ek;
-#pragma unroll
-        for (int hu = 0; hu < HU; hu++) {
-            const double r =
-                R[hidx(kH.t[hu] + kH.t[hl], kH.u[hu] + kH.u[hl], kH.v[hu] + kH.v[hl])];
-            X[hu] = INIT && k == 0 ? e * r : fma(e, r, X[hu]);
+    Slots o;
+    for (int r = hco(ps.rho0 - 1); r < hco(ps.rho1); r++) {
+        const int rho = horder(r);
+        const int need = sig_prefix(LU, rho - LL);
+        for (int g = ps.g0; g < ps.g1; g++) {
+            if (need - 4 * g <= 0) break;
+            o.r[o.n] = r;
+            o.g[o.n] = g;
+            o.sig[o.n] = need - 4 * g == 1 ? 4 * g : -1;
+            const int np = sig_prefix(LL, rho - sig_n(LU, 4 * g));
+            o.z0[o.n] = o.ztot;
+            o.nz[o.n] = (np + 3) / 4;
+            for (int gp = 0; gp < o.nz[o.n]; gp++) {
+                o.zslot[o.ztot] = o.n;
+                o.zg[o.ztot] = gp;
+                o.ztot++;
+            }
+            o.n++;
         }
-    };
-    pat_dispatch<LL>(pat, [&](auto PI) {
-        constexpr int P = decltype(PI)::value;
-        static_assert(kHP.h[LL][P][0] == 0, "pattern order");
-#pragma unroll
-        for (int k = 0; k < kHP.nz[LL][P]; k++) term(k, kHP.h[LL][P][k]);
+    }
+    return o;
+}
+template <int LU, int LL, int PASS> struct Cls {
+    static constexpr Pass ps = pass_of(LU, LL, PASS);
+    static constexpr Slots sl = make_slots(LU, LL, ps);
+    static constexpr int zwords = (sl.ztot + 3) / 4 * 64; // Z tiles in LDS, 4 x 16 values a row
+};
+
+// Position in a pass's Z area of (sigma, sigma', r), -1 if another pass has it
+int z_position(int LU, const Slots &sl, int s, int sp, int r)
+{
+    for (int i = 0; i < sl.n; i++) {
+        if (sl.r[i] != r || sl.g[i] != s / 4) continue;
+        if (sp / 4 >= sl.nz[i]) return -1;
+        const int z = sl.z0[i] + sp / 4;
+        return z / 4 * 64 + (s & 3) + 4 * (z & 3) + 16 * (sp & 3);
+    }
+    return -1;
+}
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): the hot
+// loops are written out by the front end (indices are constants before any
+// optimizer pass runs; left to the loop unroller the file takes ten times
+// longer to compile)
+template <class F, int... I>
+__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F> __device__ __forceinline__ void static_for(F &&f)
+{
+    static_for_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// The steps of hermite_R (eri_device.h) for order L, in place and in the same
+// order: R[dst] = x_axis R[a] + coef R[b] (b -1: no second term), or, for
+// axis 3, the seed R[0] = scale (-2 alpha)^n F_n with n = a.
+struct RStep {
+    short dst, a, b;
+    signed char coef, axis;
+};
+template <int L> struct RProgram {
+    static constexpr int N = (L + 1) * (L + 2) * (L + 3) * (L + 4) / 24;
+    RStep s[N] = {};
+    constexpr RProgram()
+    {
+        int at = 0;
+        for (int n = L; n >= 0; n--) {
+            for (int o = L - n; o >= 1; o--)
+                for (int t = o; t >= 0; t--)
+                    for (int u = o - t; u >= 0; u--) {
+                        const int v = o - t - u;
+                        const int ax = t > 0 ? 0 : u > 0 ? 1 : 2, k = t > 0 ? t : u > 0 ? u : v;
+                        const int dt = ax == 0, du = ax == 1, dv = ax == 2;
+                        RStep &e = s[at++];
+                        e.dst = (short)hidx(t, u, v);
+                        e.a = (short)hidx(t - dt, u - du, v - dv);
+                        e.b = k > 1 ? (short)hidx(t - 2 * dt, u - 2 * du, v - 2 * dv) : (short)-1;
+                        e.coef = (signed char)(k - 1);
+                        e.axis = (signed char)ax;
+                    }
+            s[at++] = RStep{0, (short)n, -1, 0, 3};
+        }
+    }
+};
+template <int L> struct RProg {
+    static constexpr RProgram<L> p{};
+};
+
+template <int L>
+__device__ __forceinline__ void hermite_table(double alpha, double scale, double X, double Y,
+                                              double Z, const double *F, double *R)
+{
+    const double m2a = -2.0 * alpha;
+    double sd[L + 1];
+    sd[0] = scale;
+    static_for<L>([&](auto i) { sd[i + 1] = sd[i] * m2a; });
+    static_for<RProgram<L>::N>([&](auto i) {
+        constexpr RStep e = RProg<L>::p.s[i];
+        if constexpr (e.axis == 3) {
+            R[0] = sd[e.a] * F[e.a];
+        } else {
+            const double x = e.axis == 0 ? X : e.axis == 1 ? Y : Z;
+            if constexpr (e.b < 0)
+                R[e.dst] = x * R[e.a];
+            else
+                R[e.dst] = fma((double)e.coef, R[e.b], x * R[e.a]);
+        }
     });
 }
 
-// The uniform-side arrays and the output are separate restrict arguments so
-// the compiler may read the former through the scalar cache (no store of
-// the kernel can reach them).  CLB lane-side components are processed per
-// pass: they share the Boys values and the R table of a primitive quartet.
+struct SPD {
+    const int *comp;       // AO pair index of each component
+    const int *coff;       // first component of each shell pair (nsp + 1)
+    const int *np;         // kept primitive pairs of each shell pair
+    const int64_t *roff;   // rows of each shell pair
+    const int64_t *goff;   // expansion tables of each shell pair
+    const double *rows;    // [primitive pair][kRow[L]]
+    const double *gu, *gl; // [component][entry]: G, and (-1)^|h| G
+};
 
-// Direct mode (few uniform components): every lane contracts its X with the
-// E of every uniform component, scalar E operands, nu * HU FMAs per lane and
-// primitive quartet; per-lane sums over the uniform components live in LDS.
-template <int LU, int LL, int CLB, bool PFU, bool TB, bool SP>
-__global__ __launch_bounds__(64) void k_eri_shell(PP pp, SPD sd,
-                                                  const ShellItem *__restrict__ items,
-                                                  const double *__restrict__ pu_all,
-                                                  const double *__restrict__ eu_all,
-                                                  double *__restrict__ part)
+struct ShellItem {
+    int su, sl;   // uniform and lane shell pair
+    int s0, s1;   // steps of kStepA uniform primitive pairs
+    int k0, k1;   // chunks of kLaneC lane primitive pairs
+    int64_t part; // output: [ncu][ncl]
+};
+
+struct ShellGroup {
+    int su, sl, ns, pad; // ns partial results [ncu][ncl] from part on
+    int64_t part;
+};
+
+// Two-double arithmetic for the weights (setup only).  Z holds sums of both
+// signs that cancel in the transform, so the rounding of the weights shows
+// in the integrals unless every sigma of a primitive pair belongs to the
+// same p and x to the last bit.
+struct DD {
+    double h, l;
+};
+__device__ inline DD dd_norm(double a, double b)
 {
-    constexpr int HU = hcount(LU), L = LU + LL, HR = hcount(L);
-    constexpr int NZ = SP ? kHP.nzmax[LL] : hcount(LL); // lane E per component
-    __shared__ double accs[kDirectMaxU * CLB * 64]; // it.nu <= kDirectMaxU (host-checked)
-    __shared__ double lbt[TB ? kBoysSlice : 1];     // Boys Taylor table, this L
-    if constexpr (TB) boys_table_load<L>(pp.btab, lbt);
-    const int lane = threadIdx.x;
-    int vzero = 0;
-    if constexpr (PFU) asm volatile("v_mov_b32 %0, 0" : "=v"(vzero));
-    const ShellItem it = items[blockIdx.x];
-    const int ub = sd.coff[it.su], lb = sd.coff[it.sl];
-    const int ncu = sd.coff[it.su + 1] - ub;
-    const int repl = sd.comp[lb];
-    const int nl = pp.cnt[repl];
-    const int64_t ol = pp.off[repl];
-    const double *pu = pu_all + sd.puoff[it.su];
-    const double *eu = eu_all + sd.euoff[it.su] + (int64_t)it.cu0 * HU;
-    const int64_t erow = (int64_t)ncu * HU;
-    const int nlc = it.cl1 - it.cl0;
-    // the item's lane components are whole passes of CLB (host-checked)
-    for (int cl = it.cl0; cl < it.cl1; cl += CLB) {
-        int64_t el[CLB];
-        int capl[CLB], pat[CLB], nzl[CLB];
-#pragma unroll
-        for (int j = 0; j < CLB; j++) {
-            const int Pl = sd.comp[lb + cl + j];
-            el[j] = pp.eoff[Pl];
-            capl[j] = pp.cap[Pl];
-            const int cp = sd.cpat[lb + cl + j];
-            pat[j] = cp & 0xff;
-            nzl[j] = cp >> 8;
-        }
-        for (int u = 0; u < it.nu * CLB; u++) accs[u * 64 + lane] = 0.0;
-        for (int c0 = 0; c0 < nl; c0 += 64) {
-            const int c = c0 + lane;
-            const bool live = c < nl;
-            const int cc = live ? c : c0; // in-range index for idle lanes
-            const double q = pp.p[ol + cc], iq = pp.ip[ol + cc];
-            const double Qx = pp.Px[ol + cc], Qy = pp.Py[ol + cc], Qz = pp.Pz[ol + cc];
-            const double ck = live ? pp.c[ol + cc] : 0.0;
-            // the lane E of each component (SP: its nonzero ones, pattern order)
-            double El[CLB][NZ];
-#pragma unroll
-            for (int j = 0; j < CLB; j++)
-#pragma unroll
-                for (int k = 0; k < NZ; k++) {
-                    if constexpr (SP) {
-                        El[j][k] = k < nzl[j] ? sd.ec[el[j] + (int64_t)k * capl[j] + cc] : 0.0;
-                    } else {
-                        const double e = pp.E[el[j] + (int64_t)k * capl[j] + cc];
-                        El[j][k] = ((kH.t[k] + kH.u[k] + kH.v[k]) & 1) ? -e : e;
-                    }
-                }
-            // PFU: the uniform primitive pair's data (p, 1/p, P, c and the E of
-            // the item's uniform components) are loaded into vector registers
-            // one iteration ahead instead of through the scalar cache, whose
-            // latency each iteration otherwise waits for.  The opaque zero
-            // makes their addresses lane-dependent for the compiler.
-            constexpr int NUE = PFU ? kDirectMaxU * HU : 1;
-            double nU[6], nEu[NUE];
-            auto load_u = [&](int a) {
-                const double *pa = pu + (int64_t)a * 8 + vzero;
-#pragma unroll
-                for (int t = 0; t < 6; t++) nU[t] = pa[t];
-                const double *ea = eu + (int64_t)a * erow + vzero;
-#pragma unroll
-                for (int t = 0; t < NUE; t++) nEu[t] = t < it.nu * HU ? ea[t] : 0.0;
-            };
-            if constexpr (PFU) load_u(it.a0);
-            for (int a = it.a0; a < it.a1; a++) {
-                double U[6], Eu[NUE];
-                if constexpr (PFU) {
-#pragma unroll
-                    for (int t = 0; t < 6; t++) U[t] = nU[t];
-#pragma unroll
-                    for (int t = 0; t < NUE; t++) Eu[t] = nEu[t];
-                    if (a + 1 < it.a1) load_u(a + 1);
-                } else {
-                    const double *pa = pu + (int64_t)a * 8;
-#pragma unroll
-                    for (int t = 0; t < 6; t++) U[t] = pa[t];
-                }
-                const double p = U[0], ip = U[1];
-                const double X = U[2] - Qx, Y = U[3] - Qy, Z = U[4] - Qz;
-                const double s = p + q;
-                const double rs = rsqrt_pos(s), is = rs * rs;
-                const double alpha = (p * q) * is;
-                const double T = alpha * ((X * X + Y * Y) + Z * Z);
-                double F[L + 1];
-                if constexpr (TB)
-                    boys_table<L>(T, lbt, F);
-                else
-                    boys<L>(T, F);
-                double R[HR];
-                hermite_R<L>(alpha, X, Y, Z, F, R);
-                const double f = (U[5] * ck) * (((kPi52 * ip) * iq) * rs);
-                double Xv[CLB][HU];
-                if constexpr (SP) {
-                    // HU independent FMA chains per lane component
-#pragma unroll
-                    for (int j = 0; j < CLB; j++)
-                        lane_contract<LU, LL, true>(pat[j], El[j], R, Xv[j],
-                                                    [](double e) { return e; });
-                } else {
-                    // hl outer, hu inner: CLB * HU independent FMA chains
-#pragma unroll
-                    for (int j = 0; j < CLB; j++)
-#pragma unroll
-                        for (int hu = 0; hu < HU; hu++) Xv[j][hu] = El[j][0] * R[hu];
-#pragma unroll
-                    for (int hl = 1; hl < NZ; hl++)
-#pragma unroll
-                        for (int hu = 0; hu < HU; hu++)
-#pragma unroll
-                            for (int j = 0; j < CLB; j++)
-                                Xv[j][hu] = fma(El[j][hl],
-                                                R[hidx(kH.t[hu] + kH.t[hl], kH.u[hu] + kH.u[hl],
-                                                       kH.v[hu] + kH.v[hl])],
-                                                Xv[j][hu]);
-                }
-#pragma unroll
-                for (int j = 0; j < CLB; j++)
-#pragma unroll
-                    for (int hu = 0; hu < HU; hu++) Xv[j][hu] *= f;
-                const double *ea = eu + (int64_t)a * erow;
-#pragma unroll
-                for (int u = 0; u < kDirectMaxU; u++) {
-                    if (u >= it.nu) break;
-                    // independent partial sums keep the FMA chains short
-                    constexpr int NP = CLB == 1 ? 8 : CLB == 2 ? 4 : 2;
-                    double y[CLB][NP];
-#pragma unroll
-                    for (int j = 0; j < CLB; j++)
-#pragma unroll
-                        for (int t = 0; t < NP; t++) y[j][t] = 0.0;
-#pragma unroll
-                    for (int hu = 0; hu < HU; hu++) {
-                        const double e = PFU ? Eu[(u * HU + hu) % NUE] : ea[u * HU + hu];
-#pragma unroll
-                        for (int j = 0; j < CLB; j++)
-                            y[j][hu % NP] = fma(e, Xv[j][hu], y[j][hu % NP]);
-                    }
-#pragma unroll
-                    for (int j = 0; j < CLB; j++) {
-                        double t = y[j][0];
-#pragma unroll
-                        for (int r = 1; r < NP; r++) t += y[j][r];
-                        accs[(u * CLB + j) * 64 + lane] += t;
-                    }
-                }
+    const double s = a + b;
+    return {s, b - (s - a)};
+}
+__device__ inline DD dd_mul(DD a, DD b)
+{
+    const double p = a.h * b.h;
+    return dd_norm(p, fma(a.h, b.h, -p) + (a.h * b.l + a.l * b.h));
+}
+__device__ inline DD dd_one_minus(DD a)
+{
+    const double s = 1.0 - a.h;
+    return dd_norm(s, ((1.0 - s) - a.h) - a.l);
+}
+
+// Primitive-pair rows of a shell pair (one block each)
+__global__ __launch_bounds__(128) void k_pair_rows(PP pp, SPD sd, double *rows)
+{
+    const int s = blockIdx.x;
+    const int rep = sd.comp[sd.coff[s]];
+    const int L = pp.L[rep], np = sd.np[s];
+    if (L > ZV_LMAX_T || np == 0) return;
+    const int64_t off = pp.off[rep];
+    const int rl = kRow[L], npad = (np + kLaneC - 1) / kLaneC * kLaneC;
+    double *d = rows + sd.roff[s];
+    for (int t = threadIdx.x; t < npad; t += blockDim.x) {
+        const int64_t at = off + (t < np ? t : np - 1);
+        double *o = d + (int64_t)t * rl;
+        const double p = pp.p[at], ip = pp.ip[at], al = pp.al[at], be = pp.be[at];
+        o[0] = p;
+        o[1] = pp.Px[at];
+        o[2] = pp.Py[at];
+        o[3] = pp.Pz[at];
+        for (int k = 4; k < rl; k++) o[k] = 0.0;
+        if (t >= np) continue;
+        const DD inv{ip, fma(-ip, p, 1.0) * ip}, half{0.5 * inv.h, 0.5 * inv.l};
+        // x = beta / p, y = alpha / p = 1 - x, the smaller one from its exponent
+        const DD sm = dd_mul(DD{al < be ? al : be, 0.0}, inv), lg = dd_one_minus(sm);
+        const DD x = al < be ? lg : sm, y = al < be ? sm : lg;
+        DD wn = dd_mul(DD{pp.c[at], 0.0}, inv); // c / p (1/2p)^n
+        for (int n = 0; n <= L; n++) {
+            for (int m = 0; m <= L - n; m++) {
+                DD v = wn;
+                for (int q = 0; q < m; q++) v = dd_mul(v, x);
+                for (int q = 0; q < L - n - m; q++) v = dd_mul(v, y);
+                o[4 + sig_index(L, n, m)] = v.h + v.l;
             }
+            wn = dd_mul(wn, half);
         }
-        for (int u = 0; u < it.nu; u++)
-#pragma unroll
-            for (int j = 0; j < CLB; j++) {
-                const double v = wave_sum(accs[(u * CLB + j) * 64 + lane]);
-                if (lane == 0) part[it.part + (int64_t)u * nlc + (cl + j - it.cl0)] = v;
-            }
     }
 }
 
-constexpr int pow2ceil(int x)
+// Expansion tables G of every component, one wavefront each.  First the 1D
+// Hermite polynomials of the (up to 4) power combinations per axis,
+//   e[t][k][m]: coefficient of (1/2p)^(t+k) x^m (1-x)^(a+b-t-2k-m),
+// by the Hermite recursion with D = B - A along the axis, lanes over the
+// coefficients; then lanes over the entries (nm, h), each summing the
+// products of its order n over the three axes and the r^2 variants, with the
+// degree raised from L - s - 2k to L - n by (x + 1 - x)^k.
+__global__ __launch_bounds__(64) void k_expansion(PP pp, SPD sd, const int *sp_of,
+                                                  const int *pair_i, const int *pair_k,
+                                                  const double *center, const int *npower,
+                                                  const int *itype, double *gu, double *gl)
 {
-    int p = 1;
-    while (p < x) p <<= 1;
-    return p;
+    constexpr int NE = 75; // [t 5][k 3][m 5]
+    __shared__ double e[2][12][NE];
+    const int q = blockIdx.x, lane = threadIdx.x;
+    const int P = sd.comp[q], L = pp.L[P];
+    if (L > ZV_LMAX_T) return;
+    const int s = sp_of[q];
+    const GTable &gt = kG.t[L];
+    const int64_t at = sd.goff[s] + (int64_t)(q - sd.coff[s]) * gt.n;
+    const int i = pair_i[P] - 1, k = pair_k[P] - 1;
+    const int ri = itype[i] == 2 ? 2 : 0, rk = itype[k] == 2 ? 2 : 0;
+    // polynomial 4 axis + 2 (r^2 of i on this axis) + (r^2 of k on this axis)
+    for (int t = lane; t < 12 * NE; t += 64) e[0][t / NE][t % NE] = t % NE == 0 ? 1.0 : 0.0;
+    __syncthreads();
+    for (int step = 0; step < 4; step++) {
+        for (int x = lane; x < 12 * NE; x += 64) {
+            const int pl = x / NE, c = x % NE, ax = pl / 4;
+            const int t = c / 15, kk = c / 5 % 3, m = c % 5;
+            const int pa = npower[3 * i + ax] + (pl & 2 ? ri : 0);
+            const int pb = npower[3 * k + ax] + (pl & 1 ? rk : 0);
+            const double *o = e[step & 1][pl];
+            double v = o[c];
+            if (step < pa + pb) {
+                const double D = center[3 * k + ax] - center[3 * i + ax];
+                v = t > 0 ? o[c - 15] : 0.0;
+                if (step < pa) {
+                    if (m > 0) v += D * o[c - 1];
+                } else {
+                    v -= D * o[c];
+                }
+                if (t < 4 && kk > 0) v += (t + 1) * o[c + 15 - 5];
+            }
+            e[(step + 1) & 1][pl][c] = v;
+        }
+        __syncthreads();
+    }
+    const int vi = ri ? 3 : 1, vk = rk ? 3 : 1;
+    for (int j = lane; j < gt.n; j += 64) {
+        const int sg = gt.sig[j], h = gt.h[j], t = kH.t[h], u = kH.u[h], v = kH.v[h];
+        const int dp = sig_depth(sg), n = L - dp, M = sg - dp * (dp + 1) / 2;
+        const int kk = n - (t + u + v);
+        double acc = 0.0;
+        for (int w = 0; w < vi * vk; w++) {
+            const int a = w / vk, b = w % vk;
+            const double *E[3];
+            int d[3];
+            for (int ax = 0; ax < 3; ax++) {
+                const int xi = ri && a == ax, xk = rk && b == ax;
+                E[ax] = e[0][4 * ax + 2 * xi + xk];
+                d[ax] = npower[3 * i + ax] + npower[3 * k + ax] + (xi ? 2 : 0) + (xk ? 2 : 0);
+            }
+            for (int kx = 0; kx <= kk && t + 2 * kx <= d[0]; kx++)
+                for (int ky = 0; kx + ky <= kk && u + 2 * ky <= d[1]; ky++) {
+                    const int kz = kk - kx - ky;
+                    if (v + 2 * kz > d[2]) continue;
+                    const double *ex = E[0] + 15 * t + 5 * kx, *ey = E[1] + 15 * u + 5 * ky,
+                                 *ez = E[2] + 15 * v + 5 * kz;
+                    for (int mx = 0; mx <= d[0] - t - 2 * kx; mx++)
+                        for (int my = 0; my <= d[1] - u - 2 * ky; my++) {
+                            const double xy = ex[mx] * ey[my];
+                            double bin = 1.0; // binomial(kk, z)
+                            for (int z = 0; z <= kk; z++) {
+                                const int mz = M - mx - my - z;
+                                if (mz >= 0 && mz <= d[2] - v - 2 * kz) acc += bin * xy * ez[mz];
+                                bin = bin * (kk - z) / (z + 1);
+                            }
+                        }
+                }
+        }
+        gu[at + j] = acc;
+        gl[at + j] = (t + u + v) & 1 ? -acc : acc;
+    }
 }
 
-// Reduction-mode batch size per class compiled for at least two waves per
-// SIMD (the register allocator then fits 256 registers, spilling if it
-// must); 0: none.  (2, 1) with sparse passes of 3 needed it while its Boys
-// function was the erf form (260 registers otherwise; 554 against 908 ms);
-// with the table (two reduction rounds, shell_red_rounds) it takes 202
-// registers by itself, and no class uses it now.
-constexpr int kShellTwoWaves[5][5] = {{0, 0, 0, 0, 0},
-                                      {0, 0, 0, 0, 0},
-                                      {0, 0, 0, 0, 0},
-                                      {0, 0, 0, 0, 0},
-                                      {0, 0, 0, 0, 0}};
-constexpr int shell_waves(int LU, int LL, int B) { return kShellTwoWaves[LU][LL] == B ? 2 : 1; }
-
-// Reduction mode (nu >= 4): the uniform E does not depend on the lane
-// primitive pair, so for each uniform primitive pair a the wave first forms
-// X_hu = sum over all lane primitive pairs (every lane chunk, the prefactor
-// folded into the lane E), sums it over the 64 lanes through LDS, and lane u
-// then contracts the sum with the E of its own uniform component u.  One LDS
-// reduction per (a, pass).
-// PF: lane data of the next chunk loaded one chunk ahead (kShellPrefetch)
-template <int LU, int LL, int CLB, bool PF, bool TB, bool SP, int NCH>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(shell_waves(LU, LL, CLB))))
-void k_eri_shell_red(PP pp, SPD sd,
-                                                      const ShellItem *__restrict__ items,
-                                                      const double *__restrict__ pu_all,
-                                                      const double *__restrict__ eu2_all,
-                                                      double *__restrict__ part)
+// Sums over the four blocks of 4 lanes in each row of 16: the partner 8 and 4
+// lanes away (row rotation by 8; shifts by 4 either way, merged by bank).
+__device__ __forceinline__ double lane_xor8(double v)
 {
-    constexpr int HU = hcount(LU), L = LU + LL, HR = hcount(L);
-    constexpr int NZ = SP ? kHP.nzmax[LL] : hcount(LL); // lane E per component
-    constexpr int NR = CLB * HU; // rows summed over the wave
-    constexpr int RC = NR / NCH; // rows per transpose round
-    static_assert(NR % NCH == 0, "whole transpose rounds");
-    constexpr int S = RC | 1;    // odd lane stride of the transpose buffer
-    __shared__ double lds[64 * S + NR];
-    __shared__ double lbt[TB ? kBoysSlice : 1]; // Boys Taylor table, this L
-    if constexpr (TB) boys_table_load<L>(pp.btab, lbt);
-    const int lane = threadIdx.x;
-    const ShellItem it = items[blockIdx.x];
-    const int ub = sd.coff[it.su], lb = sd.coff[it.sl];
-    const int ncu = sd.coff[it.su + 1] - ub;
-    const int repl = sd.comp[lb];
-    const int nl = pp.cnt[repl];
-    const int64_t ol = pp.off[repl];
-    const double *pu = pu_all + sd.puoff[it.su];
-    const int nlc = it.cl1 - it.cl0;
-    const bool own = lane < it.nu; // lane owns uniform component cu0 + lane
-    // lanes past the uniform range read component cu0 (in range) and drop it
-    const double *eu2 = eu2_all + sd.euoff[it.su] + it.cu0 + (own ? lane : 0);
-    // the item's lane components are whole passes of CLB (host-checked)
-    for (int cl = it.cl0; cl < it.cl1; cl += CLB) {
-        int64_t el[CLB];
-        int capl[CLB], pat[CLB], nzl[CLB];
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x128, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x128, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ int lane_xor4(int v)
+{
+    const int up = __builtin_amdgcn_update_dpp(0, v, 0x104, 0xf, 0x5, false); // lane + 4
+    return __builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xa, false);        // lane - 4
+}
+__device__ __forceinline__ double lane_xor4(double v)
+{
+    const long long b = __double_as_longlong(v);
+    return __longlong_as_double(((long long)lane_xor4((int)(b >> 32)) << 32) |
+                                (unsigned)lane_xor4((int)b));
+}
+
+// One wave's LDS accesses are in order; this keeps the compiler from moving
+// them across.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+constexpr int kTRows = 9;   // uniform components transformed at a time
+
+// waves per workgroup and per SIMD of a class's pass
+constexpr int quartet_waves(int LU, int LL, int p)
+{
+    const Slots s = make_slots(LU, LL, pass_of(LU, LL, p));
+    return 2 * (s.n + hcount(pass_of(LU, LL, p).rho1)) + 64 <= 256 ? 2 : 1;
+}
+constexpr int quartet_wpb(int LU, int LL, int p) { return quartet_waves(LU, LL, p) >= 2 ? 4 : 1; }
+
+template <int LU, int LL, int PASS>
+__global__ __launch_bounds__(64 * quartet_wpb(LU, LL, PASS))
+__attribute__((amdgpu_waves_per_eu(quartet_waves(LU, LL, PASS)))) void
+k_eri_quartet(SPD sd, const ShellItem *__restrict__ items, int nitems,
+              const double *__restrict__ btab, const short *__restrict__ ztab,
+              const double *__restrict__ rows, const double *__restrict__ gu,
+              const double *__restrict__ gl, double *__restrict__ part)
+{
+    using C = Cls<LU, LL, PASS>;
+    constexpr int WPB = quartet_wpb(LU, LL, PASS);
+    constexpr int L = C::ps.rho1, HR = hcount(L), NS = C::sl.n, NZ = C::sl.ztot;
+    constexpr int RU = kRow[LU], RLn = kRow[LL], GU = ngroup(LU), GL = ngroup(LL);
+    constexpr int NGU = kG.t[LU].n, NGL = kG.t[LL].n;
+    __shared__ double lbt[kBoysSlice];
+    __shared__ double zall[WPB][C::zwords + 1]; // the last word stays 0
+    __shared__ double tall[WPB][kTRows * NGL];
+    for (int t = threadIdx.x; t < kBoysSlice; t += 64 * WPB)
+        lbt[t] = btab[(size_t)L * kBoysSlice + t];
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const int ii = blockIdx.x * WPB + wave;
+    if (ii >= nitems) return;
+    const ShellItem it = items[ii];
+    double *Z = zall[wave];
+    for (int t = lane; t < C::zwords + 1; t += 64) Z[t] = 0.0;
+    const int al = lane >> 4, cl = lane & 15, j4 = lane & 3;
+    const double *ub = rows + sd.roff[it.su] + al * RU;
+    const double *lb = rows + sd.roff[it.sl];
+    const bool b1 = (lane & 4) != 0, b2 = (lane & 8) != 0; // block of 4 lanes in its row of 16
+
+    for (int k = it.k0; k < it.k1; k++) {
+        const double *lr = lb + (int64_t)(kLaneC * k + cl) * RLn;
+        const double q = lr[0], Qx = lr[1], Qy = lr[2], Qz = lr[3];
+        // lane weights as the A operand of the sum over c: row 4 g' + j4,
+        // inner index c = 4 block + lane / 16
+        const double *lw = lb + (int64_t)(kLaneC * k + (lane >> 2 & 3) * 4 + al) * RLn + 4 + j4;
+        double Wl[GL];
 #pragma unroll
-        for (int j = 0; j < CLB; j++) {
-            const int Pl = sd.comp[lb + cl + j];
-            el[j] = pp.eoff[Pl];
-            capl[j] = pp.cap[Pl];
-            const int cp = sd.cpat[lb + cl + j];
-            pat[j] = cp & 0xff;
-            nzl[j] = cp >> 8;
-        }
-        double acc[CLB];
+        for (int g = 0; g < GL; g++) Wl[g] = 4 * g + 4 <= RLn - 4 || 4 * g + j4 < RLn - 4 ? lw[4 * g] : 0.0;
+        double V[NS];
 #pragma unroll
-        for (int j = 0; j < CLB; j++) acc[j] = 0.0;
-        // lane data of the chunk in flight (PF)
-        double nq = 0.0, niq = 0.0, nQx = 0.0, nQy = 0.0, nQz = 0.0, nck = 0.0, nE[CLB][NZ];
-        auto load_lane = [&](int c0) {
-            const int c = c0 + lane;
-            const bool live = c < nl;
-            const int cc = live ? c : c0;
-            nq = pp.p[ol + cc];
-            niq = pp.ip[ol + cc];
-            nQx = pp.Px[ol + cc];
-            nQy = pp.Py[ol + cc];
-            nQz = pp.Pz[ol + cc];
-            nck = live ? pp.c[ol + cc] : 0.0;
+        for (int i = 0; i < NS; i++) V[i] = 0.0;
+        // uniform rows one step ahead
+        double np_, nx, ny, nz, nw[GU], ns0;
+        auto load_u = [&](int s) {
+            const double *r = ub + (int64_t)(kStepA * s) * RU;
+            np_ = r[0];
+            nx = r[1];
+            ny = r[2];
+            nz = r[3];
+            ns0 = r[4];
+            if constexpr (LU > 0) {
 #pragma unroll
-            for (int j = 0; j < CLB; j++)
-#pragma unroll
-                for (int k = 0; k < NZ; k++) {
-                    if constexpr (SP)
-                        nE[j][k] = k < nzl[j] ? sd.ec[el[j] + (int64_t)k * capl[j] + cc] : 0.0;
-                    else
-                        nE[j][k] = cl + j < it.cl1 ? pp.E[el[j] + (int64_t)k * capl[j] + cc] : 0.0;
-                }
+                for (int g = C::ps.g0; g < C::ps.g1; g++) nw[g] = r[4 + 4 * g + j4];
+            }
         };
-        if constexpr (PF) load_lane(0);
-        for (int a = it.a0; a < it.a1; a++) {
-            const double *pa = pu + (int64_t)a * 8;
-            const double p = pa[0], ip = pa[1], Px = pa[2], Py = pa[3], Pz = pa[4], cb = pa[5];
-            const double *ea = eu2 + (int64_t)a * HU * ncu;
-            double Xa[CLB][HU];
+        load_u(it.s0);
+        for (int s = it.s0; s < it.s1; s++) {
+            const double p = np_, X = nx - Qx, Y = ny - Qy, Zc = nz - Qz, w0 = ns0;
+            double w[GU];
 #pragma unroll
-            for (int j = 0; j < CLB; j++)
-#pragma unroll
-                for (int hu = 0; hu < HU; hu++) Xa[j][hu] = 0.0;
-            for (int c0 = 0; c0 < nl; c0 += 64) {
-                const int c = c0 + lane;
-                const bool live = c < nl;
-                const int cc = live ? c : c0; // in-range index for idle lanes
-                double q, iq, Qx, Qy, Qz, ck, Er[CLB][NZ];
-                if constexpr (PF) {
-                    // this chunk's lane data were loaded one chunk ahead; the
-                    // next chunk's (or, after the last, the first chunk of the
-                    // next uniform primitive pair) go in flight now, behind
-                    // this chunk's Boys, R and X work
-                    q = nq;
-                    iq = niq;
-                    Qx = nQx;
-                    Qy = nQy;
-                    Qz = nQz;
-                    ck = nck;
-#pragma unroll
-                    for (int j = 0; j < CLB; j++)
-#pragma unroll
-                        for (int k = 0; k < NZ; k++) Er[j][k] = nE[j][k];
-                    // (one chunk in all: its data stay in the prefetch set)
-                    const int n0 = c0 + 64 < nl ? c0 + 64 : 0;
-                    if (c0 + 64 < nl || (a + 1 < it.a1 && nl > 64)) load_lane(n0);
-                } else {
-                    q = pp.p[ol + cc];
-                    iq = pp.ip[ol + cc];
-                    Qx = pp.Px[ol + cc];
-                    Qy = pp.Py[ol + cc];
-                    Qz = pp.Pz[ol + cc];
-                    ck = live ? pp.c[ol + cc] : 0.0;
-                }
-                const double X = Px - Qx, Y = Py - Qy, Z = Pz - Qz;
-                const double s = p + q;
-                const double rs = rsqrt_pos(s), is = rs * rs;
-                const double alpha = (p * q) * is;
-                const double T = alpha * ((X * X + Y * Y) + Z * Z);
-                double F[L + 1];
-                if constexpr (TB)
-                    boys_table<L>(T, lbt, F);
+            for (int g = C::ps.g0; g < C::ps.g1; g++) w[g] = LU > 0 ? nw[g] : 0.0;
+            if (s + 1 < it.s1) load_u(s + 1);
+            const double sum = p + q;
+            const double rs = rsqrt_pos(sum);
+            const double alpha = (p * q) * (rs * rs);
+            const double T = alpha * fma(X, X, fma(Y, Y, Zc * Zc));
+            double F[L + 1];
+            boys_table<L>(T, lbt, F);
+            double R[HR];
+            hermite_table<L>(alpha, rs, X, Y, Zc, F, R);
+            static_for<NS>([&](auto i) {
+                constexpr int r = C::sl.r[i], g = C::sl.g[i];
+                if constexpr (C::sl.sig[i] >= 0)
+                    V[i] = fma(R[r], w0, V[i]);
                 else
-                    boys<L>(T, F);
-                double R[HR];
-                hermite_R<L>(alpha, X, Y, Z, F, R);
-                const double f = (cb * ck) * (((kPi52 * ip) * iq) * rs);
-                // the lane E (dense: with the prefactor and the Hermite sign
-                // folded in here; SP: lane_contract applies both)
-                double El[CLB][NZ];
-#pragma unroll
-                for (int j = 0; j < CLB; j++)
-#pragma unroll
-                    for (int k = 0; k < NZ; k++) {
-                        // (guarded loads: as a condition the guard keeps the
-                        // compiler from issuing them one at a time next to
-                        // their uses, which serialized their latency; cl + j <
-                        // it.cl1 always holds)
-                        if constexpr (SP) {
-                            if constexpr (PF)
-                                El[j][k] = Er[j][k];
-                            else
-                                El[j][k] =
-                                    k < nzl[j] ? sd.ec[el[j] + (int64_t)k * capl[j] + cc] : 0.0;
-                        } else {
-                            double e;
-                            if constexpr (PF)
-                                e = Er[j][k];
-                            else
-                                e = cl + j < it.cl1 ? pp.E[el[j] + (int64_t)k * capl[j] + cc] : 0.0;
-                            El[j][k] = ((kH.t[k] + kH.u[k] + kH.v[k]) & 1) ? -(e * f) : e * f;
-                        }
-                    }
-                if constexpr (SP) {
-#pragma unroll
-                    for (int j = 0; j < CLB; j++)
-                        lane_contract<LU, LL, false>(pat[j], El[j], R, Xa[j],
-                                                     [f](double e) { return e * f; });
-                } else {
-#pragma unroll
-                    for (int hl = 0; hl < NZ; hl++)
-#pragma unroll
-                        for (int hu = 0; hu < HU; hu++)
-#pragma unroll
-                            for (int j = 0; j < CLB; j++)
-                                Xa[j][hu] = fma(El[j][hl],
-                                                R[hidx(kH.t[hu] + kH.t[hl], kH.u[hu] + kH.u[hl],
-                                                       kH.v[hu] + kH.v[hl])],
-                                                Xa[j][hu]);
-                }
-            }
-            // the lane's uniform E, loaded here so that its latency hides
-            // behind the LDS reduction below
-            double ev[HU];
-#pragma unroll
-            for (int hu = 0; hu < HU; hu++) ev[hu] = ea[(int64_t)hu * ncu];
-            // row r = j HU + hu summed over the 64 lanes into lds[64 S + r],
-            // RC rows per round through the transpose buffer (NCH rounds
-            // keep the buffer small enough for the Boys table beside it)
-#pragma unroll
-            for (int ch = 0; ch < NCH; ch++) {
-                if (ch > 0) __syncthreads(); // the previous round's reads are done
-#pragma unroll
-                for (int rr = 0; rr < RC; rr++) {
-                    const int r = ch * RC + rr;
-                    lds[lane * S + rr] = Xa[r / HU][r % HU];
-                }
-                __syncthreads();
-                if constexpr (RC <= 64) {
-                    // P lanes per segment, 64 / P segments of each row
-                    constexpr int P = pow2ceil(RC), G = 64 / P, SEG = 64 / G;
-                    const int r = lane & (P - 1), k = lane / P;
-                    double t4[4] = {0.0, 0.0, 0.0, 0.0};
-                    if (r < RC) {
-#pragma unroll
-                        for (int i = 0; i < SEG; i++) t4[i & 3] += lds[(k * SEG + i) * S + r];
-                    }
-                    double v = (t4[0] + t4[1]) + (t4[2] + t4[3]);
-#pragma unroll
-                    for (int o = P; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
-                    if (k == 0 && r < RC) lds[64 * S + ch * RC + r] = v;
-                } else {
-                    for (int r = lane; r < RC; r += 64) {
-                        double t4[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                        for (int i = 0; i < 64; i++) t4[i & 3] += lds[i * S + r];
-                        lds[64 * S + ch * RC + r] = (t4[0] + t4[1]) + (t4[2] + t4[3]);
-                    }
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < CLB; j++) {
-                double y[2] = {0.0, 0.0};
-#pragma unroll
-                for (int hu = 0; hu < HU; hu++)
-                    y[hu & 1] = fma(ev[hu], lds[64 * S + j * HU + hu], y[hu & 1]);
-                acc[j] += y[0] + y[1];
-            }
+                    V[i] = __builtin_amdgcn_mfma_f64_4x4x4f64(R[r], w[g], V[i], 0, 0, 0);
+            });
         }
-#pragma unroll
-        for (int j = 0; j < CLB; j++)
-            if (own) part[it.part + (int64_t)lane * nlc + (cl + j - it.cl0)] = acc[j];
+        // per-lane sums (one of the 4 a each) to tile form: summed over a
+        const double hot = j4 == 0 ? 1.0 : 0.0;
+        static_for<NS>([&](auto i) {
+            if constexpr (C::sl.sig[i] >= 0)
+                V[i] = __builtin_amdgcn_mfma_f64_4x4x4f64(V[i], hot, 0.0, 0, 0, 0);
+        });
+        // Z tiles, four at a time: sum over c, then over the blocks, block b
+        // keeping tile b
+        static_for<(NZ + 3) / 4>([&](auto zq) {
+            double t4[4];
+            static_for<4>([&](auto b) {
+                constexpr int z = 4 * zq + b;
+                if constexpr (z < NZ)
+                    t4[b] = __builtin_amdgcn_mfma_f64_4x4x4f64(Wl[C::sl.zg[z]],
+                                                               V[C::sl.zslot[z]], 0.0, 0, 0, 0);
+                else
+                    t4[b] = 0.0;
+            });
+            const double y0 = (b2 ? t4[2] : t4[0]) + lane_xor8(b2 ? t4[0] : t4[2]);
+            const double y1 = (b2 ? t4[3] : t4[1]) + lane_xor8(b2 ? t4[1] : t4[3]);
+            Z[zq * 64 + lane] += (b1 ? y1 : y0) + lane_xor4(b1 ? y0 : y1);
+        });
+    }
+    wave_lds_fence();
+    // transform to the components
+    double *T = tall[wave];
+    const int cu0 = sd.coff[it.su], ncu = sd.coff[it.su + 1] - cu0;
+    const int ncl = sd.coff[it.sl + 1] - sd.coff[it.sl];
+    const double *Gu = gu + sd.goff[it.su], *Gl = gl + sd.goff[it.sl];
+    for (int u0 = 0; u0 < ncu; u0 += kTRows) {
+        const int nu = ncu - u0 < kTRows ? ncu - u0 : kTRows;
+        for (int t = lane; t < nu * NGL; t += 64) {
+            const int u = t / NGL, jl = t - u * NGL;
+            const double *g = Gu + (int64_t)(u0 + u) * NGU;
+            const short *zp = ztab + jl;
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 14
+            for (int j = 0; j < NGU; j++) v[j & 3] = fma(g[j], Z[zp[j * NGL]], v[j & 3]);
+            T[t] = (v[0] + v[1]) + (v[2] + v[3]);
+        }
+        wave_lds_fence();
+        for (int t = lane; t < nu * ncl; t += 64) {
+            const int u = t / ncl, l = t - u * ncl;
+            const double *g = Gl + (int64_t)l * NGL;
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 14
+            for (int j = 0; j < NGL; j++) v[j & 3] = fma(g[j], T[u * NGL + j], v[j & 3]);
+            part[it.part + (int64_t)u0 * ncl + t] = kPi52 * ((v[0] + v[1]) + (v[2] + v[3]));
+        }
+        wave_lds_fence();
     }
 }
 
@@ -601,17 +623,49 @@ void k_eri_shell_red(PP pp, SPD sd,
 // quartet (su == sl) holds every component quartet twice; the (P >= Q) copy
 // is written.  With pre, off-diagonal component quartets failing
 // |pre_P pre_Q| >= 1e-30 are written as zero (src/two_e_slater.F90:268-272).
+// A small molecule's quartets are cut into thousands of slices of one or a
+// few components, so the workgroup's threads share the slices of each
+// component (fixed shares, added in a fixed order): with one thread adding
+// them all, this kernel took more than half of a 7-AO molecule's time and the
+// long sequential sum was its largest rounding error.
 __global__ __launch_bounds__(256) void k_shell_scatter(const ShellGroup *groups, SPD sd,
                                                        const double *part, const double *pre,
                                                        double *tri)
 {
+    __shared__ double red[256];
     const ShellGroup g = groups[blockIdx.x];
-    const int n = g.nu * g.nl;
-    const int bu = sd.coff[g.su] + g.cu0, bl = sd.coff[g.sl] + g.cl0;
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
+    const int bu = sd.coff[g.su], bl = sd.coff[g.sl];
+    const int nl = sd.coff[g.sl + 1] - bl, n = (sd.coff[g.su + 1] - bu) * nl;
+    const int width = n < 256 ? n : 256, team = min(256 / width, g.ns);
+    const int tc = threadIdx.x % width, ts = threadIdx.x / width;
+    for (int t0 = 0; t0 < n; t0 += width) {
+        const int t = t0 + tc;
+        const bool mine = ts < team && t < n;
         double v = 0.0;
-        for (int s = 0; s < g.ns; s++) v += part[g.part + (int64_t)s * n + t];
-        const int u = t / g.nl, l = t - u * g.nl;
+        if (mine) {
+            const double *p = part + g.part + t;
+            double a[4] = {0.0, 0.0, 0.0, 0.0};
+            int s = ts;
+            for (; s + 3 * team < g.ns; s += 4 * team)
+#pragma unroll
+                for (int k = 0; k < 4; k++) a[k] += p[(int64_t)(s + k * team) * n];
+            for (; s < g.ns; s += team) a[0] += p[(int64_t)s * n];
+            v = (a[0] + a[1]) + (a[2] + a[3]);
+        }
+        if (team > 1) {
+            __syncthreads();
+            red[threadIdx.x] = v;
+            __syncthreads();
+            for (int h = 1; h < team; h <<= 1) {
+                double w = 0.0;
+                const bool add = mine && ts % (2 * h) == 0 && ts + h < team;
+                if (add) w = red[threadIdx.x + h * width];
+                if (add) red[threadIdx.x] = v += w;
+                __syncthreads();
+            }
+        }
+        if (!mine || ts > 0) continue;
+        const int u = t / nl, l = t - u * nl;
         const int P = sd.comp[bu + u], Q = sd.comp[bl + l];
         if (g.su == g.sl && P < Q) continue;
         if (pre && P != Q && fabs(pre[P] * pre[Q]) < 1.0e-30) v = 0.0;
@@ -625,181 +679,90 @@ __global__ void k_zero(double *x, int64_t n)
     if (i < n) x[i] = 0.0;
 }
 
-// Largest lane-component batch of each (LU, LL) class, direct and reduction
-// mode: the lane components of a shell pair run in passes of this many (and
-// one pass of the remainder); the components of one pass share the Boys
-// values and the R table of every primitive quartet, so wider passes redo
-// them less often.  Chosen so that the R table, the pass's lane E and its X
-// sums stay in the register file without spilling, and by shell-pair sizes:
-// an order-0 pair has 1 component, order 1 has 3 (p x s), order 2 has 9
-// (p x p) or 6 (d x s), so 3 covers them in as few passes as 4 does with
-// fewer registers.  (2, 2) in reduction mode runs passes of 2 at two waves
-// per SIMD, which beats passes of 3 at one wave (949 against 1088 ms on the
-// 200-AO molecule, dense lane E).  The wider passes of (2, 3), (2, 4),
-// (3, 3) and (4, 2) in reduction mode and of (3, 3) and (1, 4) in direct
-// mode pay off with the sparse lane E (kShellSparse) only.
-constexpr int kClbMax = 4;
-constexpr int kShellClb[5][5] = {{1, 3, 3, 4, 4},
-                                 {1, 3, 3, 4, 4},
-                                 {1, 3, 3, 3, 1},
-                                 {1, 3, 3, 3, 1},
-                                 {1, 3, 2, 1, 1}};
-constexpr int kShellClbRed[5][5] = {{1, 3, 3, 4, 2},
-                                    {1, 3, 3, 3, 1},
-                                    {1, 3, 2, 3, 2},
-                                    {1, 3, 3, 2, 1},
-                                    {1, 2, 2, 1, 1}};
+// ------------------------------------------------------------------ launches
+// bucket b = 25 (2 pass) + 5 LU + LL: the statistics slot is 36 + b
+constexpr int kNB = 25 * 2 * kPassMax;
+constexpr int bucket_of(int LU, int LL, int pass) { return 50 * pass + 5 * LU + LL; }
 
-// Reduction-mode classes whose lane data are loaded one chunk ahead: those
-// at one wave per SIMD anyway, with room for a second set of lane registers
-// without spilling (single-component passes of order-4 quartets stay at
-// two waves per SIMD without it and keep that), and (2, 1), whose passes
-// of 3 keep two waves with it (241 registers; 507 → 478 ms).
-constexpr bool kShellPrefetch[5][5] = {{false, false, false, false, false},
-                                       {false, false, false, true, true},
-                                       {false, true, false, true, false},
-                                       {false, true, false, true, false},
-                                       {false, true, true, false, false}};
-constexpr bool shell_prefetch(int LU, int LL, int B)
+struct LaunchArgs {
+    SPD sd;
+    const ShellItem *items;
+    int n;
+    const double *btab;
+    const short *ztab;
+    double *part;
+    hipStream_t st;
+};
+
+template <int LU, int LL, int PASS> void launch_quartet(const LaunchArgs &a)
 {
-    return kShellPrefetch[LU][LL] && !(B == 1 && LU + LL <= 4);
-}
-// Instances that evaluate the Boys function from the Taylor table in LDS
-// (boys_table, 8.8 KB per workgroup) instead of erf and the series (boys):
-// all whose LDS then still allows two workgroups of one wave per SIMD (20 KB
-// each), and the reduction kernels of order 4 and up, which run one wave
-// per SIMD anyway, up to 40 KB (four per CU).
-constexpr int shell_lds_bytes(int LU, int B, bool red, int nch = 1)
-{
-    const int HU = hcount(LU), NR = B * HU, S = (NR / nch) | 1;
-    return red ? (64 * S + NR) * 8 : kDirectMaxU * B * 64 * 8;
-}
-constexpr bool shell_table_fits(int LU, int LL, int B, bool red, int nch)
-{
-    const int bytes = shell_lds_bytes(LU, B, red, nch) + kBoysSlice * 8;
-    return LU + LL <= kBoysLmax &&
-           (bytes <= 20480 || (red && LU + LL >= 4 && bytes <= 40960));
-}
-// Reduction instances whose transpose buffer would leave no room for the
-// Boys table sum their rows in two rounds of half the rows instead, where
-// that makes it fit ((2, 1) with passes of 3, (4, x) with passes of 2).
-constexpr int shell_red_rounds(int LU, int LL, int B)
-{
-    const int NR = B * hcount(LU);
-    return !shell_table_fits(LU, LL, B, true, 1) && NR % 2 == 0 &&
-                   shell_table_fits(LU, LL, B, true, 2)
-               ? 2
-               : 1;
-}
-constexpr bool shell_boys_table(int LU, int LL, int B, bool red)
-{
-    return shell_table_fits(LU, LL, B, red, red ? shell_red_rounds(LU, LL, B) : 1);
-}
-// Direct-mode classes whose uniform data are loaded one iteration ahead into
-// vector registers (uniform side of order 0 or 1: at most 18 doubles): the
-// ones already at one wave per SIMD without it (lane order 3 and 4) and
-// still free of spills with it.
-constexpr bool shell_prefetch_u(int LU, int LL, int B)
-{
-    return LU <= 1 && LL >= 3 && !(LL == 4 && LU + B >= 4);
+    constexpr int WPB = quartet_wpb(LU, LL, PASS);
+    hipLaunchKernelGGL((k_eri_quartet<LU, LL, PASS>), dim3((unsigned)((a.n + WPB - 1) / WPB)),
+                       dim3(64 * WPB), 0, a.st, a.sd, a.items, a.n, a.btab, a.ztab, a.sd.rows,
+                       a.sd.gu, a.sd.gl, a.part);
 }
 
-// Classes that skip the structural zeros of the lane E (lane_contract), by
-// (uniform order, lane order): direct mode, reduction mode.  Chosen by
-// per-class kernel time on the 200-AO molecule: the pattern dispatch costs
-// scalar compares and registers, so it pays where the X contraction is
-// large against the Boys function and R table (uniform order >= 2 in
-// reduction mode) and not in the direct mode's short per-uniform-pair
-// iterations of uniform order <= 1 (lane order 3: 278 against 103 ms),
-// except (1, 4) with passes of 4 (about even); nor for (4, 4), whose 22
-// patterns of up to 25 coefficients spill (315 against 145 ms).
-constexpr bool kShellSparse[5][5] = {{false, false, false, false, false},
-                                     {false, false, false, false, true},
-                                     {false, false, false, false, false},
-                                     {false, false, false, true, false},
-                                     {false, false, false, false, false}};
-constexpr bool kShellSparseRed[5][5] = {{false, false, false, false, false},
-                                        {false, false, false, false, false},
-                                        {false, true, true, true, true},
-                                        {false, false, true, true, true},
-                                        {false, false, true, true, false}};
-constexpr bool shell_sparse(int LU, int LL, bool red)
-{
-    return red ? kShellSparseRed[LU][LL] : kShellSparse[LU][LL];
-}
+struct ClassInfo {
+    void (*launch)(const LaunchArgs &) = nullptr;
+    double step = 0.0, chunk = 0.0; // estimated cycles per step and per chunk
+    double acc = 0.0;               // multiply-adds per primitive quartet
+    std::vector<short> ztab;
+};
 
-template <int LU, int LL, int B>
-void launch_shell_b(bool red, unsigned grid, hipStream_t st, const PP &pp, const SPD &sd,
-                    const ShellItem *items, double *part)
+// Estimated SIMD cycles at two waves per SIMD: 5.5 per FP64 vector
+// instruction, 16.4 per 4x4x4 matrix instruction (both measured on MI355X).
+template <int LU, int LL, int PASS> void add_class(ClassInfo *t)
 {
-    if (red)
-        hipLaunchKernelGGL((k_eri_shell_red<LU, LL, B, shell_prefetch(LU, LL, B),
-                                            shell_boys_table(LU, LL, B, true),
-                                            shell_sparse(LU, LL, true),
-                                            shell_red_rounds(LU, LL, B)>),
-                           dim3(grid), dim3(64), 0, st, pp, sd, items, sd.pu, sd.eu2, part);
-    else
-        hipLaunchKernelGGL((k_eri_shell<LU, LL, B, shell_prefetch_u(LU, LL, B),
-                                        shell_boys_table(LU, LL, B, false),
-                                        shell_sparse(LU, LL, false)>),
-                           dim3(grid), dim3(64), 0, st, pp, sd, items, sd.pu, sd.eu, part);
-}
-
-// instances up to the class's batch limit only (the larger ones are never
-// planned); false for a batch outside it
-template <int LU, int LL>
-bool launch_shell_t(int clb, bool red, unsigned grid, hipStream_t st, const PP &pp,
-                    const SPD &sd, const ShellItem *items, double *part)
-{
-    constexpr int MR = kShellClbRed[LU][LL], MD = kShellClb[LU][LL];
-    if (clb < 1 || clb > (red ? MR : MD)) return false;
-    switch (clb) {
-    case 1: launch_shell_b<LU, LL, 1>(red, grid, st, pp, sd, items, part); return true;
-    case 2:
-        if constexpr (MR >= 2 || MD >= 2)
-            launch_shell_b<LU, LL, 2>(red, grid, st, pp, sd, items, part);
-        return true;
-    case 3:
-        if constexpr (MR >= 3 || MD >= 3)
-            launch_shell_b<LU, LL, 3>(red, grid, st, pp, sd, items, part);
-        return true;
-    case 4:
-        if constexpr (MR >= 4 || MD >= 4)
-            launch_shell_b<LU, LL, 4>(red, grid, st, pp, sd, items, part);
-        return true;
+    using C = Cls<LU, LL, PASS>;
+    ClassInfo &c = t[bucket_of(LU, LL, PASS)];
+    c.launch = launch_quartet<LU, LL, PASS>;
+    const int L = C::ps.rho1;
+    int ns = 0, nm = 0;
+    for (int i = 0; i < C::sl.n; i++) (C::sl.sig[i] >= 0 ? ns : nm)++;
+    const double r = (L + 1) * (L + 2) * (L + 3) * (L + 4) / 24.0 - (L + 1);
+    c.step = 5.5 * (62.0 + 3.0 * L + 1.7 * r + ns) + 16.4 * nm;
+    c.chunk = 1500.0 + 16.4 * (ns + C::sl.ztot) + 30.0 * C::sl.ztot;
+    for (int i = 0; i < C::sl.n; i++) {
+        const int need = sig_prefix(LU, horder(C::sl.r[i]) - LL) - 4 * C::sl.g[i];
+        c.acc += need < 4 ? need : 4;
     }
-    return false;
+    const GTable &u = kG.t[LU], &l = kG.t[LL];
+    c.ztab.assign((size_t)u.n * l.n, (short)C::zwords);
+    for (int j = 0; j < u.n; j++)
+        for (int jl = 0; jl < l.n; jl++) {
+            const int hu = u.h[j], hl = l.h[jl];
+            const int r3 = hidx(kH.t[hu] + kH.t[hl], kH.u[hu] + kH.u[hl], kH.v[hu] + kH.v[hl]);
+            const int z = z_position(LU, C::sl, u.sig[j], l.sig[jl], r3);
+            if (z >= 0) c.ztab[(size_t)j * l.n + jl] = (short)z;
+        }
+    if constexpr (PASS + 1 < npass(LU, LL)) add_class<LU, LL, PASS + 1>(t);
 }
 
-template <int LU>
-bool launch_shell_u(int LL, int clb, bool red, unsigned grid, hipStream_t st, const PP &pp,
-                    const SPD &sd, const ShellItem *items, double *part)
+const ClassInfo *class_table()
 {
-    switch (LL) {
-    case 0: return launch_shell_t<LU, 0>(clb, red, grid, st, pp, sd, items, part);
-    case 1: return launch_shell_t<LU, 1>(clb, red, grid, st, pp, sd, items, part);
-    case 2: return launch_shell_t<LU, 2>(clb, red, grid, st, pp, sd, items, part);
-    case 3: return launch_shell_t<LU, 3>(clb, red, grid, st, pp, sd, items, part);
-    case 4: return launch_shell_t<LU, 4>(clb, red, grid, st, pp, sd, items, part);
-    }
-    return false;
-}
-
-bool launch_shell(int LU, int LL, int clb, bool red, unsigned grid, hipStream_t st,
-                  const PP &pp, const SPD &sd, const ShellItem *items, double *part)
-{
-    switch (LU) {
-    case 0: return launch_shell_u<0>(LL, clb, red, grid, st, pp, sd, items, part);
-    case 1: return launch_shell_u<1>(LL, clb, red, grid, st, pp, sd, items, part);
-    case 2: return launch_shell_u<2>(LL, clb, red, grid, st, pp, sd, items, part);
-    case 3: return launch_shell_u<3>(LL, clb, red, grid, st, pp, sd, items, part);
-    case 4: return launch_shell_u<4>(LL, clb, red, grid, st, pp, sd, items, part);
-    }
-    return false;
+    static ClassInfo *t = [] {
+        static ClassInfo tab[kNB];
+        add_class<0, 0, 0>(tab);
+        add_class<0, 1, 0>(tab);
+        add_class<0, 2, 0>(tab);
+        add_class<0, 3, 0>(tab);
+        add_class<0, 4, 0>(tab);
+        add_class<1, 1, 0>(tab);
+        add_class<1, 2, 0>(tab);
+        add_class<1, 3, 0>(tab);
+        add_class<1, 4, 0>(tab);
+        add_class<2, 2, 0>(tab);
+        add_class<2, 3, 0>(tab);
+        add_class<2, 4, 0>(tab);
+        add_class<3, 3, 0>(tab);
+        add_class<3, 4, 0>(tab);
+        add_class<4, 4, 0>(tab);
+        return tab;
+    }();
+    return t;
 }
 
 inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
-inline int hc(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
 
 // Boys values, R recursion (2 FMA per entry over all levels) and prefactor
 double boys_r_flops(int L)
@@ -808,35 +771,7 @@ double boys_r_flops(int L)
     return 25.0 + 3.0 * (L + 1) + 4.0 * (HR4 - 1.0) + 12.0;
 }
 
-// X contraction and scaling per primitive quartet and lane component with
-// nz nonzero Hermite coefficients
-double x_flops(int LU, double nz) { return 2.0 * hc(LU) * nz + hc(LU); }
-
-// nonzero Hermite coefficients of the lane components [l0, l1) of shell pair s
-int64_t lane_nz(const zv_context *c, int s, int l0, int l1)
-{
-    return c->h_sp_nzcum[c->h_sp_coff[s] + l1] - c->h_sp_nzcum[c->h_sp_coff[s] + l0];
-}
-
-// uniform components per item and the smallest count that uses the
-// reduction mode
-constexpr int kMaxUDirect = ZV_MAXU, kMaxURed = 64, kRedMin = kDirectMaxU + 1;
-
-// Estimated kernel cost of finishing, in lane flop-equivalents: the direct
-// mode per primitive quartet and pass (scalar-operand FMAs run about three
-// times slower than register-only work); the reduction mode per uniform
-// primitive pair and pass (LDS transpose, row sums, two barriers and the
-// load of the uniform E, mostly latency at one wave per SIMD).
-double finish_direct(int LU, int clb, int nu) { return 3.0 * 2.0 * nu * clb * hc(LU); }
-double finish_red(int LU, int clb)
-{
-    const double NR = clb * hc(LU);
-    return 64.0 * (4.0 * NR + 128.0 * std::ceil(NR / 64.0)) + 40000.0;
-}
-
-// bucket b = 25 (2 (clb - 1) + red) + 5 LU + LL
-constexpr int kNB = 25 * 2 * kClbMax;
-
+// ------------------------------------------------------------------ planner
 // A plan's items (bucket b at [lo[b], lo[b + 1])) and groups live in the
 // caller's host buffer (items, then groups), from which they are copied to
 // the device as they are.
@@ -849,95 +784,22 @@ struct Plan {
     int64_t npart = 0;
     double units[kNB] = {}, flops[kNB] = {}; // per bucket
     double host_ms[4] = {};                  // orientation, items, join, bucket sort
-    bool bad = false;                        // an item the kernels cannot take
 };
 
-// lane components [0, full) run in passes of the class's batch limit, the
-// remainder [full, ncl) in one pass
-inline int lane_batch(int LU, int LL, bool red)
-{
-    return red ? kShellClbRed[LU][LL] : kShellClb[LU][LL];
-}
-inline int full_passes_end(int LU, int LL, int ncl, bool red)
-{
-    const int b = lane_batch(LU, LL, red);
-    return ncl / b * b;
-}
+inline int nchunk(int np) { return (np + kLaneC - 1) / kLaneC; }
+inline int nstep(int np) { return (np + kStepA - 1) / kStepA; }
 
-// uniform-component ranges of one orientation: ranges of kMaxURed (reduction
-// mode, from kRedMin components on) or kMaxUDirect components; a short tail
-// of a reduction-mode pair below kRedMin runs in direct mode
-inline int uniform_step(int ncu) { return ncu >= kRedMin ? kMaxURed : kMaxUDirect; }
-inline bool uniform_red(int ncu, int nu) { return ncu >= kRedMin && nu >= kRedMin; }
-
-// Kernel-time cost model of (U|L): lanes padded to 64, Boys and R redone per
-// pass of lane components and per uniform range; nz: mean nonzero Hermite
-// coefficients of a lane component.
-double pass_cost(int LU, int LL, int clb, int nu, bool red, double npu, double lanes, double nz)
+// Estimated cycles of one pass over a shell quartet and of its transform to
+// the components.
+double quartet_cost(const ClassInfo &ci, int npu, int npl)
 {
-    const double work = lanes * npu * (boys_r_flops(LU + LL) + clb * x_flops(LU, nz));
-    return work + (red ? npu * finish_red(LU, clb) : lanes * npu * finish_direct(LU, clb, nu));
+    return nchunk(npl) * (nstep(npu) * ci.step + ci.chunk);
 }
-
-double item_cost_of(int LU, int LL, int ncu, int ncl, double npu, double lanes)
+double transform_cost(int LU, int LL, int ncu, int ncl)
 {
-    const double nz = hc(LL);
-    const int step = uniform_step(ncu);
-    double cost = 0.0;
-    for (int cu0 = 0; cu0 < ncu; cu0 += step) {
-        const int nu = std::min(step, ncu - cu0);
-        const bool red = uniform_red(ncu, nu);
-        const int bm = lane_batch(LU, LL, red), n2 = full_passes_end(LU, LL, ncl, red);
-        cost += n2 / bm * pass_cost(LU, LL, bm, nu, red, npu, lanes, nz);
-        if (ncl > n2) cost += pass_cost(LU, LL, ncl - n2, nu, red, npu, lanes, nz);
-    }
-    return cost;
+    const double gu = kG.t[LU].n, gl = kG.t[LL].n;
+    return 2500.0 + 12.0 * (ncu * gl * gu + (double)ncu * ncl * gl) / 64.0;
 }
-
-// The planned cost of an orientation is npu (lanes A + B) with A and B fixed
-// by the (order, components) types of the uniform and the lane shell pair
-// (pass_cost is linear in npu and lanes), tabulated once per plan.
-struct CostTable {
-    std::vector<int> type;        // per shell pair
-    std::vector<double> npu, lanes; // per shell pair
-    std::vector<double> A, B;     // [type u][type l]
-    int nt = 0;
-    explicit CostTable(const zv_context *c)
-    {
-        const int nsp = c->nsp;
-        std::vector<std::pair<int, int>> keys;
-        type.resize(nsp);
-        npu.resize(nsp);
-        lanes.resize(nsp);
-        for (int s = 0; s < nsp; s++) {
-            const std::pair<int, int> k{c->h_sp_L[s], c->h_sp_coff[s + 1] - c->h_sp_coff[s]};
-            auto it = std::find(keys.begin(), keys.end(), k);
-            type[s] = (int)(it - keys.begin());
-            if (it == keys.end()) keys.push_back(k);
-            npu[s] = c->h_sp_np[s];
-            lanes[s] = std::ceil(c->h_sp_np[s] / 64.0) * 64.0;
-        }
-        nt = (int)keys.size();
-        A.resize((size_t)nt * nt);
-        B.resize((size_t)nt * nt);
-        for (int u = 0; u < nt; u++)
-            for (int l = 0; l < nt; l++) {
-                const auto [LU, ncu] = keys[u];
-                const auto [LL, ncl] = keys[l];
-                // shell quartets of these orders only (the others go through
-                // component lists and have no shell kernel)
-                if (LU > ZV_LMAX_T || LL > ZV_LMAX_T) continue;
-                const double b = item_cost_of(LU, LL, ncu, ncl, 1.0, 0.0);
-                A[(size_t)u * nt + l] = item_cost_of(LU, LL, ncu, ncl, 1.0, 1.0) - b;
-                B[(size_t)u * nt + l] = b;
-            }
-    }
-    double cost(int su, int sl) const
-    {
-        const size_t k = (size_t)type[su] * nt + type[sl];
-        return npu[su] * (lanes[sl] * A[k] + B[k]);
-    }
-};
 
 // Host threads for the planner: up to 16 (the host share of one GPU), one
 // for short lists.
@@ -983,85 +845,50 @@ struct Orient {
 
 void plan_items(const zv_context *c, const Orient *ors, size_t n, double budget, PlanPart &pp)
 {
+    const ClassInfo *ct = class_table();
     for (size_t q = 0; q < n; q++) {
         const Orient &o = ors[q];
-        const int LU = c->h_sp_L[o.su], LL = c->h_sp_L[o.sl], L = LU + LL;
+        const int LU = c->h_sp_L[o.su], LL = c->h_sp_L[o.sl];
         const int ncu = c->h_sp_coff[o.su + 1] - c->h_sp_coff[o.su];
         const int ncl = c->h_sp_coff[o.sl + 1] - c->h_sp_coff[o.sl];
         const int npu = c->h_sp_np[o.su], npl = c->h_sp_np[o.sl];
-        const double lanes = std::ceil(npl / 64.0) * 64.0;
-        const int k = 5 * LU + LL;
-        const double HU = hc(LU);
-        const double nz = hc(LL);
-        const int step = uniform_step(ncu);
-        bool br_counted = false; // Boys and R counted once per shell quartet
-        for (int cu0 = 0; cu0 < ncu; cu0 += step) {
-            const int nu = std::min(step, ncu - cu0);
-            const bool red = uniform_red(ncu, nu);
-            const int bm = lane_batch(LU, LL, red), n2 = full_passes_end(LU, LL, ncl, red);
-            // segment [0, n2) in passes of bm components, [n2, ncl) in one pass
-            for (int seg = 0; seg < 2; seg++) {
-                const int clb = seg == 0 ? bm : ncl - n2;
-                const int s0 = seg == 0 ? 0 : n2, s1 = seg == 0 ? n2 : ncl;
-                if (clb <= 0) continue;
-                const int npass = (s1 - s0) / clb;
-                if (npass <= 0) continue;
-                const double wp = pass_cost(LU, LL, clb, nu, red, npu, lanes, nz); // per pass
-                const int k1 = (int)std::min<double>(
-                    npass, std::max(1.0, std::ceil(npass * wp / budget)));
-                const int b = 25 * (2 * (clb - 1) + (red ? 1 : 0)) + k;
-                for (int r = 0; r < k1; r++) {
-                    const int p0 = (int)((int64_t)npass * r / k1);
-                    const int p1 = (int)((int64_t)npass * (r + 1) / k1);
-                    const int l0 = s0 + p0 * clb, l1 = s0 + p1 * clb;
-                    const int nlr = l1 - l0;
-                    const double cr = (p1 - p0) * wp;
-                    const int ns =
-                        (int)std::min<double>(npu, std::max(1.0, std::ceil(cr / budget)));
-                    pp.groups.push_back(ShellGroup{o.su, o.sl, cu0, nu, l0, nlr, ns, 0, pp.npart});
-                    // algorithmic flops: Boys and R once per primitive quartet
-                    // (however many lane passes redo them); per lane component
-                    // the X contraction over its nonzero Hermite coefficients,
-                    // then either nu direct dot products per primitive quartet
-                    // or the sum over lane primitives per primitive quartet
-                    // plus nu dot products per uniform primitive
-                    const double pq = (double)npu * npl;
-                    pp.units[b] += pq * nlr;
-                    const double xf =
-                        2.0 * HU * (double)lane_nz(c, o.sl, l0, l1) + nlr * HU; // sum of x_flops
-                    double fl = pq * ((br_counted ? 0.0 : boys_r_flops(L)) + xf);
-                    br_counted = true;
-                    fl += red ? nlr * (pq * HU + (double)npu * 2.0 * nu * HU)
-                              : nlr * pq * 2.0 * nu * HU;
-                    pp.flops[b] += fl;
-                    for (int sl = 0; sl < ns; sl++) {
-                        const int a0 = (int)((int64_t)npu * sl / ns);
-                        const int a1 = (int)((int64_t)npu * (sl + 1) / ns);
-                        pp.tmp[b].push_back(ShellItem{o.su, o.sl, a0, a1, l0, l1, cu0, nu,
-                                                      pp.npart + (int64_t)sl * nu * nlr});
-                        pp.tcost[b].push_back((float)(cr * (a1 - a0) / npu));
-                    }
-                    pp.npart += (int64_t)ns * nu * nlr;
+        const int nk = nchunk(npl), nst = nstep(npu), nc = ncu * ncl;
+        // slices of chunks first (they repeat the transform only), then of steps;
+        // none much shorter than the transform that it repeats
+        const double least = 3.0 * transform_cost(LU, LL, ncu, ncl);
+        const double want = std::ceil(o.cost / std::max(budget, least));
+        const int kc = (int)std::min<double>(nk, std::max(1.0, want));
+        const int ks = (int)std::min<double>(nst, std::max(1.0, std::ceil(want / kc)));
+        const int np = npass(LU, LL);
+        pp.groups.push_back(ShellGroup{o.su, o.sl, kc * ks * np, 0, pp.npart});
+        const double pq = (double)npu * npl;
+        for (int p = 0; p < np; p++) {
+            const int b = bucket_of(LU, LL, p);
+            const double cost = quartet_cost(ct[b], npu, npl) / (kc * ks);
+            // algorithmic flops: Boys and R once per primitive quartet, one
+            // multiply-add per needed (sigma, row)
+            if (p == 0) pp.units[b] += pq;
+            pp.flops[b] += pq * ((p == 0 ? boys_r_flops(LU + LL) : 0.0) + 2.0 * ct[b].acc);
+            for (int i = 0; i < kc; i++)
+                for (int j = 0; j < ks; j++) {
+                    pp.tmp[b].push_back(ShellItem{o.su, o.sl, (int)((int64_t)nst * j / ks),
+                                                  (int)((int64_t)nst * (j + 1) / ks),
+                                                  (int)((int64_t)nk * i / kc),
+                                                  (int)((int64_t)nk * (i + 1) / kc), pp.npart});
+                    pp.tcost[b].push_back((float)cost);
+                    pp.npart += nc;
                 }
-            }
         }
     }
 }
 
 // Orientation, splitting and ordering of a list of shell quartets (x, y),
-// both shell pairs of order <= ZV_LMAX_T with kept primitive pairs.  Items
-// are cut along lane-component passes first (no extra work), then along
-// uniform primitive-pair slices (partial sums added by the scatter).  Long
-// lists are planned on host threads over contiguous runs of quartets whose
-// items are joined in order, so the plan is the same for any thread count.
-// the kernels assume whole lane passes (no guard per lane component) and,
-// in direct mode, at most kDirectMaxU uniform components
-inline bool item_ok(const ShellItem &it, int clb, bool red)
-{
-    return it.cl1 > it.cl0 && (it.cl1 - it.cl0) % clb == 0 &&
-           (red || (it.nu >= 1 && it.nu <= kDirectMaxU));
-}
-
+// both shell pairs of order <= ZV_LMAX_T with kept primitive pairs.  The
+// uniform side is the pair of lower order (fewer sigma, so fewer
+// accumulators per row), of equal ones the cheaper by padded steps and
+// chunks.  Long lists are planned on host threads over contiguous runs of
+// quartets whose items are joined in order, so the plan is the same for any
+// thread count.
 void plan_shell(const zv_context *c, const std::vector<std::pair<int, int>> &sq, Plan &pl,
                 std::vector<char> &hbuf)
 {
@@ -1072,12 +899,21 @@ void plan_shell(const zv_context *c, const std::vector<std::pair<int, int>> &sq,
     auto tt = clk::now();
     const size_t nq = sq.size();
     const int nt = plan_threads(nq);
-    const CostTable ct(c);
+    const ClassInfo *ct = class_table();
     std::vector<Orient> ors(nq);
     run_threads(nt, [&](int t) {
         for (size_t q = nq * t / nt; q < nq * (t + 1) / nt; q++) {
-            const int x = sq[q].first, y = sq[q].second;
-            double cxy = ct.cost(x, y), cyx = x == y ? cxy : ct.cost(y, x);
+            int x = sq[q].first, y = sq[q].second;
+            if (c->h_sp_L[x] > c->h_sp_L[y]) std::swap(x, y);
+            const int LU = c->h_sp_L[x], LL = c->h_sp_L[y];
+            auto cost = [&](int u, int l) {
+                double s = transform_cost(LU, LL, c->h_sp_coff[u + 1] - c->h_sp_coff[u],
+                                          c->h_sp_coff[l + 1] - c->h_sp_coff[l]);
+                for (int p = 0; p < npass(LU, LL); p++)
+                    s += quartet_cost(ct[bucket_of(LU, LL, p)], c->h_sp_np[u], c->h_sp_np[l]);
+                return s;
+            };
+            const double cxy = cost(x, y), cyx = LU == LL && x != y ? cost(y, x) : cxy;
             ors[q] = cxy <= cyx ? Orient{x, y, cxy} : Orient{y, x, cyx};
         }
     });
@@ -1087,7 +923,7 @@ void plan_shell(const zv_context *c, const std::vector<std::pair<int, int>> &sq,
     // so the sorted queue ends on short items
     const double nitems =
         c->tune[ZV_TUNE_ERI_ITEMS] > 0 ? (double)c->tune[ZV_TUNE_ERI_ITEMS] : 40000.0;
-    const double budget = std::max(total / nitems, 2.0e6);
+    const double budget = std::max(total / nitems, 20000.0);
     pl.host_ms[0] = ms_since(tt);
     tt = clk::now();
     std::vector<PlanPart> parts(nt);
@@ -1142,7 +978,6 @@ void plan_shell(const zv_context *c, const std::vector<std::pair<int, int>> &sq,
     // independent and spread over the threads
     constexpr int NBIN = 256;
     static_assert(NBIN <= 256, "bins are stored as bytes");
-    std::vector<char> bad(nt, 0);
     run_threads(nt, [&](int t) {
         std::vector<uint8_t> bin;
         std::vector<const ShellItem *> src;
@@ -1150,8 +985,6 @@ void plan_shell(const zv_context *c, const std::vector<std::pair<int, int>> &sq,
         for (int b = t; b < kNB; b += nt) {
             const size_t n = nb_items[b];
             if (!n) continue;
-            const int clb = b / 50 + 1;
-            const bool red = ((b / 25) & 1) != 0;
             src.clear();
             cst.clear();
             std::vector<int64_t> shift;
@@ -1172,107 +1005,94 @@ void plan_shell(const zv_context *c, const std::vector<std::pair<int, int>> &sq,
             for (size_t i = 0; i < n; i++) {
                 ShellItem it = *src[i];
                 it.part += shift[i];
-                if (!item_ok(it, clb, red)) bad[t] = 1;
                 pl.items[pl.lo[b] + cnt[bin[i]]++] = it;
             }
         }
     });
-    for (char x : bad) pl.bad = pl.bad || x;
     pl.host_ms[3] = ms_since(tt);
 }
 
 } // namespace
 
 // ====================================================================== host
-static SPD spd_of(zv_context *c);
+// Device layout of the shell-pair tables in b_spmeta: roff[nsp], goff[nsp]
+// (int64), comp[npair], coff[nsp + 1], np[nsp], component -> shell pair
+// [npair] (int); b_spu: primitive rows; b_spe: the two expansion tables.
+static SPD spd_of(zv_context *c)
+{
+    const int64_t *d_roff = (const int64_t *)c->b_spmeta.p;
+    const int64_t *d_goff = d_roff + c->nsp;
+    const int *d_comp = (const int *)(d_goff + c->nsp);
+    const int *d_coff = d_comp + c->npair;
+    const int *d_np = d_coff + c->nsp + 1;
+    const double *g = (const double *)c->b_spe.p;
+    return SPD{d_comp, d_coff, d_np, d_roff, d_goff, (const double *)c->b_spu.p, g,
+               g + c->sp_g_total};
+}
 
-// Shell-pair tables on the device and the AoS copies of the uniform side.
 int zv_shell_ready(zv_context *c, const PP &pp)
 {
-    const int nsp = c->nsp;
-    size_t meta =
-        sizeof(int) * (2 * (size_t)c->npair + nsp + 1) + sizeof(int64_t) * 2 * nsp + 64;
+    const int nsp = c->nsp, np = c->npair;
+    size_t meta = sizeof(int64_t) * 2 * nsp + sizeof(int) * (2 * (size_t)np + 2 * nsp + 1) + 64;
     ZV_CHECK(zv_ensure(c, c->b_spmeta, meta));
     if (c->sp_ready) return ZV_OK;
-    // Hermite pattern of each component with a shell-kernel order
-    c->h_sp_cpat.assign(c->npair, 0);
-    for (int q = 0; q < c->npair; q++) {
-        const int P = c->h_sp_comp[q];
-        const int L = c->h_pair_L[P];
-        if (L > ZV_LMAX_T) continue;
-        const int i = c->h_pair_i[P] - 1, k = c->h_pair_k[P] - 1;
-        int S[3], deg = 0;
-        for (int d = 0; d < 3; d++) {
-            S[d] = c->h_npower[3 * i + d] + c->h_npower[3 * k + d];
-            deg += S[d];
+    // Z positions of every class and pass, once per context
+    if (!c->ztab_ready) {
+        const ClassInfo *ct = class_table();
+        std::vector<short> all;
+        c->h_ztab_off.assign(kNB, 0);
+        for (int b = 0; b < kNB; b++) {
+            c->h_ztab_off[b] = (int64_t)all.size();
+            all.insert(all.end(), ct[b].ztab.begin(), ct[b].ztab.end());
         }
-        const int nr = (c->h_itype[i] == 2) + (c->h_itype[k] == 2);
-        const int pid = deg + 2 * nr == L ? kHP.find(L, herm_union(S[0], S[1], S[2], nr)) : -1;
-        if (pid < 0)
-            return zv_fail(c, ZV_ERR_STATE, "AO pair %d: no Hermite pattern of order %d", P, L);
-        c->h_sp_cpat[q] = pid | kHP.nz[L][pid] << 8;
+        ZV_CHECK(zv_ensure(c, c->b_ztab, sizeof(short) * all.size()));
+        ZV_HIPCHECK(c, hipMemcpy(c->b_ztab.p, all.data(), sizeof(short) * all.size(),
+                                 hipMemcpyHostToDevice));
+        c->ztab_ready = true;
     }
-    c->h_sp_nzcum.assign(c->npair + 1, 0);
-    for (int q = 0; q < c->npair; q++)
-        c->h_sp_nzcum[q + 1] = c->h_sp_nzcum[q] + (c->h_sp_cpat[q] >> 8);
-    std::vector<int64_t> puoff(nsp), euoff(nsp);
+    std::vector<int64_t> off(2 * (size_t)nsp);
+    int64_t *roff = off.data(), *goff = roff + nsp;
+    std::vector<int> tab;
+    tab.reserve(2 * (size_t)np + 2 * nsp + 1);
+    tab.insert(tab.end(), c->h_sp_comp.begin(), c->h_sp_comp.end());
+    tab.insert(tab.end(), c->h_sp_coff.begin(), c->h_sp_coff.end());
     c->h_sp_np.assign(nsp, 0);
-    int64_t pu_tot = 0, eu_tot = 0;
+    int64_t r_tot = 0, g_tot = 0;
     for (int s = 0; s < nsp; s++) {
-        const int c0 = c->h_sp_coff[s], nc = c->h_sp_coff[s + 1] - c0;
-        const int np = c->h_cnt[c->h_sp_comp[c0]];
-        c->h_sp_np[s] = np;
-        puoff[s] = pu_tot;
-        euoff[s] = eu_tot;
-        pu_tot += 8 * (int64_t)np;
-        eu_tot += (int64_t)np * nc * hc(c->h_sp_L[s]);
+        const int c0 = c->h_sp_coff[s], nc = c->h_sp_coff[s + 1] - c0, L = c->h_sp_L[s];
+        const int n = c->h_cnt[c->h_sp_comp[c0]];
+        c->h_sp_np[s] = n;
+        tab.push_back(n);
+        roff[s] = r_tot;
+        goff[s] = g_tot;
+        if (L > ZV_LMAX_T) continue;
+        r_tot += (int64_t)nchunk(n) * kLaneC * kRow[L];
+        g_tot += (int64_t)nc * kG.t[L].n;
     }
-    ZV_CHECK(zv_ensure(c, c->b_spu, sizeof(double) * std::max<int64_t>(pu_tot, 1)));
-    // two layouts of the uniform-side E: [a][comp][h] then [a][h][comp]
-    ZV_CHECK(zv_ensure(c, c->b_spe, sizeof(double) * std::max<int64_t>(2 * eu_tot, 1)));
-    ZV_CHECK(zv_ensure(c, c->b_spec, sizeof(double) * std::max<int64_t>(c->e_total, 1)));
-    c->sp_eu_total = eu_tot;
-    int64_t *d_puoff = (int64_t *)c->b_spmeta.p;
-    int64_t *d_euoff = d_puoff + nsp;
-    int *d_comp = (int *)(d_euoff + nsp);
-    int *d_coff = d_comp + c->npair;
-    int *d_cpat = d_coff + nsp + 1;
-    ZV_HIPCHECK(c, hipMemcpyAsync(d_puoff, puoff.data(), sizeof(int64_t) * nsp,
+    for (int s = 0; s < nsp; s++)
+        for (int q = c->h_sp_coff[s]; q < c->h_sp_coff[s + 1]; q++) tab.push_back(s);
+    ZV_CHECK(zv_ensure(c, c->b_spu, sizeof(double) * std::max<int64_t>(r_tot, 1)));
+    ZV_CHECK(zv_ensure(c, c->b_spe, sizeof(double) * std::max<int64_t>(2 * g_tot, 1)));
+    c->sp_g_total = g_tot;
+    char *m = (char *)c->b_spmeta.p;
+    ZV_HIPCHECK(c, hipMemcpyAsync(m, off.data(), sizeof(int64_t) * off.size(),
                                   hipMemcpyHostToDevice, c->stream));
-    ZV_HIPCHECK(c, hipMemcpyAsync(d_euoff, euoff.data(), sizeof(int64_t) * nsp,
-                                  hipMemcpyHostToDevice, c->stream));
-    ZV_HIPCHECK(c, hipMemcpyAsync(d_comp, c->h_sp_comp.data(), sizeof(int) * c->npair,
-                                  hipMemcpyHostToDevice, c->stream));
-    ZV_HIPCHECK(c, hipMemcpyAsync(d_coff, c->h_sp_coff.data(), sizeof(int) * (nsp + 1),
-                                  hipMemcpyHostToDevice, c->stream));
-    ZV_HIPCHECK(c, hipMemcpyAsync(d_cpat, c->h_sp_cpat.data(), sizeof(int) * c->npair,
-                                  hipMemcpyHostToDevice, c->stream));
-    SPD sd = spd_of(c);
+    ZV_HIPCHECK(c, hipMemcpyAsync(m + sizeof(int64_t) * off.size(), tab.data(),
+                                  sizeof(int) * tab.size(), hipMemcpyHostToDevice, c->stream));
+    const SPD sd = spd_of(c);
     {
         PhaseTimer tm(c, PH_PRIM);
-        hipLaunchKernelGGL(k_shellpairs, dim3(nsp), dim3(256), 0, c->stream, pp, sd,
-                           (double *)c->b_spu.p, (double *)c->b_spe.p,
-                           (double *)c->b_spe.p + eu_tot);
+        hipLaunchKernelGGL(k_pair_rows, dim3(nsp), dim3(128), 0, c->stream, pp, sd,
+                           (double *)c->b_spu.p);
         ZV_HIPCHECK(c, hipGetLastError());
-        hipLaunchKernelGGL(k_compact_e, dim3(c->npair), dim3(256), 0, c->stream, pp, sd,
-                           (double *)c->b_spec.p);
+        hipLaunchKernelGGL(k_expansion, dim3(np), dim3(64), 0, c->stream, pp, sd, sd.np + nsp,
+                           c->d_pair_i, c->d_pair_k, c->d_center, c->d_npower, c->d_itype,
+                           (double *)c->b_spe.p, (double *)c->b_spe.p + g_tot);
         ZV_HIPCHECK(c, hipGetLastError());
     }
     ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
     c->sp_ready = true;
     return ZV_OK;
-}
-
-static SPD spd_of(zv_context *c)
-{
-    int64_t *d_puoff = (int64_t *)c->b_spmeta.p;
-    int64_t *d_euoff = d_puoff + c->nsp;
-    int *d_comp = (int *)(d_euoff + c->nsp);
-    int *d_coff = d_comp + c->npair;
-    const int *d_cpat = d_coff + c->nsp + 1;
-    const double *eu = (const double *)c->b_spe.p;
-    return SPD{d_comp, d_coff, d_puoff, d_euoff, (const double *)c->b_spu.p, eu,
-               eu + c->sp_eu_total, d_cpat, (const double *)c->b_spec.p};
 }
 
 // Plan and launch the shell kernels of one Schwarz phase over the shell
@@ -1288,17 +1108,6 @@ int zv_shell_run(zv_context *c, const PP &pp, const std::vector<std::pair<int, i
     const auto t1 = clk::now();
     *ngroups = (int64_t)pl.ngroups;
     if (!pl.nitems) return ZV_OK;
-    if (pl.bad) {
-        // the first offending item, for the message
-        for (int b = 0; b < kNB; b++)
-            for (int t = pl.lo[b]; t < pl.lo[b + 1]; t++) {
-                const ShellItem &it = pl.items[t];
-                if (!item_ok(it, b / 50 + 1, ((b / 25) & 1) != 0))
-                    return zv_fail(c, ZV_ERR_STATE, "shell item with lane components [%d, %d) "
-                                   "and %d uniform components in bucket %d", it.cl0, it.cl1,
-                                   it.nu, b);
-            }
-    }
     const size_t bi = sizeof(ShellItem) * pl.nitems;
     const size_t bg = sizeof(ShellGroup) * pl.ngroups;
     const auto t2 = clk::now();
@@ -1317,13 +1126,14 @@ int zv_shell_run(zv_context *c, const PP &pp, const std::vector<std::pair<int, i
                 pl.host_ms[1], pl.host_ms[2], pl.host_ms[3], ms(t3 - t2));
     }
     const SPD sd = spd_of(c);
+    const ClassInfo *ct = class_table();
     const ShellItem *di = (const ShellItem *)bitem.p;
     // The buckets write disjoint partial sums, so they run side by side on
     // the context's stream and its side streams (a bucket's last items leave
     // CUs idle that the next bucket fills), joined back before the scatter.
     // Largest planned cost first, each to the stream with the least planned
     // cost so far.
-    // bucket b = 25 v + 5 LU + LL, v = 2 (clb - 1) + red: statistics slot 36 + b
+    // bucket b = 50 pass + 5 LU + LL: statistics slot 36 + b
     static_assert(36 + kNB <= ZV_NSTAT, "statistics slots");
     constexpr int NST = 1 + zv_context::NSIDE;
     hipStream_t sts[NST] = {c->stream};
@@ -1342,7 +1152,6 @@ int zv_shell_run(zv_context *c, const PP &pp, const std::vector<std::pair<int, i
     for (int t = 0; t < nb; t++) {
         const int b = order[t];
         const int n = pl.lo[b + 1] - pl.lo[b];
-        const int v = b / 25, k = b % 25, LU = k / 5, LL = k % 5;
         const int cls = 36 + b;
         c->cls_pq[cls] += pl.units[b];
         c->cls_flops[cls] += pl.flops[b];
@@ -1355,9 +1164,10 @@ int zv_shell_run(zv_context *c, const PP &pp, const std::vector<std::pair<int, i
             if (load[q] < load[s]) s = q;
         load[s] += pl.flops[b];
         PhaseTimer tm(c, PH_N, cls, sts[s]);
-        if (!launch_shell(LU, LL, v / 2 + 1, (v & 1) != 0, (unsigned)n, sts[s], pp, sd,
-                          di + pl.lo[b], (double *)bpart.p))
-            return zv_fail(c, ZV_ERR_STATE, "no shell kernel for (%d,%d)", LU, LL);
+        if (!ct[b].launch) return zv_fail(c, ZV_ERR_STATE, "no shell kernel for bucket %d", b);
+        ct[b].launch(LaunchArgs{sd, di + pl.lo[b], n, pp.btab,
+                                (const short *)c->b_ztab.p + c->h_ztab_off[b],
+                                (double *)bpart.p, sts[s]});
         ZV_HIPCHECK(c, hipGetLastError());
     }
     for (int k = 0; k < zv_context::NSIDE; k++) {

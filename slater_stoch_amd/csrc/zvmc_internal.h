@@ -17,7 +17,6 @@
 #define ZV_LMAX_T 4    // largest pair angular momentum with a templated ERI kernel
 #define ZV_LPAIR_MAX 8 // largest pair angular momentum supported at all
 #define ZV_SHMAX 15    // largest shell (Cartesian components sharing one Gaussian fit)
-#define ZV_MAXU 36     // components of the uniform side handled by one shell work item
 #define ZV_NSTAT 236   // ERI statistics slots (component and shell kernel variants)
 
 struct DevBuf {
@@ -93,14 +92,14 @@ struct zv_context {
     DevBuf b_part;                     // split partial sums
     DevBuf b_misc;
     bool pp_ready = false;
-    // shell-pair data: component tables and the uniform-side copies
-    DevBuf b_spmeta;                   // puoff[nsp], euoff[nsp], comp[npair], coff[nsp+1], cpat[npair]
-    DevBuf b_spu, b_spe;               // per primitive pair: p,1/p,P,c; E [a][comp][h]
-    DevBuf b_spec;                     // lane-side E without structural zeros (k_compact_e)
+    // shell-pair data
+    DevBuf b_spmeta;                   // offsets, component tables (spd_of, k_eri_shell.hip)
+    DevBuf b_spu, b_spe;               // primitive-pair rows; expansion tables of the components
+    DevBuf b_ztab;                     // Z positions of every shell-kernel class and pass
+    bool ztab_ready = false;
+    std::vector<int64_t> h_ztab_off;   // start of each class and pass in b_ztab
     std::vector<int> h_sp_np;          // kept primitive pairs per shell pair
-    std::vector<int> h_sp_cpat;        // per component: Hermite pattern | nonzero count << 8
-    std::vector<int64_t> h_sp_nzcum;   // running sum of the components' nonzero counts
-    int64_t sp_eu_total = 0;           // doubles of one uniform-side E layout
+    int64_t sp_g_total = 0;            // doubles of one expansion table
     bool sp_ready = false;
     // group-blocked estimator: units of 1, 3 or 6 components of one shell
     // pair per class, tiles per pair of classes (built on first use per basis)
@@ -129,7 +128,7 @@ struct zv_context {
     int64_t t_n[PH_N] = {};
     std::vector<int> pend_cls;        // ERI class of each pending timer (-1: none)
     // ERI statistics: [0, 36) component kernels 6 LB + LK; [36, 236) shell
-    // kernels 36 + 25 v + 5 LU + LL, v = 2 (lane batch - 1) + reduction mode
+    // kernels 36 + 50 pass + 5 LU + LL
     double cls_ms[ZV_NSTAT] = {};
     int64_t cls_n[ZV_NSTAT] = {};
     double cls_pq[ZV_NSTAT] = {};     // primitive-quartet evaluations per class

@@ -1,0 +1,42 @@
+"""The shell-quartet ERI kernels against the CPU oracle at the edges of their
+tiles: the number of kept primitive pairs of a shell pair (ng^2 for AOs on one
+centre) below, at and above the step of 4 uniform-side and the chunk of 16
+lane-side primitive pairs, for every pair of shell-pair orders 0..4, each
+reached by products of different shells (p x p, d x s and r^2-type s x s are
+all of order 2)."""
+import numpy as np
+import pytest
+
+from slater_stoch_amd import basis as B
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def engine():
+    from slater_stoch_amd.zvmc import Engine
+    e = Engine(0)
+    yield e
+    e.close()
+
+
+# 1, 4, 9, 16, 25 and 49 primitive pairs on one centre; the tolerance is that
+# of the other comparisons with the oracle (its polynomial recursion loses
+# digits relative to the largest integral, not to each one)
+@pytest.mark.parametrize("ng", [1, 2, 3, 4, 5, 7])
+def test_shell_kernels_at_tile_edges(engine, oracle, ng):
+    geom = B.geometry_from_angstrom(["O", "H"], [[0.05, -0.1, 0.2], [0.7, 0.4, -0.5]])
+    basis = {"O": [("1S", 2.6), ("2S", 1.9), ("2P", 2.1), ("3D", 1.7)],
+             "H": [("1S", 1.2), ("3P", 1.4), ("4F", 1.8)]}
+    bas = B.expand_basis(geom, basis, ng0=ng)
+    engine.set_basis(bas)
+    eri, pre, _ = engine.gauss_eri()
+    orders = {key[1:3] for key in engine.eri_stats() if key[0] == "shell"}
+    assert orders == {(a, b) for a in range(5) for b in range(a, 5)}
+    q = B.quartet_mapping(bas.n)
+    rng = np.random.default_rng(ng)
+    keep = np.flatnonzero(np.abs(pre[q[2] - 1, q[0] - 1] * pre[q[3] - 1, q[1] - 1]) >= 1e-30)
+    pick = rng.choice(keep, 2500, replace=False)
+    oracle.set_basis(bas)
+    ref, _ = oracle.gauss_eri([a[pick] for a in q], None)
+    np.testing.assert_allclose(eri[pick], ref, rtol=1e-10, atol=1e-12 * np.abs(ref).max())
