@@ -421,6 +421,13 @@ static int ensure_boys_table(zv_context *c)
     return ZV_OK;
 }
 
+int zv_boys_table(zv_context *c, const double **tab)
+{
+    ZV_CHECK(ensure_boys_table(c));
+    *tab = (const double *)c->b_btab.p;
+    return ZV_OK;
+}
+
 static PP pp_view(zv_context *c)
 {
     PP pp;

@@ -185,6 +185,8 @@ int zv_run_draw(zv_context *c, uint64_t seed, uint64_t stream, int64_t m0, int64
 int zv_run_pair_samples(zv_context *c, int i, int k, int ns, const double *r1, const double *r2,
                         double *ut1, double *ut2, double *rho1, double *rho2, double *rhog1,
                         double *rhog2, double *jac1, double *jac2);
+// device copy of the Boys Taylor table (k_eri.hip), made on first use
+int zv_boys_table(zv_context *c, const double **tab);
 int zv_run_gauss_eri(zv_context *c, double *ijkl, double *precond, int64_t *n_screened);
 int zv_run_exact_monocenter(zv_context *c, double *ijkl, double *err, int64_t *n_mono);
 int zv_run_one_e(zv_context *c, int nnuc, const double *charge, const double *nuc, double *S,
