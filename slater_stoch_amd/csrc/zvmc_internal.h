@@ -85,6 +85,8 @@ struct zv_context {
     DevBuf b_pp;                       // primitive-pair data
     DevBuf b_btab;                     // Boys Taylor table (zv_boys_table)
     bool btab_ready = false;
+    DevBuf b_mono;                     // angular table of the one-centre integrals (k_mono.hip)
+    bool mono_ready = false;
     DevBuf b_ppE;                      // primitive-pair Hermite coefficients
     DevBuf b_ppcnt;                    // kept primitive pairs per AO pair
     DevBuf b_tri;                      // triangle-order ERIs
