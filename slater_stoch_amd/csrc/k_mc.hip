@@ -393,8 +393,8 @@ __global__ __launch_bounds__(256) void k_est_group(
     const T *__restrict__ comp, const T *__restrict__ grp, const int *__restrict__ urow_pos,
     const int *__restrict__ urow_sp, int nurow, const int *__restrict__ ucol_pos,
     const int *__restrict__ ucol_sp, int nucol, const int2 *__restrict__ tiles,
-    const int *__restrict__ pos_pair, int Mround, int mspan, int Mc, int npos, int nsp_pad,
-    double *__restrict__ acc, double *__restrict__ mpart, int64_t ntri)
+    const int *__restrict__ pos_pair, int Mround, int nsplit, int mspan, int bstride, int Mc,
+    int npos, int nsp_pad, double *__restrict__ acc, bool add, int64_t ntri)
 {
     constexpr int SUB = GroupSub<T>::SUB;
     constexpr int RU = 16 * TR, CU = 16 * TC, ROWS = RU * NR, COLS = CU * NC;
@@ -496,15 +496,21 @@ __global__ __launch_bounds__(256) void k_est_group(
         for (int k = 0; k < LV; k++)
             if (lv[k] >= 0) fU2[lv[k]] = vv[k];
     };
-    // SPLIT: sample split blockIdx.y covers [ms0, ms1); split 0 adds into
-    // acc, split s > 0 into row s - 1 of mpart (folded in at the end of the
-    // block).  Without splits the chunk is walked whole (a separate
-    // instantiation: the general bounds cost the FP32 kernels 15 %).
+    // Grid row y = block * nsplit + split: the samples of one Monte Carlo
+    // block of the chunk (bstride apart) or, with SPLIT, [ms0, ms1) of them,
+    // summed into row y of acc.  Without splits the block is walked whole (a
+    // separate instantiation: the general bounds cost the FP32 kernels 15 %).
+    acc += (size_t)blockIdx.y * ntri;
     int ms0 = 0, ms1 = Mround;
     if constexpr (SPLIT) {
-        ms0 = (int)blockIdx.y * mspan;
+        const int blk = (int)blockIdx.y / nsplit, sp = (int)blockIdx.y % nsplit;
+        comp += (size_t)blk * bstride;
+        grp += (size_t)blk * bstride;
+        ms0 = sp * mspan;
         ms1 = ms0 + mspan < Mround ? ms0 + mspan : Mround;
-        if (blockIdx.y > 0) acc = mpart + (size_t)(blockIdx.y - 1) * ntri;
+    } else {
+        comp += (size_t)blockIdx.y * bstride;
+        grp += (size_t)blockIdx.y * bstride;
     }
     if (ms0 < ms1) gload(ms0);
     for (int m0 = ms0; m0 < ms1; m0 += SUB) {
@@ -661,7 +667,8 @@ __global__ __launch_bounds__(256) void k_est_group(
                     const int Q = pos_pair[ucol_pos[gv] + c];
                     if (P >= Q) {
                         const size_t t = (size_t)zv_tri(P, Q);
-                        acc[t] = acc[t] + acc64[i * NR + r][j * NC + c];
+                        const double v = acc64[i * NR + r][j * NC + c];
+                        acc[t] = add ? acc[t] + v : v;
                     }
                 }
             }
@@ -774,23 +781,16 @@ __global__ void k_sel_zero(int64_t nsel, const int64_t *__restrict__ tri, double
 // ------------------------------------------------------------------ statistics
 // End of a block (src/two_e_slater.F90:463-481): x = e_S/npts - e_G/npts,
 // sums of x and x^2, accumulators cleared.
-// With sample splits, their nextra partial rows are added to e_S (in split
-// order) and cleared.
 __global__ void k_block_end(int64_t ntri, double f, double *accS, double *accG, double *s1,
-                            double *s2, double *blk, int nextra, double *mpart)
+                            double *s2, double *blk)
 {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntri) return;
-    double eS = accS[t];
-    for (int s = 0; s < nextra; s++) {
-        eS += mpart[(size_t)s * ntri + t];
-        mpart[(size_t)s * ntri + t] = 0.0;
-    }
-    double x = accG ? eS * f - accG[t] * f : eS * f;
+    double x = accS[t] * f - accG[t] * f;
     s1[t] = s1[t] + x;
     s2[t] = s2[t] + x * x;
     accS[t] = 0.0;
-    if (accG) accG[t] = 0.0;
+    accG[t] = 0.0;
     if (blk) blk[t] = x;
 }
 
@@ -821,6 +821,41 @@ __global__ void k_scatter_ref(int64_t ntri, const double *__restrict__ in, doubl
     tri_decode(t, P, Q);
     int i = pi[P], k = pk[P], j = pi[Q], l = pk[Q];
     out[zv_kcp(kbase, n, i, j, k, l)] = in[t];
+}
+
+// End of nb blocks of the group estimator: block b's sum is the sum of its
+// nsplit rows (in split order), x = sum / npts.  s1, s2 carry the sums of x
+// and x^2 between calls (first: none yet); the last call writes the mean and
+// the standard error (k_final_stats) to their reference positions.  blk (may
+// be null, nb = 1): the block's x.
+__global__ void k_block_rows(int64_t ntri, double f, const double *__restrict__ rows, int nb,
+                             int nsplit, bool first, bool last, int nbl, double *s1, double *s2,
+                             double *blk, double *mean, double *err, const int *pi, const int *pk,
+                             const int64_t *kbase, int n)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= ntri) return;
+    double a1 = first ? 0.0 : s1[t], a2 = first ? 0.0 : s2[t];
+    for (int b = 0; b < nb; b++) {
+        const double *r = rows + (size_t)b * nsplit * ntri + t;
+        double e = r[0];
+        for (int s = 1; s < nsplit; s++) e += r[(size_t)s * ntri];
+        const double x = e * f;
+        a1 += x;
+        a2 += x * x;
+        if (blk) blk[t] = x;
+    }
+    if (!last) {
+        s1[t] = a1;
+        s2[t] = a2;
+        return;
+    }
+    int64_t P, Q;
+    tri_decode(t, P, Q);
+    const int64_t at = zv_kcp(kbase, n, pi[P], pi[Q], pk[P], pk[Q]);
+    const double m1 = a1 / nbl, m2 = a2 / nbl;
+    mean[at] = m1;
+    err[at] = sqrt(fabs(m2 - m1 * m1)) / sqrt((double)nbl);
 }
 
 inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -1013,23 +1048,37 @@ static int pick_chunk(zv_context *c, int64_t npts, int precision)
     return (int)mc;
 }
 
+// Monte Carlo blocks run together: as many as fit in a chunk of samples and
+// in 2 GiB of accumulator rows (one per block and split), in rounds of equal
+// size.  Each round is one draw, one density launch, one set of nine
+// estimator launches and one statistics launch, so small molecules pay their
+// launches once instead of per block (10 AOs, 10 x 1000 samples FP32: 2.34 ms
+// block by block) and large ones their last, partly empty wave of tiles.
+static int pick_blocks(zv_context *c, int nbl, int64_t npts, int64_t chunk)
+{
+    const int64_t rows = std::max<int64_t>(1, ((int64_t)1 << 28) / std::max<int64_t>(1, c->nint));
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(chunk / npts, rows));
+    const int64_t rounds = (nbl + most - 1) / most;
+    return (int)((nbl + rounds - 1) / rounds);
+}
+
 // Sample splits of the group estimator: a molecule with few tiles would
-// leave most CUs idle while each tile walks the whole chunk, so the chunk's
+// leave most CUs idle while each tile walks a whole block, so the block's
 // stages are split over up to 64 workgroups per tile, aiming at about 1024
 // workgroups in all (about one resident round: 4 per CU by LDS), with at
 // least 4 stages per split and at most 1 GiB of partial rows.
-static int pick_split(zv_context *c, int Mc, int precision, int64_t tiles)
+static int pick_split(zv_context *c, int mblock, int precision, int64_t tiles, int nb)
 {
     if (tiles <= 0) return 1;
     const bool single = precision == ZV_PREC_FP32 || precision == ZV_PREC_BF16;
     const int sub = single ? GroupSub<float>::SUB : GroupSub<double>::SUB;
-    int64_t n = (1024 + tiles - 1) / tiles;
+    int64_t n = (1024 + tiles * nb - 1) / (tiles * nb);
     // a caller's choice (zv_set_tuning) replaces the count, within the
     // same bounds of stages and partial-row memory
     if (c->tune[ZV_TUNE_EST_SPLIT] > 0) n = c->tune[ZV_TUNE_EST_SPLIT];
     n = std::min<int64_t>(n, 64);
-    n = std::min<int64_t>(n, std::max<int64_t>(1, Mc / sub / 4));
-    n = std::min<int64_t>(n, 1 + ((int64_t)1 << 27) / std::max<int64_t>(1, c->nint));
+    n = std::min<int64_t>(n, std::max<int64_t>(1, mblock / sub / 4));
+    n = std::min<int64_t>(n, 1 + ((int64_t)1 << 27) / std::max<int64_t>(1, nb * c->nint));
     return (int)std::max<int64_t>(n, 1);
 }
 
@@ -1128,36 +1177,43 @@ static int group_ready(zv_context *c)
     return ZV_OK;
 }
 
+// samples of one launch set: nb blocks of mround samples (bstride apart in the
+// chunk of Mc), each in nsplit splits of mspan
+struct GroupSpan {
+    int nb, mround, nsplit, mspan, bstride, Mc;
+    bool add; // add to the rows instead of storing them
+};
+
 template <typename T, bool BF, int NR, int NC, int TR, int TC>
 static void launch_group_t(zv_context *c, hipStream_t st, unsigned ntile, const T *comp,
                            const T *grp, const int *urp, const int *urs, int nur, const int *ucp,
                            const int *ucs, int nuc, const int2 *tiles, const int *pos_pair,
-                           int Mround, int nsplit, int mspan, int Mc, double *acc,
-                           double *mpart)
+                           const GroupSpan &g, double *rows)
 {
-    if (nsplit > 1)
-        hipLaunchKernelGGL((k_est_group<T, NR, NC, TR, TC, true, BF>), dim3(ntile, (unsigned)nsplit),
-                           dim3(256), 0, st, comp, grp, urp, urs, nur, ucp, ucs, nuc, tiles,
-                           pos_pair, Mround, mspan, Mc, c->npair, c->grp_nsp_pad, acc, mpart,
-                           c->nint);
+    const dim3 grid(ntile, (unsigned)(g.nb * g.nsplit));
+    if (g.nsplit > 1)
+        hipLaunchKernelGGL((k_est_group<T, NR, NC, TR, TC, true, BF>), grid, dim3(256), 0, st,
+                           comp, grp, urp, urs, nur, ucp, ucs, nuc, tiles, pos_pair, g.mround,
+                           g.nsplit, g.mspan, g.bstride, g.Mc, c->npair, c->grp_nsp_pad, rows,
+                           g.add, c->nint);
     else
-        hipLaunchKernelGGL((k_est_group<T, NR, NC, TR, TC, false, BF>), dim3(ntile), dim3(256), 0, st,
-                           comp, grp, urp, urs, nur, ucp, ucs, nuc, tiles, pos_pair, Mround,
-                           mspan, Mc, c->npair, c->grp_nsp_pad, acc, mpart, c->nint);
+        hipLaunchKernelGGL((k_est_group<T, NR, NC, TR, TC, false, BF>), grid, dim3(256), 0, st,
+                           comp, grp, urp, urs, nur, ucp, ucs, nuc, tiles, pos_pair, g.mround,
+                           g.nsplit, g.mspan, g.bstride, g.Mc, c->npair, c->grp_nsp_pad, rows,
+                           g.add, c->nint);
 }
 
 // One launch per pair of unit classes; each is too small to fill the device
 // alone, so they run side by side on the main and the side streams (they
-// write disjoint quartets) and are joined back into the main stream.  With
-// nsplit > 1 every tile is also split over the samples of the chunk.
+// write disjoint quartets) and are joined back into the main stream.  The
+// grid's rows are the blocks of the chunk and their sample splits.
 template <typename T, bool BF>
-static int run_group_estimator(zv_context *c, const T *comp, const T *grp, int Mround, int Mc,
-                               int nsplit, double *acc, double *mpart)
+static int run_group_estimator(zv_context *c, const T *comp, const T *grp, GroupSpan span,
+                               double *rows)
 {
     constexpr int SUB = GroupSub<T>::SUB;
-    const int nstage = Mround / SUB;
-    const int per = (nstage + nsplit - 1) / nsplit;
-    const int mspan = per * SUB;
+    const int nstage = span.mround / SUB;
+    span.mspan = (nstage + span.nsplit - 1) / span.nsplit * SUB;
     const int *g = (const int *)c->b_gmeta.p;
     const int *pos_pair = g;
     hipStream_t sts[1 + zv_context::NSIDE] = {c->stream};
@@ -1182,7 +1238,7 @@ static int run_group_estimator(zv_context *c, const T *comp, const T *grp, int M
             const int2 *tiles = (const int2 *)g + c->grp_tile_off[3 * a + b];
 #define ZV_GROUP(NR, NC, TR, TC)                                                                  \
     launch_group_t<T, BF, NR, NC, TR, TC>(c, st, nt, comp, grp, urp, urs, nur, ucp, ucs, nuc, tiles, \
-                                      pos_pair, Mround, nsplit, mspan, Mc, acc, mpart)
+                                      pos_pair, span, rows)
             switch (9 * c->grp_tileset + 3 * a + b) {
             case 0: ZV_GROUP(1, 1, 4, 4); break;
             case 1: ZV_GROUP(1, 3, 4, 2); break;
@@ -1214,122 +1270,81 @@ static int run_group_estimator(zv_context *c, const T *comp, const T *grp, int M
     return ZV_OK;
 }
 
-// nbl blocks of npts samples over every quartet; the mean is left in accS
-// and the standard error in b_out2, both in triangle order.
-static int run_mc_core(zv_context *c, int nbl, int64_t npts, int mode, uint64_t seed,
-                       uint64_t stream, int precision, const double *r1, const double *r2,
-                       const double *pi0, double *block_means)
+// samples of blocks [b, b + nb) at offset m0 of each (nb > 1: m0 = 0) into
+// the chunk's sample buffers
+static int fill_samples(zv_context *c, int mode, uint64_t seed, uint64_t stream, uint64_t g0, int M,
+                        const double *r1, const double *r2, const double *pi0)
+{
+    double *d_r1 = (double *)c->b_r1.p, *d_r2 = (double *)c->b_r2.p, *d_pi0 = (double *)c->b_pi0.p;
+    if (mode == ZV_SAMPLES_FIXED) {
+        PhaseTimer tm(c, PH_COPY);
+        ZV_HIPCHECK(c, hipMemcpyAsync(d_r1, r1 + 3 * g0, sizeof(double) * 3 * M,
+                                      hipMemcpyHostToDevice, c->stream));
+        ZV_HIPCHECK(c, hipMemcpyAsync(d_r2, r2 + 3 * g0, sizeof(double) * 3 * M,
+                                      hipMemcpyHostToDevice, c->stream));
+        ZV_HIPCHECK(c, hipMemcpyAsync(d_pi0, pi0 + g0, sizeof(double) * M, hipMemcpyHostToDevice,
+                                      c->stream));
+    } else {
+        PhaseTimer tm(c, PH_SAMPLE);
+        hipLaunchKernelGGL(k_draw, dim3(nblk(M, 256)), dim3(256), 0, c->stream, seed, stream, g0, M,
+                           M, d_r1, d_r2, d_pi0);
+        ZV_HIPCHECK(c, hipGetLastError());
+    }
+    return ZV_OK;
+}
+
+static void block_line(zv_context *c, int b, int nbl, int64_t npts)
+{
+    printf(" MC block %d / %d done (%lld samples, %lld quartets)\n", b + 1, nbl, (long long)npts,
+           (long long)c->nint);
+    fflush(stdout);
+}
+
+// The parity estimator, block by block: the mean is left in accS and the
+// standard error in b_out2, both in triangle order.
+static int run_mc_parity(zv_context *c, int nbl, int64_t npts, int mode, uint64_t seed,
+                         uint64_t stream, const double *r1, const double *r2, const double *pi0,
+                         double *block_means)
 {
     const int64_t ntri = c->nint;
     const int np = c->npair, npp = c->npair_pad;
-    const int Mc = pick_chunk(c, npts, precision);
-    const bool single = precision == ZV_PREC_FP32 || precision == ZV_PREC_BF16;
-    size_t fbytes = single ? 4 : 8;
-    if (precision != ZV_PREC_FP64_PARITY) ZV_CHECK(group_ready(c));
-    const size_t ncomp = (size_t)4 * Mc * np, ngrp = (size_t)6 * Mc * c->nsp;
+    const int Mc = pick_chunk(c, npts, ZV_PREC_FP64_PARITY);
     ZV_CHECK(zv_ensure(c, c->b_r1, sizeof(double) * 3 * Mc));
     ZV_CHECK(zv_ensure(c, c->b_r2, sizeof(double) * 3 * Mc));
     ZV_CHECK(zv_ensure(c, c->b_pi0, sizeof(double) * Mc));
-    ZV_CHECK(zv_ensure(c, c->b_pd, precision == ZV_PREC_FP64_PARITY
-                                       ? fbytes * kParityFields * (size_t)Mc * npp
-                                       : fbytes * (ncomp + ngrp)));
-    ZV_CHECK(zv_ensure(c, c->b_accS, sizeof(double) * ntri));
-    if (precision == ZV_PREC_FP64_PARITY) ZV_CHECK(zv_ensure(c, c->b_accG, sizeof(double) * ntri));
-    ZV_CHECK(zv_ensure(c, c->b_s1, sizeof(double) * ntri));
-    ZV_CHECK(zv_ensure(c, c->b_s2, sizeof(double) * ntri));
+    ZV_CHECK(zv_ensure(c, c->b_pd, sizeof(double) * kParityFields * (size_t)Mc * npp));
+    for (DevBuf *b : {&c->b_accS, &c->b_accG, &c->b_s1, &c->b_s2, &c->b_out2})
+        ZV_CHECK(zv_ensure(c, *b, sizeof(double) * ntri));
     if (block_means) ZV_CHECK(zv_ensure(c, c->b_blk, sizeof(double) * ntri));
-    int64_t ntiles = 0;
-    for (int k = 0; k < 9; k++) ntiles += c->grp_ntile[k];
-    const int nsplit = precision == ZV_PREC_FP64_PARITY ? 1 : pick_split(c, Mc, precision, ntiles);
-    if (nsplit > 1) ZV_CHECK(zv_ensure(c, c->b_mpart, sizeof(double) * (nsplit - 1) * ntri));
-    double *mpart = nsplit > 1 ? (double *)c->b_mpart.p : nullptr;
-    double *accS = (double *)c->b_accS.p;
-    double *accG = precision == ZV_PREC_FP64_PARITY ? (double *)c->b_accG.p : nullptr;
+    double *accS = (double *)c->b_accS.p, *accG = (double *)c->b_accG.p;
     double *s1 = (double *)c->b_s1.p, *s2 = (double *)c->b_s2.p;
     {
         PhaseTimer tm(c, PH_STATS);
-        ZV_CHECK(zv_fill_dev(c, accS, ntri, 0.0));
-        if (accG) ZV_CHECK(zv_fill_dev(c, accG, ntri, 0.0));
-        ZV_CHECK(zv_fill_dev(c, s1, ntri, 0.0));
-        ZV_CHECK(zv_fill_dev(c, s2, ntri, 0.0));
-        if (mpart) ZV_CHECK(zv_fill_dev(c, mpart, (int64_t)(nsplit - 1) * ntri, 0.0));
+        for (double *p : {accS, accG, s1, s2}) ZV_CHECK(zv_fill_dev(c, p, ntri, 0.0));
     }
-    Basis B = dev_basis(c);
-    PairTab PT = dev_pairs(c);
-    double *d_r1 = (double *)c->b_r1.p, *d_r2 = (double *)c->b_r2.p, *d_pi0 = (double *)c->b_pi0.p;
     for (int b = 0; b < nbl; b++) {
         for (int64_t m0 = 0; m0 < npts; m0 += Mc) {
-            int Mv = (int)((npts - m0) < Mc ? (npts - m0) : Mc);
-            uint64_t g0 = (uint64_t)b * (uint64_t)npts + (uint64_t)m0;
-            int sub = single ? GroupSub<float>::SUB : GroupSub<double>::SUB;
-            int Mround = (Mv + sub - 1) / sub * sub;
-            if (mode == ZV_SAMPLES_FIXED) {
-                PhaseTimer tm(c, PH_COPY);
-                ZV_HIPCHECK(c, hipMemcpyAsync(d_r1, r1 + 3 * g0, sizeof(double) * 3 * Mv,
-                                              hipMemcpyHostToDevice, c->stream));
-                ZV_HIPCHECK(c, hipMemcpyAsync(d_r2, r2 + 3 * g0, sizeof(double) * 3 * Mv,
-                                              hipMemcpyHostToDevice, c->stream));
-                ZV_HIPCHECK(c, hipMemcpyAsync(d_pi0, pi0 + g0, sizeof(double) * Mv,
-                                              hipMemcpyHostToDevice, c->stream));
-            } else {
-                PhaseTimer tm(c, PH_SAMPLE);
-                hipLaunchKernelGGL(k_draw, dim3(nblk(Mv, 256)), dim3(256), 0, c->stream, seed,
-                                   stream, g0, Mv, Mv, d_r1, d_r2, d_pi0);
+            const int Mv = (int)std::min<int64_t>(npts - m0, Mc);
+            ZV_CHECK(fill_samples(c, mode, seed, stream, (uint64_t)b * npts + m0, Mv, r1, r2, pi0));
+            {
+                PhaseTimer tm(c, PH_DENS);
+                hipLaunchKernelGGL(k_dens_parity, dim3(nblk((int64_t)Mv * npp, 256)), dim3(256), 0,
+                                   c->stream, dev_basis(c), dev_pairs(c), np, npp, Mv, Mc,
+                                   (const double *)c->b_r1.p, (const double *)c->b_r2.p,
+                                   (double *)c->b_pd.p);
                 ZV_HIPCHECK(c, hipGetLastError());
             }
-            if (precision == ZV_PREC_FP64_PARITY) {
-                {
-                    PhaseTimer tm(c, PH_DENS);
-                    hipLaunchKernelGGL(k_dens_parity, dim3(nblk((int64_t)Mv * npp, 256)),
-                                       dim3(256), 0, c->stream, B, PT, np, npp, Mv, Mc, d_r1,
-                                       d_r2, (double *)c->b_pd.p);
-                    ZV_HIPCHECK(c, hipGetLastError());
-                }
-                PhaseTimer tm(c, PH_EST);
-                hipLaunchKernelGGL(k_est_parity, dim3(nblk(ntri, 256)), dim3(256), 0, c->stream,
-                                   (const double *)c->b_pd.p, d_pi0, Mv, Mc, npp, ntri, accS,
-                                   accG);
-                ZV_HIPCHECK(c, hipGetLastError());
-            } else {
-                const int *g = (const int *)c->b_gmeta.p;
-                const int *pos_pair = g, *sp_first = g + c->grp_possp_off + np;
-                const dim3 grid(nblk(Mc, 256) * (unsigned)c->nsp);
-                if (single) {
-                    float *comp = (float *)c->b_pd.p, *grp = comp + ncomp;
-                    {
-                        PhaseTimer tm(c, PH_DENS);
-                        hipLaunchKernelGGL(k_dens_group<float>, grid, dim3(256), 0, c->stream, B,
-                                           PT, npp, pos_pair, sp_first, np, c->nsp, Mv, Mc, d_r1,
-                                           d_r2, d_pi0, comp, grp, (const int *)nullptr);
-                        ZV_HIPCHECK(c, hipGetLastError());
-                    }
-                    PhaseTimer tm(c, PH_EST);
-                    if (precision == ZV_PREC_BF16)
-                        ZV_CHECK((run_group_estimator<float, true>(c, comp, grp, Mround, Mc,
-                                                                   nsplit, accS, mpart)));
-                    else
-                        ZV_CHECK((run_group_estimator<float, false>(c, comp, grp, Mround, Mc,
-                                                                    nsplit, accS, mpart)));
-                } else {
-                    double *comp = (double *)c->b_pd.p, *grp = comp + ncomp;
-                    {
-                        PhaseTimer tm(c, PH_DENS);
-                        hipLaunchKernelGGL(k_dens_group<double>, grid, dim3(256), 0, c->stream, B,
-                                           PT, npp, pos_pair, sp_first, np, c->nsp, Mv, Mc, d_r1,
-                                           d_r2, d_pi0, comp, grp, (const int *)nullptr);
-                        ZV_HIPCHECK(c, hipGetLastError());
-                    }
-                    PhaseTimer tm(c, PH_EST);
-                    ZV_CHECK((run_group_estimator<double, false>(c, comp, grp, Mround, Mc,
-                                                                 nsplit, accS, mpart)));
-                }
-            }
+            PhaseTimer tm(c, PH_EST);
+            hipLaunchKernelGGL(k_est_parity, dim3(nblk(ntri, 256)), dim3(256), 0, c->stream,
+                               (const double *)c->b_pd.p, (const double *)c->b_pi0.p, Mv, Mc, npp,
+                               ntri, accS, accG);
+            ZV_HIPCHECK(c, hipGetLastError());
         }
         {
             PhaseTimer tm(c, PH_STATS);
             hipLaunchKernelGGL(k_block_end, dim3(nblk(ntri, 256)), dim3(256), 0, c->stream, ntri,
                                1.0 / (double)npts, accS, accG, s1, s2,
-                               block_means ? (double *)c->b_blk.p : nullptr, nsplit - 1, mpart);
+                               block_means ? (double *)c->b_blk.p : nullptr);
             ZV_HIPCHECK(c, hipGetLastError());
         }
         if (block_means)
@@ -1337,18 +1352,106 @@ static int run_mc_core(zv_context *c, int nbl, int64_t npts, int mode, uint64_t 
                                         block_means + (size_t)b * ntri));
         if (c->verbose >= 2) {
             ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
-            printf(" MC block %d / %d done (%lld samples, %lld quartets)\n", b + 1, nbl,
-                   (long long)npts, (long long)ntri);
-            fflush(stdout);
+            block_line(c, b, nbl, npts);
         }
     }
-    ZV_CHECK(zv_ensure(c, c->b_out2, sizeof(double) * ntri));
+    PhaseTimer tm(c, PH_STATS);
+    // mean -> accS, err -> out2 (triangle order), then scatter
+    hipLaunchKernelGGL(k_final_stats, dim3(nblk(ntri, 256)), dim3(256), 0, c->stream, ntri, nbl, s1,
+                       s2, accS, (double *)c->b_out2.p);
+    ZV_HIPCHECK(c, hipGetLastError());
+    return ZV_OK;
+}
+
+// densities of the chunk's Mv samples and the estimator's launches for them
+template <typename T, bool BF>
+static int run_group_chunk(zv_context *c, int Mv, const GroupSpan &span, double *rows)
+{
+    const int np = c->npair;
+    T *comp = (T *)c->b_pd.p, *grp = comp + (size_t)4 * span.Mc * np;
+    const int *pos_pair = (const int *)c->b_gmeta.p;
     {
-        PhaseTimer tm(c, PH_STATS);
-        // mean -> accS, err -> out2 (triangle order), then scatter
-        hipLaunchKernelGGL(k_final_stats, dim3(nblk(ntri, 256)), dim3(256), 0, c->stream, ntri,
-                           nbl, s1, s2, accS, (double *)c->b_out2.p);
+        PhaseTimer tm(c, PH_DENS);
+        hipLaunchKernelGGL(k_dens_group<T>, dim3(nblk(span.Mc, 256) * (unsigned)c->nsp), dim3(256),
+                           0, c->stream, dev_basis(c), dev_pairs(c), c->npair_pad, pos_pair,
+                           pos_pair + c->grp_possp_off + np, np, c->nsp, Mv, span.Mc,
+                           (const double *)c->b_r1.p, (const double *)c->b_r2.p,
+                           (const double *)c->b_pi0.p, comp, grp, (const int *)nullptr);
         ZV_HIPCHECK(c, hipGetLastError());
+    }
+    PhaseTimer tm(c, PH_EST);
+    return run_group_estimator<T, BF>(c, comp, grp, span, rows);
+}
+
+// The group estimator: the mean and the standard error go to the result
+// buffers in reference order.  Rounds of nb blocks when a block fits in a
+// chunk; otherwise block by block, the chunks of a block added up in its
+// rows.  Block means and the per-block progress lines take one block a round.
+static int run_mc_group(zv_context *c, int nbl, int64_t npts, int mode, uint64_t seed,
+                        uint64_t stream, int precision, const double *r1, const double *r2,
+                        const double *pi0, double *block_means)
+{
+    const int64_t ntri = c->nint;
+    ZV_CHECK(group_ready(c));
+    const bool single = precision != ZV_PREC_FP64;
+    const int cap = pick_chunk(c, (int64_t)nbl * npts, precision);
+    int nb = cap >= npts ? pick_blocks(c, nbl, npts, cap) : 1;
+    if (block_means || c->verbose >= 2) nb = 1;
+    const int Mc = cap >= npts ? (int)(nb * npts) : cap;
+    const size_t fields = (size_t)Mc * (4 * (size_t)c->npair + 6 * (size_t)c->nsp);
+    ZV_CHECK(zv_ensure(c, c->b_r1, sizeof(double) * 3 * Mc));
+    ZV_CHECK(zv_ensure(c, c->b_r2, sizeof(double) * 3 * Mc));
+    ZV_CHECK(zv_ensure(c, c->b_pi0, sizeof(double) * Mc));
+    ZV_CHECK(zv_ensure(c, c->b_pd, (single ? 4 : 8) * fields));
+    int64_t ntiles = 0;
+    for (int k = 0; k < 9; k++) ntiles += c->grp_ntile[k];
+    const int mblock = (int)std::min<int64_t>(npts, Mc);
+    const int nsplit = pick_split(c, mblock, precision, ntiles, nb);
+    ZV_CHECK(zv_ensure(c, c->b_mpart, sizeof(double) * nb * nsplit * ntri));
+    double *rows = (double *)c->b_mpart.p;
+    if (nb < nbl) {
+        ZV_CHECK(zv_ensure(c, c->b_s1, sizeof(double) * ntri));
+        ZV_CHECK(zv_ensure(c, c->b_s2, sizeof(double) * ntri));
+    }
+    if (block_means) ZV_CHECK(zv_ensure(c, c->b_blk, sizeof(double) * ntri));
+    for (int which : {ZV_RESULT_MEAN, ZV_RESULT_STDERR}) {
+        c->res_valid[which] = false;
+        ZV_CHECK(zv_ensure(c, c->b_res[which], sizeof(double) * ntri));
+    }
+    const int sub = single ? GroupSub<float>::SUB : GroupSub<double>::SUB;
+    for (int b = 0; b < nbl; b += nb) {
+        const int bn = std::min(nb, nbl - b);
+        // a block longer than the chunk (nb = 1) takes several chunks
+        for (int64_t m0 = 0; m0 < npts; m0 += nb > 1 ? npts : Mc) {
+            const int mb = (int)std::min<int64_t>(npts - m0, nb > 1 ? npts : Mc);
+            const int Mv = nb > 1 ? bn * mb : mb;
+            ZV_CHECK(fill_samples(c, mode, seed, stream, (uint64_t)b * npts + m0, Mv, r1, r2, pi0));
+            const GroupSpan span{bn, (mb + sub - 1) / sub * sub, nsplit, 0, mb, Mc, m0 > 0};
+            if (precision == ZV_PREC_FP64)
+                ZV_CHECK((run_group_chunk<double, false>(c, Mv, span, rows)));
+            else if (precision == ZV_PREC_BF16)
+                ZV_CHECK((run_group_chunk<float, true>(c, Mv, span, rows)));
+            else
+                ZV_CHECK((run_group_chunk<float, false>(c, Mv, span, rows)));
+        }
+        {
+            PhaseTimer tm(c, PH_STATS);
+            hipLaunchKernelGGL(k_block_rows, dim3(nblk(ntri, 256)), dim3(256), 0, c->stream, ntri,
+                               1.0 / (double)npts, (const double *)rows, bn, nsplit, b == 0,
+                               b + bn == nbl, nbl, (double *)c->b_s1.p, (double *)c->b_s2.p,
+                               block_means ? (double *)c->b_blk.p : nullptr,
+                               (double *)c->b_res[ZV_RESULT_MEAN].p,
+                               (double *)c->b_res[ZV_RESULT_STDERR].p, c->d_pair_i, c->d_pair_k,
+                               c->d_kbase, c->n);
+            ZV_HIPCHECK(c, hipGetLastError());
+        }
+        if (block_means)
+            ZV_CHECK(zv_run_scatter_ref(c, (const double *)c->b_blk.p,
+                                        block_means + (size_t)b * ntri));
+        if (c->verbose >= 2) {
+            ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
+            block_line(c, b, nbl, npts);
+        }
     }
     return ZV_OK;
 }
@@ -1357,9 +1460,21 @@ int zv_run_mc(zv_context *c, int nbl, int64_t npts, int mode, uint64_t seed, uin
               int precision, const double *r1, const double *r2, const double *pi0, double *mean,
               double *err, double *block_means)
 {
-    ZV_CHECK(run_mc_core(c, nbl, npts, mode, seed, stream, precision, r1, r2, pi0, block_means));
-    ZV_CHECK(zv_keep_result(c, (const double *)c->b_accS.p, ZV_RESULT_MEAN, mean));
-    ZV_CHECK(zv_keep_result(c, (const double *)c->b_out2.p, ZV_RESULT_STDERR, err));
+    if (precision == ZV_PREC_FP64_PARITY) {
+        ZV_CHECK(run_mc_parity(c, nbl, npts, mode, seed, stream, r1, r2, pi0, block_means));
+        ZV_CHECK(zv_keep_result(c, (const double *)c->b_accS.p, ZV_RESULT_MEAN, mean));
+        return zv_keep_result(c, (const double *)c->b_out2.p, ZV_RESULT_STDERR, err);
+    }
+    ZV_CHECK(run_mc_group(c, nbl, npts, mode, seed, stream, precision, r1, r2, pi0, block_means));
+    for (int which : {ZV_RESULT_MEAN, ZV_RESULT_STDERR}) {
+        double *host = which == ZV_RESULT_MEAN ? mean : err;
+        if (!host) continue;
+        PhaseTimer tm(c, PH_COPY);
+        ZV_HIPCHECK(c, hipMemcpyAsync(host, c->b_res[which].p, sizeof(double) * c->nint,
+                                      hipMemcpyDeviceToHost, c->stream));
+    }
+    ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
+    c->res_valid[ZV_RESULT_MEAN] = c->res_valid[ZV_RESULT_STDERR] = true;
     return ZV_OK;
 }
 

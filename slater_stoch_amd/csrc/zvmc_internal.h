@@ -81,7 +81,7 @@ struct zv_context {
     // ZV_RESULT_MEAN, ZV_RESULT_STDERR of the last zv_gauss_eri / zv_mc_blocks
     DevBuf b_res[3];
     bool res_valid[3] = {false, false, false};
-    DevBuf b_mpart;                    // estimator partial sums of sample splits 1..n-1
+    DevBuf b_mpart;                    // estimator sums per (block, sample split) of a round
     DevBuf b_pp;                       // primitive-pair data
     DevBuf b_btab;                     // Boys Taylor table (zv_boys_table)
     bool btab_ready = false;
