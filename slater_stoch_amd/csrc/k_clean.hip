@@ -503,9 +503,7 @@ int zv_run_svd_clean(zv_context *c, int rank, int q, uint64_t seed, double *eri,
     hipLaunchKernelGGL(k_gather, dim3(nblk(c->nint, 256)), dim3(256), 0, c->stream, c->nint,
                        (const double *)W, d_eri, c->n, c->d_pair_i, c->d_pair_k, c->d_kbase, 1);
     ZV_HIPCHECK(c, hipGetLastError());
-    ZV_HIPCHECK(c, hipMemcpyAsync(eri, d_eri, sizeof(double) * c->nint, hipMemcpyDeviceToHost,
-                                  c->stream));
-    ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
+    ZV_CHECK(zv_copy_out(c, eri, d_eri, sizeof(double) * c->nint));
     if (n_removed) *n_removed = removed;
     return ZV_OK;
 }
@@ -555,9 +553,7 @@ int zv_run_davidson_clean(zv_context *c, double *eri, int *n_removed)
     hipLaunchKernelGGL(k_gather, dim3(nblk(c->nint, 256)), dim3(256), 0, c->stream, c->nint,
                        (const double *)W, d_eri, c->n, c->d_pair_i, c->d_pair_k, c->d_kbase, 0);
     ZV_HIPCHECK(c, hipGetLastError());
-    ZV_HIPCHECK(c, hipMemcpyAsync(eri, d_eri, sizeof(double) * c->nint, hipMemcpyDeviceToHost,
-                                  c->stream));
-    ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
+    ZV_CHECK(zv_copy_out(c, eri, d_eri, sizeof(double) * c->nint));
     if (n_removed) *n_removed = l;
     return ZV_OK;
 }
@@ -708,10 +704,7 @@ static int gather_V(zv_context *c, const double *V, double *d_eri, double *eri_h
     hipLaunchKernelGGL(k_gather_V, dim3(nblk(c->nint, 256)), dim3(256), 0, c->stream, c->nint, V,
                        d_eri, N, c->n, c->d_pair_i, c->d_pair_k, c->d_kbase);
     ZV_HIPCHECK(c, hipGetLastError());
-    ZV_HIPCHECK(c, hipMemcpyAsync(eri_host, d_eri, sizeof(double) * c->nint,
-                                  hipMemcpyDeviceToHost, c->stream));
-    ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return ZV_OK;
+    return zv_copy_out(c, eri_host, d_eri, sizeof(double) * c->nint);
 }
 
 // V -= X diag(lam) X^T for the first m columns of X (N x m) with lam[j] < 0

@@ -891,10 +891,8 @@ int zv_run_scatter_ref(zv_context *c, const double *d_tri, double *host_out)
                            d_tri, (double *)c->b_out.p, c->d_pair_i, c->d_pair_k, c->d_kbase,
                            c->n);
         ZV_HIPCHECK(c, hipGetLastError());
-        ZV_HIPCHECK(c, hipMemcpyAsync(host_out, c->b_out.p, sizeof(double) * ntri,
-                                      hipMemcpyDeviceToHost, c->stream));
+        ZV_CHECK(zv_copy_out(c, host_out, c->b_out.p, sizeof(double) * ntri));
     }
-    ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
     return ZV_OK;
 }
 
@@ -909,9 +907,7 @@ int zv_keep_result(zv_context *c, const double *d_tri, int which, double *host_o
         hipLaunchKernelGGL(k_scatter_ref, dim3(nblk(ntri, 256)), dim3(256), 0, c->stream, ntri,
                            d_tri, (double *)res.p, c->d_pair_i, c->d_pair_k, c->d_kbase, c->n);
         ZV_HIPCHECK(c, hipGetLastError());
-        if (host_out)
-            ZV_HIPCHECK(c, hipMemcpyAsync(host_out, res.p, sizeof(double) * ntri,
-                                          hipMemcpyDeviceToHost, c->stream));
+        if (host_out) ZV_CHECK(zv_copy_out(c, host_out, res.p, sizeof(double) * ntri));
     }
     ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
     c->res_valid[which] = true;
@@ -1470,8 +1466,7 @@ int zv_run_mc(zv_context *c, int nbl, int64_t npts, int mode, uint64_t seed, uin
         double *host = which == ZV_RESULT_MEAN ? mean : err;
         if (!host) continue;
         PhaseTimer tm(c, PH_COPY);
-        ZV_HIPCHECK(c, hipMemcpyAsync(host, c->b_res[which].p, sizeof(double) * c->nint,
-                                      hipMemcpyDeviceToHost, c->stream));
+        ZV_CHECK(zv_copy_out(c, host, c->b_res[which].p, sizeof(double) * c->nint));
     }
     ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
     c->res_valid[ZV_RESULT_MEAN] = c->res_valid[ZV_RESULT_STDERR] = true;

@@ -123,6 +123,7 @@ struct zv_context {
 
     // timings of the last call: events recorded around each launch group
     std::vector<hipEvent_t> ev_pool;
+    std::vector<hipEvent_t> ev_stage; // one per slab of the copy ring (zv_copy_out)
     size_t ev_used = 0;
     std::vector<int> pend_phase;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pend_ev;
@@ -149,6 +150,9 @@ int zv_run_gauss_list_noalloc(zv_context *c, int64_t nq, const int *qi, const in
 int zv_fail(zv_context *c, int code, const char *fmt, ...);
 int zv_hip(zv_context *c, hipError_t e, const char *what);
 int zv_ensure(zv_context *c, DevBuf &b, size_t bytes);
+
+// device -> host copy after the work on the context's stream; returns when done
+int zv_copy_out(zv_context *c, void *host, const void *dev, size_t bytes);
 
 // triangle index of (P, Q), P >= Q (0-based pair indices)
 __host__ __device__ inline int64_t zv_tri(int64_t P, int64_t Q) { return P * (P + 1) / 2 + Q; }
