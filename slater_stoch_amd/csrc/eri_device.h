@@ -98,44 +98,74 @@ template <int L> __device__ inline void boys(double T, double *F)
     }
 }
 
-// Tabulated Boys function (the shell kernels): for T < 36 a Taylor
-// expansion of F_L about the nearest grid point T_i = i / 2,
-//   F_L(T_i + d) = sum_k (-1)^k F_{L+k}(T_i) d^k / k!,  |d| <= 1/4, k <= 14
-// (remainder below 1e-21 of F_L), then the downward recursion
-//   F_m = (2 T F_{m+1} + exp(-T)) / (2m + 1),
-// which is stable; the table holds (-1)^k F_{L+k}(T_i) / k! for L <= 8,
-// computed on the host in extended precision from the series
-// F_m(T) = exp(-T) sum_j (2T)^j / ((2m+1)(2m+3)...(2m+2j+1)) (zv_boys_table).
-// From T = 36 on the branch of boys<L> (F_0 = sqrt(pi/T)/2, erf rounding to
-// 1, upward recursion).  Relative error below 1e-15 against the series in
-// extended precision; one code path for all T < 36, where boys<L> splits at
-// T = 1 and evaluates erf above it.  lt: the kernel's LDS copy of the
-// L-slice, [k][i].
+// Tabulated Boys function (shell kernels, one-electron kernels): for T < 36 a
+// Taylor expansion about the nearest grid point T_i = i / 2, |d| <= 1/4,
+//   F_L(T_i + d) = sum_k (-1)^k F_{L+k}(T_i) d^k / k!,
+// with the terms k <= 12 (remainder below 3e-18 of F_L); the table holds
+// (-1)^k F_{L+k}(T_i) / k! for L <= 8, k <= 14, computed on the host in
+// extended precision from the series F_m(T) = exp(-T) sum_j (2T)^j /
+// ((2m+1)(2m+3)...(2m+2j+1)) (zv_boys_table).  Orders below L follow by the
+// stable downward recursion F_m = (2 T F_{m+1} + exp(-T)) / (2m + 1) for
+// L >= 3.  For L <= 2 they are the derivatives of the F_0 expansion instead
+// (F_1 = -F_0', F_2 = F_0''; two and four terms more, Horner's scheme for all
+// of them at once): 12 + 13 multiply-adds for L = 1 where the exponential and
+// its constants take about 40 instructions.  From T = 36 on the branch of
+// boys<L> (F_0 = sqrt(pi/T)/2, erf rounding to 1, upward recursion), whose
+// exponential is skipped by a wave beyond T = 80.  Relative error below 1e-15
+// against the series in extended precision; one code path for all T < 36,
+// where boys<L> splits at T = 1 and evaluates erf above it.  lt: the kernel's
+// LDS copy of slice boys_slice(L), [k][i].
 constexpr int kBoysK = 14, kBoysN = 73; // orders 0..kBoysK, grid 0, 0.5, .., 36
 constexpr int kBoysLmax = 8;
 constexpr int kBoysSlice = (kBoysK + 1) * kBoysN;
+constexpr int boys_slice(int L) { return L <= 2 ? 0 : L; }
+
+// 1/sqrt(x) for a positive normal x: the hardware estimate (about 5e-8
+// relative) and one third-order step y' = y (1 + e/2 + 3 e^2/8), e = 1 - x y^2
+// (remainder 5 e^3 / 16 < 1e-21), an ulp or two; it replaces a correctly
+// rounded division and square root (1/s and sqrt(1/s)) in the prefactor.
+__device__ inline double rsqrt_pos(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
 
 template <int L> __device__ inline void boys_table(double T, const double *lt, double *F)
 {
     if (T < 36.0) {
         const int i = (int)(T * 2.0 + 0.5);
         const double d = T - 0.5 * (double)i;
-        double s = lt[kBoysK * kBoysN + i];
+        if constexpr (L <= 2) {
+            constexpr int K = 12 + L;
+            double b0 = lt[K * kBoysN + i], b1 = 0.0, b2 = 0.0;
 #pragma unroll
-        for (int k = kBoysK - 1; k >= 0; k--) s = fma(s, d, lt[k * kBoysN + i]);
-        F[L] = s;
-        if (L > 0) {
+            for (int k = K - 1; k >= 0; k--) {
+                if (L >= 2 && k <= K - 2) b2 = k == K - 2 ? b1 : fma(b2, d, b1);
+                if (L >= 1) b1 = k == K - 1 ? b0 : fma(b1, d, b0);
+                b0 = fma(b0, d, lt[k * kBoysN + i]);
+            }
+            F[0] = b0;
+            if constexpr (L >= 1) F[1] = -b1;
+            if constexpr (L >= 2) F[2] = 2.0 * b2;
+        } else {
+            constexpr int K = 12;
+            double s = lt[K * kBoysN + i];
+#pragma unroll
+            for (int k = K - 1; k >= 0; k--) s = fma(s, d, lt[k * kBoysN + i]);
+            F[L] = s;
             const double e = exp(-T);
 #pragma unroll
             for (int m = L - 1; m >= 0; m--)
                 F[m] = fma(2.0 * T, F[m + 1], e) * (1.0 / (2 * m + 1));
         }
     } else {
-        double u_inv = rsqrt(T);
+        const double u_inv = rsqrt_pos(T);
         F[0] = (0.5 * u_inv) * kSqrtPi;
         if (L > 0) {
-            double e = T > 80.0 ? 0.0 : exp(-T);
-            double tri = (0.5 * u_inv) * u_inv;
+            double e = 0.0;
+            if (T <= 80.0) e = exp(-T);
+            const double tri = (0.5 * u_inv) * u_inv;
 #pragma unroll
             for (int m = 0; m < L; m++) F[m + 1] = (F[m] * (2 * m + 1) - e) * tri;
         }
@@ -164,19 +194,6 @@ __device__ inline void boys_rt(int L, double T, double *F)
         double tri = (0.5 * u_inv) * u_inv;
         for (int m = 0; m < L; m++) F[m + 1] = (F[m] * (2 * m + 1) - e) * tri;
     }
-}
-
-// 1/sqrt(x) for a positive normal x (an exponent sum p + q in the shell
-// kernels): the hardware estimate (about 5e-8 relative) and two Newton
-// steps y' = y + y (1 - x y^2) / 2, a few ulp; it replaces a correctly
-// rounded division and square root (1/s and sqrt(1/s)) in the prefactor.
-__device__ inline double rsqrt_pos(double x)
-{
-    double y = __builtin_amdgcn_rsq(x);
-    double e = fma(-(x * y), y, 1.0);
-    y = fma(y * 0.5, e, y);
-    e = fma(-(x * y), y, 1.0);
-    return fma(y * 0.5, e, y);
 }
 
 // ------------------------------------------------------------------ R table

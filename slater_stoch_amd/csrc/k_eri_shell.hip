@@ -141,17 +141,16 @@ constexpr int kPassMax = 4;
 constexpr int npass(int LU, int LL)
 {
     if (LU == 4) return 4;
-    if (LU == 3) return 2;
+    if (LU == 3 && LL == 4) return 2;
     return 1;
 }
 constexpr Pass pass_of(int LU, int LL, int p)
 {
     const int ng = ngroup(LU);
     if (LU == 4)
-        return p == 0 ? Pass{0, 5, 0, 2} : p == 1 ? Pass{0, 5, 2, 4} : p == 2 ? Pass{6, 7, 0, 4}
+        return p == 0 ? Pass{0, 5, 0, 1} : p == 1 ? Pass{0, 5, 1, 4} : p == 2 ? Pass{6, 7, 0, 4}
                                                                            : Pass{8, 8, 0, 1};
-    if (LU == 3 && LL == 3) return p == 0 ? Pass{0, 6, 0, 1} : Pass{0, 4, 1, 3};
-    if (LU == 3) return p == 0 ? Pass{0, 5, 0, 3} : Pass{6, 7, 0, 1};
+    if (LU == 3 && LL == 4) return p == 0 ? Pass{0, 7, 0, 1} : Pass{0, 5, 1, 3};
     return Pass{0, LU + LL, 0, ng};
 }
 
@@ -195,6 +194,14 @@ template <int LU, int LL, int PASS> struct Cls {
     static constexpr Pass ps = pass_of(LU, LL, PASS);
     static constexpr Slots sl = make_slots(LU, LL, ps);
     static constexpr int zwords = (sl.ztot + 3) / 4 * 64; // Z tiles in LDS, 4 x 16 values a row
+    // accumulators of row r: [first(r), first(r) + count(r))
+    static constexpr int first(int r)
+    {
+        int i = 0;
+        while (i < sl.n && sl.r[i] < r) i++;
+        return i;
+    }
+    static constexpr int count(int r) { return first(r + 1) - first(r); }
 };
 
 // Position in a pass's Z area of (sigma, sigma', r), -1 if another pass has it
@@ -258,26 +265,44 @@ template <int L> struct RProg {
     static constexpr RProgram<L> p{};
 };
 
-template <int L>
-__device__ __forceinline__ void hermite_table(double alpha, double scale, double X, double Y,
-                                              double Z, const double *F, double *R)
+// use(r, R^0_r) is called for every row.  With FENCE it is called as the row is
+// made (no later step reads it), so the table in registers is that of the
+// levels above 0, the orders below L, and the compiler's scheduler is kept
+// inside a level, or eight rows of the last one: left alone it starts many
+// rows at once and needs 100-150 registers more.  Without, the rows are used
+// after the last step, when none of them has to be waited for.
+template <int L, bool FENCE, class U>
+__device__ __forceinline__ void hermite_rows(double alpha, double scale, double X, double Y,
+                                             double Z, const double *F, U &&use)
 {
+    double R[FENCE ? (L > 0 ? hcount(L - 1) : 1) : hcount(L)];
     const double m2a = -2.0 * alpha;
     double sd[L + 1];
     sd[0] = scale;
     static_for<L>([&](auto i) { sd[i + 1] = sd[i] * m2a; });
     static_for<RProgram<L>::N>([&](auto i) {
         constexpr RStep e = RProg<L>::p.s[i];
+        // the last hcount(L) steps are level n = 0
+        constexpr bool row = FENCE && i >= RProgram<L>::N - hcount(L);
+        double v;
         if constexpr (e.axis == 3) {
-            R[0] = sd[e.a] * F[e.a];
+            v = sd[e.a] * F[e.a];
         } else {
             const double x = e.axis == 0 ? X : e.axis == 1 ? Y : Z;
             if constexpr (e.b < 0)
-                R[e.dst] = x * R[e.a];
+                v = x * R[e.a];
             else
-                R[e.dst] = fma((double)e.coef, R[e.b], x * R[e.a]);
+                v = fma((double)e.coef, R[e.b], x * R[e.a]);
         }
+        if constexpr (row)
+            use(std::integral_constant<int, e.dst>{}, v);
+        else
+            R[e.dst] = v;
+        if constexpr (FENCE && (e.axis == 3 || (row && i % 8 == 0)))
+            __builtin_amdgcn_sched_barrier(0);
     });
+    if constexpr (!FENCE)
+        static_for<hcount(L)>([&](auto r) { use(r, R[r]); });
 }
 
 struct SPD {
@@ -476,15 +501,40 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_wave_barrier();
 }
 
-constexpr int kTRows = 9;   // uniform components transformed at a time
+// uniform components transformed at a time: those of the largest shell pair
+// (p x s, p x p, p x d) or as many as nine
+constexpr int transform_rows(int LU) { return LU == 0 ? 1 : LU == 1 ? 3 : 9; }
 
-// waves per workgroup and per SIMD of a class's pass
+// Estimated registers (accumulators, R table, the rest) and LDS doubles of one
+// wave of a class's pass
+constexpr int quartet_regs(int LU, int LL, int p, bool fence)
+{
+    const Pass ps = pass_of(LU, LL, p);
+    return 2 * (make_slots(LU, LL, ps).n + hco(fence ? ps.rho1 - 1 : ps.rho1)) + 60;
+}
+constexpr int quartet_lds(int LU, int LL, int p)
+{
+    return (make_slots(LU, LL, pass_of(LU, LL, p)).ztot + 3) / 4 * 64 + 1 +
+           transform_rows(LU) * kG.t[LL].n;
+}
+// Waves per SIMD a pass is compiled for: two, in workgroups of four waves that
+// share the Boys table, where registers and LDS (two workgroups per CU) allow
+// it; otherwise one, each wave a workgroup of its own, whose transform reuses
+// the table's LDS (four per CU need 40 KB each).
 constexpr int quartet_waves(int LU, int LL, int p)
 {
-    const Slots s = make_slots(LU, LL, pass_of(LU, LL, p));
-    return 2 * (s.n + hcount(pass_of(LU, LL, p).rho1)) + 64 <= 256 ? 2 : 1;
+    return quartet_regs(LU, LL, p, true) <= 250 &&
+                   (4 * quartet_lds(LU, LL, p) + kBoysSlice) * 8 <= 81920
+               ? 2
+               : 1;
 }
 constexpr int quartet_wpb(int LU, int LL, int p) { return quartet_waves(LU, LL, p) >= 2 ? 4 : 1; }
+// instances that would leave their register budget (256 or 512) without:
+// fences cost the others 3-7 % ((2, 2) and (2, 3) on the 128-AO hydrocarbon)
+constexpr bool quartet_fence(int LU, int LL, int p)
+{
+    return quartet_regs(LU, LL, p, false) > (quartet_waves(LU, LL, p) >= 2 ? 230 : 400);
+}
 
 template <int LU, int LL, int PASS>
 __global__ __launch_bounds__(64 * quartet_wpb(LU, LL, PASS))
@@ -496,14 +546,16 @@ k_eri_quartet(SPD sd, const ShellItem *__restrict__ items, int nitems,
 {
     using C = Cls<LU, LL, PASS>;
     constexpr int WPB = quartet_wpb(LU, LL, PASS);
-    constexpr int L = C::ps.rho1, HR = hcount(L), NS = C::sl.n, NZ = C::sl.ztot;
+    constexpr int L = C::ps.rho1, NS = C::sl.n, NZ = C::sl.ztot;
     constexpr int RU = kRow[LU], RLn = kRow[LL], GU = ngroup(LU), GL = ngroup(LL);
-    constexpr int NGU = kG.t[LU].n, NGL = kG.t[LL].n;
-    __shared__ double lbt[kBoysSlice];
+    constexpr int NGU = kG.t[LU].n, NGL = kG.t[LL].n, TR = transform_rows(LU);
+    constexpr bool OWN = WPB > 1; // transform rows beside the table, not in its place
+    constexpr int NT = TR * NGL;
+    __shared__ double lbt[OWN || kBoysSlice > NT ? kBoysSlice : NT];
     __shared__ double zall[WPB][C::zwords + 1]; // the last word stays 0
-    __shared__ double tall[WPB][kTRows * NGL];
+    __shared__ double tall[OWN ? WPB * NT : 1];
     for (int t = threadIdx.x; t < kBoysSlice; t += 64 * WPB)
-        lbt[t] = btab[(size_t)L * kBoysSlice + t];
+        lbt[t] = btab[(size_t)boys_slice(L) * kBoysSlice + t];
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -556,14 +608,15 @@ k_eri_quartet(SPD sd, const ShellItem *__restrict__ items, int nitems,
             const double T = alpha * fma(X, X, fma(Y, Y, Zc * Zc));
             double F[L + 1];
             boys_table<L>(T, lbt, F);
-            double R[HR];
-            hermite_table<L>(alpha, rs, X, Y, Zc, F, R);
-            static_for<NS>([&](auto i) {
-                constexpr int r = C::sl.r[i], g = C::sl.g[i];
-                if constexpr (C::sl.sig[i] >= 0)
-                    V[i] = fma(R[r], w0, V[i]);
-                else
-                    V[i] = __builtin_amdgcn_mfma_f64_4x4x4f64(R[r], w[g], V[i], 0, 0, 0);
+            hermite_rows<L, quartet_fence(LU, LL, PASS)>(alpha, rs, X, Y, Zc, F, [&](auto rc, double v) {
+                constexpr int r = decltype(rc)::value;
+                static_for<C::count(r)>([&](auto k) {
+                    constexpr int i = C::first(r) + k;
+                    if constexpr (C::sl.sig[i] >= 0)
+                        V[i] = fma(v, w0, V[i]);
+                    else
+                        V[i] = __builtin_amdgcn_mfma_f64_4x4x4f64(v, w[C::sl.g[i]], V[i], 0, 0, 0);
+                });
             });
         }
         // per-lane sums (one of the 4 a each) to tile form: summed over a
@@ -591,12 +644,12 @@ k_eri_quartet(SPD sd, const ShellItem *__restrict__ items, int nitems,
     }
     wave_lds_fence();
     // transform to the components
-    double *T = tall[wave];
+    double *T = OWN ? tall + wave * NT : lbt;
     const int cu0 = sd.coff[it.su], ncu = sd.coff[it.su + 1] - cu0;
     const int ncl = sd.coff[it.sl + 1] - sd.coff[it.sl];
     const double *Gu = gu + sd.goff[it.su], *Gl = gl + sd.goff[it.sl];
-    for (int u0 = 0; u0 < ncu; u0 += kTRows) {
-        const int nu = ncu - u0 < kTRows ? ncu - u0 : kTRows;
+    for (int u0 = 0; u0 < ncu; u0 += TR) {
+        const int nu = ncu - u0 < TR ? ncu - u0 : TR;
         for (int t = lane; t < nu * NGL; t += 64) {
             const int u = t / NGL, jl = t - u * NGL;
             const double *g = Gu + (int64_t)(u0 + u) * NGU;

@@ -223,7 +223,7 @@ __global__ __launch_bounds__(128) void k_one_e_pair(OneEArgs A, const int2 *pair
 {
     constexpr int H = hcount(L);
     __shared__ double lbt[kBoysSlice];
-    for (int t = threadIdx.x; t < kBoysSlice; t += 128) lbt[t] = btab[(size_t)L * kBoysSlice + t];
+    for (int t = threadIdx.x; t < kBoysSlice; t += 128) lbt[t] = btab[(size_t)boys_slice(L) * kBoysSlice + t];
     __syncthreads();
     const int i = pairs[blockIdx.x].x, k = pairs[blockIdx.x].y;
     const int ngi = A.ngauss[i], ngk = A.ngauss[k];
