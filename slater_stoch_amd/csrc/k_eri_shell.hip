@@ -907,8 +907,11 @@ void plan_items(const zv_context *c, const Orient *ors, size_t n, double budget,
         const int npu = c->h_sp_np[o.su], npl = c->h_sp_np[o.sl];
         const int nk = nchunk(npl), nst = nstep(npu), nc = ncu * ncl;
         // slices of chunks first (they repeat the transform only), then of steps;
-        // none much shorter than the transform that it repeats
-        const double least = 3.0 * transform_cost(LU, LL, ncu, ncl);
+        // none shorter than 10 times the transform that it repeats: shorter ones
+        // fill the chip no better and pay for it in partial sums (7 AOs 1.28 ms
+        // at 3 times, 1.14 at 6, 1.05 at 10, 1.13 at 16; 45 AOs 22.5, 20.8, 20.4,
+        // 19.8)
+        const double least = 10.0 * transform_cost(LU, LL, ncu, ncl);
         const double want = std::ceil(o.cost / std::max(budget, least));
         const int kc = (int)std::min<double>(nk, std::max(1.0, want));
         const int ks = (int)std::min<double>(nst, std::max(1.0, std::ceil(want / kc)));
@@ -972,10 +975,11 @@ void plan_shell(const zv_context *c, const std::vector<std::pair<int, int>> &sq,
     });
     double total = 0.0;
     for (const Orient &o : ors) total += o.cost;
-    // items of at most 1/40000 of the total cost: larger quartets are split,
-    // so the sorted queue ends on short items
+    // items of at most 1/20000 of the total cost: larger quartets are split,
+    // so the sorted queue ends on short items (110 AOs 162.7 ms, with 1/40000
+    // 164.7; 128-AO hydrocarbon 409.5 and 410.7)
     const double nitems =
-        c->tune[ZV_TUNE_ERI_ITEMS] > 0 ? (double)c->tune[ZV_TUNE_ERI_ITEMS] : 40000.0;
+        c->tune[ZV_TUNE_ERI_ITEMS] > 0 ? (double)c->tune[ZV_TUNE_ERI_ITEMS] : 20000.0;
     const double budget = std::max(total / nitems, 20000.0);
     pl.host_ms[0] = ms_since(tt);
     tt = clk::now();
