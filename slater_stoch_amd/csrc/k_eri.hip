@@ -184,19 +184,32 @@ __device__ inline void quartet_of(const QSrc &S, int64_t x, int &Pb, int &Pk, in
     oidx = S.mode == Q_LIST ? x : (Pb > Pk ? zv_tri(Pb, Pk) : zv_tri(Pk, Pb));
 }
 
-// Loop order: each lane owns one ket primitive pair (its position, exponent,
-// coefficient and Hermite coefficients stay in registers); the bra primitive
-// pairs are walked in the inner loop with wave-uniform (scalar) loads, so the
-// hot loop issues no vector memory traffic.
+// Loop order: each lane owns one ket primitive pair (its position and exponent
+// in registers, its Hermite coefficients in the lane's LDS column); the bra
+// primitive pairs are walked in the inner loop with wave-uniform (scalar)
+// loads, so the hot loop issues no vector memory traffic.
+//
+// What bounds it: FP64 work of the R table and the HB x HK contraction, with
+// the R table (84 to 165 doubles from L = 6 on) filling the registers.  The
+// contraction therefore runs over the bra index inside: its coefficients are
+// scalars, and each ket coefficient is read from LDS once per primitive
+// quartet, where a ket-inside order kept all HK of them in registers beside R
+// and moved operands through the AGPRs (2000 quartets of
+// all classes 2.2 ms with it and the erf-based Boys values, 1.65 ms here).
 template <int LB, int LK>
 __global__ __launch_bounds__(256) void k_eri_class(PP pp, QSrc S, int nsplit, double *out,
                                                    double *part)
 {
     constexpr int HB = hcount(LB), HK = hcount(LK), L = LB + LK, HR = hcount(L);
-    int lane = threadIdx.x & 63;
+    __shared__ double lbt[kBoysSlice];
+    __shared__ double lek[4][HK][64];
+    for (int t = threadIdx.x; t < kBoysSlice; t += 256)
+        lbt[t] = pp.btab[(size_t)boys_slice(L) * kBoysSlice + t];
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
     // wave index made provably uniform so the per-quartet data come in by scalar loads
-    int64_t item = (int64_t)blockIdx.x * (blockDim.x >> 6) +
-                   __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int64_t item = (int64_t)blockIdx.x * 4 + wave;
     if (item >= S.nq * nsplit) return;
     int64_t x = item / nsplit;
     int sp = (int)(item % nsplit);
@@ -218,34 +231,35 @@ __global__ __launch_bounds__(256) void k_eri_class(PP pp, QSrc S, int nsplit, do
             double q = pp.p[ok + cc], iq = pp.ip[ok + cc];
             double Qx = pp.Px[ok + cc], Qy = pp.Py[ok + cc], Qz = pp.Pz[ok + cc];
             double ck = live ? pp.c[ok + cc] : 0.0;
-            double Ek[HK];
 #pragma unroll
             for (int h = 0; h < HK; h++)
-                Ek[h] = ((kH.t[h] + kH.u[h] + kH.v[h]) & 1) ? -pp.E[ek + (int64_t)h * capk + cc]
-                                                             : pp.E[ek + (int64_t)h * capk + cc];
+                lek[wave][h][lane] = ((kH.t[h] + kH.u[h] + kH.v[h]) & 1)
+                                         ? -pp.E[ek + (int64_t)h * capk + cc]
+                                         : pp.E[ek + (int64_t)h * capk + cc];
             for (int a = a0; a < a1; a++) {
                 double p = pp.p[ob + a], ip = pp.ip[ob + a];
                 double X = pp.Px[ob + a] - Qx, Y = pp.Py[ob + a] - Qy, Z = pp.Pz[ob + a] - Qz;
                 double cb = pp.c[ob + a];
                 double s = p + q;
-                double is = 1.0 / s;
-                double alpha = (p * q) * is;
+                double rs = rsqrt_pos(s);
+                double alpha = (p * q) * (rs * rs);
                 double T = alpha * ((X * X + Y * Y) + Z * Z);
                 double F[L + 1];
-                boys<L>(T, F);
+                boys_table<L>(T, lbt, F);
                 double R[HR];
                 hermite_R<L>(alpha, X, Y, Z, F, R);
                 double sum = 0.0;
 #pragma unroll
-                for (int hb = 0; hb < HB; hb++) {
+                for (int hk = 0; hk < HK; hk++) {
                     double w = 0.0;
 #pragma unroll
-                    for (int hk = 0; hk < HK; hk++)
-                        w = fma(Ek[hk], R[hidx(kH.t[hb] + kH.t[hk], kH.u[hb] + kH.u[hk],
-                                                kH.v[hb] + kH.v[hk])], w);
-                    sum = fma(pp.E[eb + (int64_t)hb * capb + a], w, sum);
+                    for (int hb = 0; hb < HB; hb++)
+                        w = fma(pp.E[eb + (int64_t)hb * capb + a],
+                                R[hidx(kH.t[hb] + kH.t[hk], kH.u[hb] + kH.u[hk],
+                                       kH.v[hb] + kH.v[hk])], w);
+                    sum = fma(lek[wave][hk][lane], w, sum);
                 }
-                double pref = ((kPi52 * ip) * iq) * sqrt(is);
+                double pref = ((kPi52 * ip) * iq) * rs;
                 acc = fma((cb * ck) * pref, sum, acc);
             }
         }
@@ -329,6 +343,28 @@ __global__ void k_reduce_parts(QSrc S, int nsplit, const double *part, double *o
     double s = 0.0;
     for (int t = 0; t < nsplit; t++) s += part[x * nsplit + t];
     out[oidx] = s;
+}
+
+// the same over the classes of one list: class b holds list entries
+// lo[b] .. lo[b+1] - 1 and its partial sums start at poff[b] (ns[b] each; none
+// where ns[b] = 1)
+constexpr int kListCls = (ZV_LMAX_T + 2) * (ZV_LMAX_T + 2);
+struct ListParts {
+    int64_t lo[kListCls + 1], poff[kListCls];
+    int ns[kListCls];
+};
+
+__global__ void k_reduce_list(ListParts lp, const double *part, double *out)
+{
+    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= lp.lo[kListCls]) return;
+    int b = 0;
+    while (x >= lp.lo[b + 1]) b++;
+    if (lp.ns[b] <= 1) return;
+    const double *p = part + lp.poff[b] + (x - lp.lo[b]) * lp.ns[b];
+    double s = 0.0;
+    for (int t = 0; t < lp.ns[b]; t++) s += p[t];
+    out[x] = s;
 }
 
 __global__ void k_diag_pre(int np, const double *tri, double *pre)
@@ -531,28 +567,38 @@ static double component_flops(int LB, int LK)
 // pairs when there are too few quartets to fill the device.  pq and flops
 // (primitive quartets and algorithmic flops of the list) feed the statistics.
 // Split of a class launch over the bra primitive pairs: short lists are
-// spread over up to 32 waves per quartet, about 16384 waves in all.  The
-// partial sums then take nq * nsplit < 16384 + nq doubles.
+// spread over up to 128 waves per quartet, about 16384 waves in all (a pair
+// holds up to a few hundred primitive pairs, and the longest waves decide:
+// 2000 quartets 1.61 ms with at most 32, 1.40 with 64, 1.32 with 128, 1.40
+// with 256).  The partial sums then take nq * nsplit < 16384 + nq doubles.
 static int class_split(int64_t nq)
 {
     const int64_t target_waves = 16384;
     if (nq >= target_waves) return 1;
-    return (int)std::min<int64_t>(32, (target_waves + nq - 1) / nq);
+    return (int)std::min<int64_t>(128, (target_waves + nq - 1) / nq);
+}
+
+// The class kernel of one list on stream st.
+static int launch_class_on(zv_context *c, hipStream_t st, const PP &pp, QSrc S, int LB, int LK,
+                           double *out, double *part, int nsplit)
+{
+    int64_t items = S.nq * nsplit;
+    if (LB <= ZV_LMAX_T && LK <= ZV_LMAX_T) {
+        if (!launch_class_t(LB, LK, nblk(items * 64, 256), st, pp, S, nsplit, out, part))
+            return zv_fail(c, ZV_ERR_STATE, "no ERI kernel for class (%d,%d)", LB, LK);
+    } else {
+        hipLaunchKernelGGL(k_eri_generic, dim3(nblk(items * 64, 64)), dim3(64), 0, st, pp, S,
+                           nsplit, out, part);
+    }
+    ZV_HIPCHECK(c, hipGetLastError());
+    return ZV_OK;
 }
 
 // The kernels of one class: no allocation, no timing.
 static int launch_class_raw(zv_context *c, const PP &pp, QSrc S, int LB, int LK, double *out,
                             double *part, int nsplit)
 {
-    int64_t items = S.nq * nsplit;
-    if (LB <= ZV_LMAX_T && LK <= ZV_LMAX_T) {
-        if (!launch_class_t(LB, LK, nblk(items * 64, 256), c->stream, pp, S, nsplit, out, part))
-            return zv_fail(c, ZV_ERR_STATE, "no ERI kernel for class (%d,%d)", LB, LK);
-    } else {
-        hipLaunchKernelGGL(k_eri_generic, dim3(nblk(items * 64, 64)), dim3(64), 0, c->stream, pp,
-                           S, nsplit, out, part);
-    }
-    ZV_HIPCHECK(c, hipGetLastError());
+    ZV_CHECK(launch_class_on(c, c->stream, pp, S, LB, LK, out, part, nsplit));
     if (nsplit > 1) {
         hipLaunchKernelGGL(k_reduce_parts, dim3(nblk(S.nq, 256)), dim3(256), 0, c->stream, S,
                            nsplit, (const double *)part, out);
@@ -761,7 +807,7 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
 {
     PP pp;
     ZV_CHECK(ensure_primpairs(c, pp));
-    int ncls = ZV_LMAX_T + 2;
+    constexpr int ncls = ZV_LMAX_T + 2;
     auto order = [&](int P) {
         int L = c->h_pair_L[P];
         return L > ZV_LMAX_T ? ZV_LMAX_T + 1 : L;
@@ -802,11 +848,66 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
                                   c->stream));
     ZV_CHECK(zv_ensure(c, c->b_out, sizeof(double) * nq));
     double *dout = (double *)c->b_out.p;
-    for (int b = 0; b < ncls * ncls; b++) {
-        int64_t cnt = lo[b + 1] - lo[b];
-        if (!cnt) continue;
-        QSrc S{Q_LIST, dqb + lo[b], dqk + lo[b], cnt};
-        ZV_CHECK(launch_class(c, pp, S, b / ncls, b % ncls, dout + lo[b], bpq[b], bfl[b]));
+    // The classes write disjoint parts of the list, so they run side by side on
+    // the context's stream and its side streams, the costliest first, each on
+    // the stream with the least work so far: a class of a few hundred quartets
+    // ends on long waves that leave most of the chip idle (15 classes of 2000
+    // quartets: 3.25 ms one after another, 2.2 ms
+    // side by side).  Runtime orders stay on the context's
+    // stream, whose scratch memory they need.
+    static_assert(ncls * ncls == kListCls, "list classes");
+    ListParts lp;
+    int64_t npart = 0;
+    for (int b = 0; b < kListCls; b++) {
+        lp.lo[b] = lo[b];
+        lp.ns[b] = class_split(std::max<int64_t>(lo[b + 1] - lo[b], 1));
+        lp.poff[b] = npart;
+        if (lp.ns[b] > 1) npart += (lo[b + 1] - lo[b]) * lp.ns[b];
+    }
+    lp.lo[kListCls] = nq;
+    if (npart) ZV_CHECK(zv_ensure(c, c->b_part, sizeof(double) * npart));
+    double *part = (double *)c->b_part.p;
+    {
+        constexpr int NST = 1 + zv_context::NSIDE;
+        hipStream_t sts[NST] = {c->stream};
+        for (int k = 0; k < zv_context::NSIDE; k++) sts[1 + k] = c->side[k];
+        int cl[kListCls], nc = 0;
+        for (int b = 0; b < kListCls; b++)
+            if (lo[b + 1] > lo[b]) cl[nc++] = b;
+        std::sort(cl, cl + nc, [&](int x, int y) { return bfl[x] > bfl[y]; });
+        const int nst = nc > 1 ? NST : 1;
+        double load[NST] = {};
+        PhaseTimer wall(c, PH_ERI);
+        if (nst > 1) {
+            ZV_HIPCHECK(c, hipEventRecord(c->ev_fork, c->stream));
+            for (int k = 0; k < zv_context::NSIDE; k++)
+                ZV_HIPCHECK(c, hipStreamWaitEvent(c->side[k], c->ev_fork, 0));
+        }
+        for (int t = 0; t < nc; t++) {
+            const int b = cl[t], LB = b / ncls, LK = b % ncls;
+            int s = 0;
+            if (LB <= ZV_LMAX_T && LK <= ZV_LMAX_T)
+                for (int q = 1; q < nst; q++)
+                    if (load[q] < load[s]) s = q;
+            load[s] += bfl[b];
+            const int slot = LB * 6 + LK;
+            c->cls_pq[slot] += bpq[b];
+            c->cls_flops[slot] += bfl[b];
+            PhaseTimer tm(c, PH_N, slot, sts[s]);
+            QSrc S{Q_LIST, dqb + lo[b], dqk + lo[b], lo[b + 1] - lo[b]};
+            ZV_CHECK(launch_class_on(c, sts[s], pp, S, LB, LK, dout + lo[b], part + lp.poff[b],
+                                     lp.ns[b]));
+        }
+        if (nst > 1)
+            for (int k = 0; k < zv_context::NSIDE; k++) {
+                ZV_HIPCHECK(c, hipEventRecord(c->ev_join[k], c->side[k]));
+                ZV_HIPCHECK(c, hipStreamWaitEvent(c->stream, c->ev_join[k], 0));
+            }
+        if (npart) {
+            hipLaunchKernelGGL(k_reduce_list, dim3(nblk(nq, 256)), dim3(256), 0, c->stream, lp,
+                               (const double *)part, dout);
+            ZV_HIPCHECK(c, hipGetLastError());
+        }
     }
     std::vector<double> h(nq);
     ZV_HIPCHECK(c, hipMemcpyAsync(h.data(), dout, sizeof(double) * nq, hipMemcpyDeviceToHost,

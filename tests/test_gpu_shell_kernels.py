@@ -40,3 +40,31 @@ def test_shell_kernels_at_tile_edges(engine, oracle, ng):
     oracle.set_basis(bas)
     ref, _ = oracle.gauss_eri([a[pick] for a in q], None)
     np.testing.assert_allclose(eri[pick], ref, rtol=1e-10, atol=1e-12 * np.abs(ref).max())
+
+
+# lists short enough for the largest split of a quartet over waves (more waves
+# than the one or 16 primitive pairs of a pair), of mixed splits and with
+# classes of one wave per quartet; f x f pairs reach the runtime-order kernel
+@pytest.mark.parametrize("nq,ng", [(1, 4), (40, 1), (40, 4), (1500, 7), (60000, 2)])
+def test_list_classes_side_by_side(engine, nq, ng):
+    geom = B.geometry_from_angstrom(["O", "H"], [[0.05, -0.1, 0.2], [0.7, 0.4, -0.5]])
+    basis = {"O": [("1S", 2.6), ("2S", 1.9), ("2P", 2.1), ("3D", 1.7)],
+             "H": [("1S", 1.2), ("3P", 1.4), ("4F", 1.8)]}
+    bas = B.expand_basis(geom, basis, ng0=ng)
+    engine.set_basis(bas)
+    eri, _, _ = engine.gauss_eri()
+    qi, qj, qk, ql = B.quartet_mapping(bas.n)
+    full = np.empty((bas.n + 1,) * 4)
+    for a, b in ((qi, qk), (qk, qi)):
+        for c, d in ((qj, ql), (ql, qj)):
+            full[a, b, c, d] = eri
+            full[c, d, a, b] = eri
+    rng = np.random.default_rng(nq)
+    i, k, j, l = rng.integers(1, bas.n + 1, (4, nq))
+    got = engine.gauss_ijkl(i, k, j, l)
+    # the tolerance of the other comparison of the two sets of kernels
+    np.testing.assert_allclose(got, full[i, k, j, l], rtol=1e-12,
+                               atol=1e-15 * np.abs(eri).max())
+    np.testing.assert_array_equal(engine.gauss_ijkl(i, k, j, l), got)
+    if nq <= 16384:
+        np.testing.assert_array_equal(engine.gauss_ijkl_noalloc(i, k, j, l), got)
