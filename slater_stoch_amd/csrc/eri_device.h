@@ -48,7 +48,7 @@ struct PP {
     const int64_t *off, *eoff;          // per pair
     const int *cap;                     // n_gauss(i) n_gauss(k)
     const int *L;                       // Hermite order per pair
-    const double *btab;                 // Boys Taylor table [L][k][i] (boys_table)
+    const double *btab;                 // Boys tables of all orders (boys_table)
 };
 
 // ------------------------------------------------------------------ Boys
@@ -98,27 +98,47 @@ template <int L> __device__ inline void boys(double T, double *F)
     }
 }
 
-// Tabulated Boys function (shell kernels, one-electron kernels): for T < 36 a
-// Taylor expansion about the nearest grid point T_i = i / 2, |d| <= 1/4,
-//   F_L(T_i + d) = sum_k (-1)^k F_{L+k}(T_i) d^k / k!,
-// with the terms k <= 12 (remainder below 3e-18 of F_L); the table holds
-// (-1)^k F_{L+k}(T_i) / k! for L <= 8, k <= 14, computed on the host in
-// extended precision from the series F_m(T) = exp(-T) sum_j (2T)^j /
-// ((2m+1)(2m+3)...(2m+2j+1)) (zv_boys_table).  Orders below L follow by the
-// stable downward recursion F_m = (2 T F_{m+1} + exp(-T)) / (2m + 1) for
-// L >= 3.  For L <= 2 they are the derivatives of the F_0 expansion instead
-// (F_1 = -F_0', F_2 = F_0''; two and four terms more, Horner's scheme for all
-// of them at once): 12 + 13 multiply-adds for L = 1 where the exponential and
-// its constants take about 40 instructions.  From T = 36 on the branch of
-// boys<L> (F_0 = sqrt(pi/T)/2, erf rounding to 1, upward recursion), whose
-// exponential is skipped by a wave beyond T = 80.  Relative error below 1e-15
-// against the series in extended precision; one code path for all T < 36,
-// where boys<L> splits at T = 1 and evaluates erf above it.  lt: the kernel's
-// LDS copy of slice boys_slice(L), [k][i].
-constexpr int kBoysK = 14, kBoysN = 73; // orders 0..kBoysK, grid 0, 0.5, .., 36
-constexpr int kBoysLmax = 8;
-constexpr int kBoysSlice = (kBoysK + 1) * kBoysN;
-constexpr int boys_slice(int L) { return L <= 2 ? 0 : L; }
+// Tabulated Boys function: polynomials in d = T - T_i about the nearest grid
+// point T_i = i h, |d| <= h/2.  The Taylor series
+//   F_m(T_i + d) = sum_k (-1)^k F_{m+k}(T_i) d^k / k!
+// taken to k = 20 is economized (highest Chebyshev term after highest term
+// dropped) to a polynomial q of degree boys_deg, within 6e-18 of F_L, on the
+// host in extended precision (zv_boys_table).  Three forms:
+//   L = 0:      q is F_0.
+//   L = 1..5:   the table holds p = F_{L-1}(T_i) - int q, whose derivative
+//               is -F_L: one Horner scheme gives both, and the orders below
+//               follow from F_{m-1} = (2 T F_m + exp(-T)) / (2m - 1), with
+//               exp(-T) = (2L-1) F_{L-1} - 2T F_L.  That difference is as
+//               accurate as each step needs (its error is an ulp of 2T F_L,
+//               which the step adds to 2T F_{L-1} > 2T F_L), and the
+//               exponential's 20 operations and 20 constants are saved.  From
+//               boys_tmax on, where Gamma(L+1/2, T) / Gamma(L+1/2) is below
+//               4e-17, F_m is the complete integral, again without exp.
+//   L = 6..8:   F_L from q and the exponential, and the upward recursion with
+//               it from T = 36 on: these kernels have no LDS for the longer
+//               table and spend 2 % of their time here.
+// A grid of h = 1/4 takes 9 + 8 multiply-adds for L = 1..4, h = 1/2 two more
+// of each; Taylor terms to the same error about 13 + 12.  Relative error below
+// 1.2e-15 against the series in extended precision.
+// lt: the kernel's LDS copy of the table of order L, [i][k]: the coefficients
+// of one expansion lie together, two to a read.
+// Against the 13-term expansions, [k][i], with exp for L >= 3 and T >= 36
+// (cycles per wave and 64 primitive quartets, 128-AO hydrocarbon): (0,1)
+// 426 -> 339, (1,1) 666 -> 551, (1,2) 979 -> 831, (2,2) 1681 -> 1589,
+// (2,3) 3288 -> 3111, of which the layout is a tenth to a third.
+constexpr int kBoysLmax = 8, kBoysM = 20;
+constexpr bool boys_pair(int L) { return L >= 1 && L <= 5; }
+constexpr int boys_inv_h(int L) { return L <= 4 ? 4 : 2; }
+constexpr int boys_deg(int L) { return L <= 4 ? 8 : 10; }
+constexpr double boys_tmax(int L)
+{
+    constexpr double t[kBoysLmax + 1] = {36.0, 40.0, 43.5, 46.5, 49.5, 52.0, 36.0, 36.0, 36.0};
+    return t[L];
+}
+constexpr int boys_rows(int L) { return boys_deg(L) + (boys_pair(L) ? 2 : 1); }
+constexpr int boys_cols(int L) { return (int)(boys_tmax(L) * boys_inv_h(L)) + 1; }
+constexpr int boys_words(int L) { return boys_rows(L) * boys_cols(L); }
+constexpr int boys_off(int L) { return L == 0 ? 0 : boys_off(L - 1) + boys_words(L - 1); }
 
 // 1/sqrt(x) for a positive normal x: the hardware estimate (about 5e-8
 // relative) and one third-order step y' = y (1 + e/2 + 3 e^2/8), e = 1 - x y^2
@@ -133,41 +153,45 @@ __device__ inline double rsqrt_pos(double x)
 
 template <int L> __device__ inline void boys_table(double T, const double *lt, double *F)
 {
-    if (T < 36.0) {
-        const int i = (int)(T * 2.0 + 0.5);
-        const double d = T - 0.5 * (double)i;
-        if constexpr (L <= 2) {
-            constexpr int K = 12 + L;
-            double b0 = lt[K * kBoysN + i], b1 = 0.0, b2 = 0.0;
+    constexpr int K = boys_rows(L) - 1;
+    if (T < boys_tmax(L)) {
+        const int i = (int)(T * boys_inv_h(L) + 0.5);
+        const double d = T - (1.0 / boys_inv_h(L)) * (double)i;
+        const double *c = lt + i * (K + 1);
+        double b0 = c[K], b1 = 0.0;
 #pragma unroll
-            for (int k = K - 1; k >= 0; k--) {
-                if (L >= 2 && k <= K - 2) b2 = k == K - 2 ? b1 : fma(b2, d, b1);
-                if (L >= 1) b1 = k == K - 1 ? b0 : fma(b1, d, b0);
-                b0 = fma(b0, d, lt[k * kBoysN + i]);
-            }
+        for (int k = K - 1; k >= 0; k--) {
+            if constexpr (boys_pair(L)) b1 = k == K - 1 ? b0 : fma(b1, d, b0);
+            b0 = fma(b0, d, c[k]);
+        }
+        if constexpr (L == 0) {
             F[0] = b0;
-            if constexpr (L >= 1) F[1] = -b1;
-            if constexpr (L >= 2) F[2] = 2.0 * b2;
         } else {
-            constexpr int K = 12;
-            double s = lt[K * kBoysN + i];
+            const double t2 = 2.0 * T;
+            double e;
+            if constexpr (boys_pair(L)) {
+                F[L - 1] = b0;
+                F[L] = -b1;
+                e = fma(t2, b1, (2 * L - 1) * b0);
+            } else {
+                F[L] = b0;
+                e = exp(-T);
+                F[L - 1] = fma(t2, F[L], e) * (1.0 / (2 * L - 1));
+            }
 #pragma unroll
-            for (int k = K - 1; k >= 0; k--) s = fma(s, d, lt[k * kBoysN + i]);
-            F[L] = s;
-            const double e = exp(-T);
-#pragma unroll
-            for (int m = L - 1; m >= 0; m--)
-                F[m] = fma(2.0 * T, F[m + 1], e) * (1.0 / (2 * m + 1));
+            for (int m = L - 2; m >= 0; m--) F[m] = fma(t2, F[m + 1], e) * (1.0 / (2 * m + 1));
         }
     } else {
         const double u_inv = rsqrt_pos(T);
         F[0] = (0.5 * u_inv) * kSqrtPi;
-        if (L > 0) {
-            double e = 0.0;
-            if (T <= 80.0) e = exp(-T);
+        if constexpr (L > 0) {
             const double tri = (0.5 * u_inv) * u_inv;
+            double e = 0.0;
+            if constexpr (!boys_pair(L))
+                if (T <= 80.0) e = exp(-T);
 #pragma unroll
-            for (int m = 0; m < L; m++) F[m + 1] = (F[m] * (2 * m + 1) - e) * tri;
+            for (int m = 0; m < L; m++)
+                F[m + 1] = boys_pair(L) ? F[m] * ((2 * m + 1) * tri) : (F[m] * (2 * m + 1) - e) * tri;
         }
     }
 }

@@ -524,7 +524,8 @@ constexpr int quartet_lds(int LU, int LL, int p)
 constexpr int quartet_waves(int LU, int LL, int p)
 {
     return quartet_regs(LU, LL, p, true) <= 250 &&
-                   (4 * quartet_lds(LU, LL, p) + kBoysSlice) * 8 <= 81920
+                   (4 * quartet_lds(LU, LL, p) + boys_words(pass_of(LU, LL, p).rho1)) * 8 <=
+                       81920
                ? 2
                : 1;
 }
@@ -551,11 +552,10 @@ k_eri_quartet(SPD sd, const ShellItem *__restrict__ items, int nitems,
     constexpr int NGU = kG.t[LU].n, NGL = kG.t[LL].n, TR = transform_rows(LU);
     constexpr bool OWN = WPB > 1; // transform rows beside the table, not in its place
     constexpr int NT = TR * NGL;
-    __shared__ double lbt[OWN || kBoysSlice > NT ? kBoysSlice : NT];
+    __shared__ __align__(16) double lbt[OWN || boys_words(L) > NT ? boys_words(L) : NT];
     __shared__ double zall[WPB][C::zwords + 1]; // the last word stays 0
     __shared__ double tall[OWN ? WPB * NT : 1];
-    for (int t = threadIdx.x; t < kBoysSlice; t += 64 * WPB)
-        lbt[t] = btab[(size_t)boys_slice(L) * kBoysSlice + t];
+    for (int t = threadIdx.x; t < boys_words(L); t += 64 * WPB) lbt[t] = btab[boys_off(L) + t];
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -1085,6 +1085,73 @@ static SPD spd_of(zv_context *c)
     const double *g = (const double *)c->b_spe.p;
     return SPD{d_comp, d_coff, d_np, d_roff, d_goff, (const double *)c->b_spu.p, g,
                g + c->sp_g_total};
+}
+
+// The Boys tables of boys_table (eri_device.h), computed once per process in
+// extended precision (x87 long double on the host).
+// F_m(T) = exp(-T) sum_j (2T)^j / ((2m+1)(2m+3)...(2m+2j+1)), all terms
+// positive, summed until they fall below 1e-22 of the sum, for the highest m;
+// the others by the stable downward recursion.
+static const std::vector<double> &boys_table_host()
+{
+    static std::vector<double> tab;
+    if (!tab.empty()) return tab;
+    typedef long double LD;
+    constexpr int M = kBoysM, NM = kBoysLmax + M;
+    // Chebyshev polynomials T_k in powers of x
+    LD ch[M + 1][M + 1] = {};
+    ch[0][0] = ch[1][1] = 1.0L;
+    for (int k = 2; k <= M; k++)
+        for (int j = 0; j <= k; j++)
+            ch[k][j] = (j ? 2.0L * ch[k - 1][j - 1] : 0.0L) - ch[k - 2][j];
+    std::vector<double> t((size_t)boys_off(kBoysLmax + 1));
+    for (int L = 0; L <= kBoysLmax; L++)
+        for (int i = 0; i < boys_cols(L); i++) {
+            const LD T = (LD)i / boys_inv_h(L), delta = 0.5L / boys_inv_h(L), ex = expl(-T);
+            LD F[NM + 1], term = 1.0L / (2 * NM + 1), sum = term;
+            for (int j = 1; j < 2000; j++) {
+                term *= 2.0L * T / (2 * NM + 2 * j + 1);
+                sum += term;
+                if (term < 1e-22L * sum) break;
+            }
+            F[NM] = sum * ex;
+            for (int m = NM - 1; m >= 0; m--) F[m] = (2.0L * T * F[m + 1] + ex) / (2 * m + 1);
+            // q in powers of x = d / delta
+            const int D = boys_deg(L);
+            LD q[M + 1], s = 1.0L;
+            for (int k = 0; k <= M; k++) {
+                q[k] = F[L + k] * s;
+                s *= -delta / (k + 1);
+            }
+            for (int k = M; k > D; k--) {
+                const LD a = q[k] / ch[k][k];
+                for (int j = 0; j <= k; j++) q[j] -= a * ch[k][j];
+            }
+            double *o = t.data() + boys_off(L) + (size_t)i * boys_rows(L);
+            if (boys_pair(L)) o[0] = (double)F[L - 1];
+            s = 1.0L;
+            for (int k = 0; k <= D; k++) {
+                const LD v = q[k] * s;
+                s /= delta;
+                if (boys_pair(L)) o[k + 1] = (double)(-v / (k + 1));
+                else o[k] = (double)v;
+            }
+        }
+    tab.swap(t);
+    return tab;
+}
+
+// the table on the context's device (once per context)
+int zv_boys_table(zv_context *c, const double **tab)
+{
+    const std::vector<double> &t = boys_table_host();
+    ZV_CHECK(zv_ensure(c, c->b_btab, sizeof(double) * t.size()));
+    *tab = (const double *)c->b_btab.p;
+    if (c->btab_ready) return ZV_OK;
+    ZV_HIPCHECK(c, hipMemcpyAsync(c->b_btab.p, t.data(), sizeof(double) * t.size(),
+                                  hipMemcpyHostToDevice, c->stream));
+    c->btab_ready = true;
+    return ZV_OK;
 }
 
 int zv_shell_ready(zv_context *c, const PP &pp)

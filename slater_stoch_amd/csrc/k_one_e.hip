@@ -222,8 +222,8 @@ __global__ __launch_bounds__(128) void k_one_e_pair(OneEArgs A, const int2 *pair
                                                     const double *btab)
 {
     constexpr int H = hcount(L);
-    __shared__ double lbt[kBoysSlice];
-    for (int t = threadIdx.x; t < kBoysSlice; t += 128) lbt[t] = btab[(size_t)boys_slice(L) * kBoysSlice + t];
+    __shared__ __align__(16) double lbt[boys_words(L)];
+    for (int t = threadIdx.x; t < boys_words(L); t += 128) lbt[t] = btab[boys_off(L) + t];
     __syncthreads();
     const int i = pairs[blockIdx.x].x, k = pairs[blockIdx.x].y;
     const int ngi = A.ngauss[i], ngk = A.ngauss[k];

@@ -83,7 +83,7 @@ struct zv_context {
     bool res_valid[3] = {false, false, false};
     DevBuf b_mpart;                    // estimator sums per (block, sample split) of a round
     DevBuf b_pp;                       // primitive-pair data
-    DevBuf b_btab;                     // Boys Taylor table (zv_boys_table)
+    DevBuf b_btab;                     // Boys tables (zv_boys_table)
     bool btab_ready = false;
     DevBuf b_mono;                     // angular table of the one-centre integrals (k_mono.hip)
     bool mono_ready = false;
@@ -191,7 +191,7 @@ int zv_run_draw(zv_context *c, uint64_t seed, uint64_t stream, int64_t m0, int64
 int zv_run_pair_samples(zv_context *c, int i, int k, int ns, const double *r1, const double *r2,
                         double *ut1, double *ut2, double *rho1, double *rho2, double *rhog1,
                         double *rhog2, double *jac1, double *jac2);
-// device copy of the Boys Taylor table (k_eri.hip), made on first use
+// device copy of the Boys tables (k_eri_shell.hip), made on first use
 int zv_boys_table(zv_context *c, const double **tab);
 int zv_run_gauss_eri(zv_context *c, double *ijkl, double *precond, int64_t *n_screened);
 int zv_run_exact_monocenter(zv_context *c, double *ijkl, double *err, int64_t *n_mono);
