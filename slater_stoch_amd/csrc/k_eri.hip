@@ -34,6 +34,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <map>
+#include <optional>
 #include <thread>
 
 #include "eri_device.h"
@@ -331,17 +332,27 @@ __global__ __launch_bounds__(64) void k_eri_generic(PP pp, QSrc S, int nsplit, d
     }
 }
 
-// ordered sum of the split partials of each quartet
-__global__ void k_reduce_parts(QSrc S, int nsplit, const double *part, double *out)
+// Sum of a quartet's n <= 128 partial sums by one wave, lanes adding two each:
+// one thread adding them all took 20 us of a call on one quartet.
+__device__ inline double wave_sum_parts(const double *p, int n, int lane)
 {
-    int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    double s = lane < n ? p[lane] : 0.0;
+    if (lane + 64 < n) s += p[lane + 64];
+    return wave_sum(s);
+}
+
+// the split partials of each quartet of a class, one wave each
+__global__ __launch_bounds__(256) void k_reduce_parts(QSrc S, int nsplit, const double *part,
+                                                      double *out)
+{
+    const int64_t x = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (x >= S.nq) return;
     int Pb, Pk;
     int64_t oidx;
     quartet_of(S, x, Pb, Pk, oidx);
-    double s = 0.0;
-    for (int t = 0; t < nsplit; t++) s += part[x * nsplit + t];
-    out[oidx] = s;
+    const int lane = threadIdx.x & 63;
+    const double s = wave_sum_parts(part + x * nsplit, nsplit, lane);
+    if (lane == 0) out[oidx] = s;
 }
 
 // the same over the classes of one list: class b holds list entries
@@ -353,17 +364,16 @@ struct ListParts {
     int ns[kListCls];
 };
 
-__global__ void k_reduce_list(ListParts lp, const double *part, double *out)
+__global__ __launch_bounds__(256) void k_reduce_list(ListParts lp, const double *part, double *out)
 {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t x = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (x >= lp.lo[kListCls]) return;
     int b = 0;
     while (x >= lp.lo[b + 1]) b++;
     if (lp.ns[b] <= 1) return;
-    const double *p = part + lp.poff[b] + (x - lp.lo[b]) * lp.ns[b];
-    double s = 0.0;
-    for (int t = 0; t < lp.ns[b]; t++) s += p[t];
-    out[x] = s;
+    const int lane = threadIdx.x & 63;
+    const double s = wave_sum_parts(part + lp.poff[b] + (x - lp.lo[b]) * lp.ns[b], lp.ns[b], lane);
+    if (lane == 0) out[x] = s;
 }
 
 __global__ void k_diag_pre(int np, const double *tri, double *pre)
@@ -509,16 +519,17 @@ static double component_flops(int LB, int LK)
 // Launch one class over an explicit quartet list S, splitting bra primitive
 // pairs when there are too few quartets to fill the device.  pq and flops
 // (primitive quartets and algorithmic flops of the list) feed the statistics.
-// Split of a class launch over the bra primitive pairs: short lists are
-// spread over up to 128 waves per quartet, about 16384 waves in all (a pair
-// holds up to a few hundred primitive pairs, and the longest waves decide:
-// 2000 quartets 1.61 ms with at most 32, 1.40 with 64, 1.32 with 128, 1.40
-// with 256).  The partial sums then take nq * nsplit < 16384 + nq doubles.
-static int class_split(int64_t nq)
+// Split of a class launch over the bra primitive pairs, of which its longest
+// quartet has nbra: short lists are spread over up to 128 waves per quartet,
+// about 16384 waves in all (the longest waves decide: 2000 quartets 1.61 ms
+// with at most 32, 1.40 with 64, 1.32 with 128, 1.40 with 256).  The partial
+// sums then take nq * nsplit < 16384 + nq doubles.
+static int class_split(int64_t nq, int nbra)
 {
     const int64_t target_waves = 16384;
     if (nq >= target_waves) return 1;
-    return (int)std::min<int64_t>(128, (target_waves + nq - 1) / nq);
+    return (int)std::min<int64_t>(std::min(128, std::max(nbra, 1)),
+                                  (target_waves + nq - 1) / nq);
 }
 
 // The class kernel of one list on stream st.
@@ -543,7 +554,7 @@ static int launch_class_raw(zv_context *c, const PP &pp, QSrc S, int LB, int LK,
 {
     ZV_CHECK(launch_class_on(c, c->stream, pp, S, LB, LK, out, part, nsplit));
     if (nsplit > 1) {
-        hipLaunchKernelGGL(k_reduce_parts, dim3(nblk(S.nq, 256)), dim3(256), 0, c->stream, S,
+        hipLaunchKernelGGL(k_reduce_parts, dim3(nblk(S.nq, 4)), dim3(256), 0, c->stream, S,
                            nsplit, (const double *)part, out);
         ZV_HIPCHECK(c, hipGetLastError());
     }
@@ -551,10 +562,10 @@ static int launch_class_raw(zv_context *c, const PP &pp, QSrc S, int LB, int LK,
 }
 
 static int launch_class(zv_context *c, const PP &pp, QSrc S, int LB, int LK, double *out,
-                        double pq, double flops)
+                        int nbra, double pq, double flops)
 {
     if (S.nq <= 0) return ZV_OK;
-    const int nsplit = class_split(S.nq);
+    const int nsplit = class_split(S.nq, nbra);
     double *part = nullptr;
     if (nsplit > 1) {
         ZV_CHECK(zv_ensure(c, c->b_part, sizeof(double) * S.nq * nsplit));
@@ -575,7 +586,9 @@ static int run_generic_pairs(zv_context *c, const PP &pp, const std::vector<int>
     const int64_t nq = (int64_t)qb.size();
     if (!nq) return ZV_OK;
     double pq = 0.0, flops = 0.0;
+    int nbra = 0;
     for (int64_t t = 0; t < nq; t++) {
+        nbra = std::max(nbra, c->h_cnt[qb[t]]);
         double v = (double)c->h_cnt[qb[t]] * c->h_cnt[qk[t]];
         pq += v;
         flops += v * component_flops(c->h_pair_L[qb[t]], c->h_pair_L[qk[t]]);
@@ -588,7 +601,7 @@ static int run_generic_pairs(zv_context *c, const PP &pp, const std::vector<int>
     ZV_HIPCHECK(c, hipMemcpyAsync(d, c->h_plist.data(), sizeof(int) * 2 * nq,
                                   hipMemcpyHostToDevice, c->stream));
     QSrc S{Q_PAIRS, d, d + nq, nq};
-    return launch_class(c, pp, S, ZV_LMAX_T + 1, ZV_LMAX_T + 1, tri, pq, flops);
+    return launch_class(c, pp, S, ZV_LMAX_T + 1, ZV_LMAX_T + 1, tri, nbra, pq, flops);
 }
 
 // The reference's Schwarz driver (src/two_e_slater.F90:230-273) over shell
@@ -771,6 +784,7 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
     std::vector<int64_t> perm;
     std::vector<int64_t> lo(ncls * ncls + 1, 0);
     std::vector<double> bpq(ncls * ncls, 0.0), bfl(ncls * ncls, 0.0);
+    std::vector<int> bnb(ncls * ncls, 0);
     for (int b = 0; b < ncls * ncls; b++) {
         lo[b] = (int64_t)perm.size();
         for (int64_t t : bucket[b]) {
@@ -779,6 +793,7 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
             qk2.push_back(pk[t]);
             double v = (double)c->h_cnt[pb[t]] * c->h_cnt[pk[t]];
             bpq[b] += v;
+            bnb[b] = std::max(bnb[b], c->h_cnt[pb[t]]);
             bfl[b] += v * component_flops(c->h_pair_L[pb[t]], c->h_pair_L[pk[t]]);
         }
     }
@@ -803,7 +818,7 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
     int64_t npart = 0;
     for (int b = 0; b < kListCls; b++) {
         lp.lo[b] = lo[b];
-        lp.ns[b] = class_split(std::max<int64_t>(lo[b + 1] - lo[b], 1));
+        lp.ns[b] = class_split(std::max<int64_t>(lo[b + 1] - lo[b], 1), bnb[b]);
         lp.poff[b] = npart;
         if (lp.ns[b] > 1) npart += (lo[b + 1] - lo[b]) * lp.ns[b];
     }
@@ -818,10 +833,16 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
         for (int b = 0; b < kListCls; b++)
             if (lo[b + 1] > lo[b]) cl[nc++] = b;
         std::sort(cl, cl + nc, [&](int x, int y) { return bfl[x] > bfl[y]; });
-        const int nst = nc > 1 ? NST : 1;
+        // below 4 Mflop in all the fork and join (about 25 us) cost more than the
+        // launches that they overlap (10 quartets of 16 x 16 primitive pairs: even)
+        double total = 0.0;
+        for (int t = 0; t < nc; t++) total += bfl[cl[t]];
+        const int nst = nc > 1 && total > 4.0e6 ? NST : 1;
         double load[NST] = {};
-        PhaseTimer wall(c, PH_ERI);
+        // on one stream the classes' spans are the phase's
+        std::optional<PhaseTimer> wall;
         if (nst > 1) {
+            wall.emplace(c, PH_ERI);
             ZV_HIPCHECK(c, hipEventRecord(c->ev_fork, c->stream));
             for (int k = 0; k < zv_context::NSIDE; k++)
                 ZV_HIPCHECK(c, hipStreamWaitEvent(c->side[k], c->ev_fork, 0));
@@ -836,7 +857,7 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
             const int slot = LB * 6 + LK;
             c->cls_pq[slot] += bpq[b];
             c->cls_flops[slot] += bfl[b];
-            PhaseTimer tm(c, PH_N, slot, sts[s]);
+            PhaseTimer tm(c, nst > 1 ? PH_N : PH_ERI, slot, sts[s]);
             QSrc S{Q_LIST, dqb + lo[b], dqk + lo[b], lo[b + 1] - lo[b]};
             ZV_CHECK(launch_class_on(c, sts[s], pp, S, LB, LK, dout + lo[b], part + lp.poff[b],
                                      lp.ns[b]));
@@ -847,7 +868,7 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
                 ZV_HIPCHECK(c, hipStreamWaitEvent(c->stream, c->ev_join[k], 0));
             }
         if (npart) {
-            hipLaunchKernelGGL(k_reduce_list, dim3(nblk(nq, 256)), dim3(256), 0, c->stream, lp,
+            hipLaunchKernelGGL(k_reduce_list, dim3(nblk(nq, 4)), dim3(256), 0, c->stream, lp,
                                (const double *)part, dout);
             ZV_HIPCHECK(c, hipGetLastError());
         }
@@ -923,6 +944,7 @@ int zv_run_gauss_list_noalloc(zv_context *c, int64_t nq, const int *qi, const in
     static int h_qb[kNaQ], h_qk[kNaQ], h_pos[kNaQ];
     static unsigned char h_bk[kNaQ];
     int64_t lo[ncls * ncls + 1] = {};
+    int nbra[ncls * ncls] = {};
     auto order = [&](int P) {
         const int L = c->h_pair_L[P];
         return L > ZV_LMAX_T ? ZV_LMAX_T + 1 : L;
@@ -934,6 +956,7 @@ int zv_run_gauss_list_noalloc(zv_context *c, int64_t nq, const int *qi, const in
         if (order(P) < order(Q)) std::swap(P, Q);
         h_bk[t] = (unsigned char)(order(P) * ncls + order(Q));
         lo[h_bk[t] + 1]++;
+        nbra[h_bk[t]] = std::max(nbra[h_bk[t]], c->h_cnt[P]);
     }
     for (int b = 0; b < ncls * ncls; b++) lo[b + 1] += lo[b];
     {
@@ -961,7 +984,7 @@ int zv_run_gauss_list_noalloc(zv_context *c, int64_t nq, const int *qi, const in
     for (int b = 0; b < ncls * ncls; b++) {
         const int64_t cnt = lo[b + 1] - lo[b];
         if (!cnt) continue;
-        const int nsplit = class_split(cnt);
+        const int nsplit = class_split(cnt, nbra[b]);
         if (nsplit > 1 && (size_t)(cnt * nsplit) > kNaPart)
             return zv_fail(c, ZV_ERR_STATE, "split partials exceed the scratch");
         QSrc S{Q_LIST, dqb + lo[b], dqk + lo[b], cnt};

@@ -1267,22 +1267,26 @@ int zv_shell_run(zv_context *c, const PP &pp, const std::vector<std::pair<int, i
         if (pl.lo[b + 1] > pl.lo[b]) order[nb++] = b;
     std::sort(order, order + nb, [&](int x, int y) { return pl.flops[x] > pl.flops[y]; });
     double load[NST] = {};
+    // ZV_TUNE_ERI_STREAMS limits the streams (1: buckets one after another); a
+    // single bucket needs no fork
+    const int nst = nb == 1 ? 1
+                    : c->tune[ZV_TUNE_ERI_STREAMS] > 0
+                        ? (int)std::min<int64_t>(c->tune[ZV_TUNE_ERI_STREAMS], NST)
+                        : NST;
     // phase time: one span around the fork and join; the buckets' own spans
     // overlap and only go to their statistics slots
     PhaseTimer wall(c, PH_ERI);
-    ZV_HIPCHECK(c, hipEventRecord(c->ev_fork, c->stream));
-    for (int k = 0; k < zv_context::NSIDE; k++)
-        ZV_HIPCHECK(c, hipStreamWaitEvent(c->side[k], c->ev_fork, 0));
+    if (nst > 1) {
+        ZV_HIPCHECK(c, hipEventRecord(c->ev_fork, c->stream));
+        for (int k = 0; k < nst - 1; k++)
+            ZV_HIPCHECK(c, hipStreamWaitEvent(c->side[k], c->ev_fork, 0));
+    }
     for (int t = 0; t < nb; t++) {
         const int b = order[t];
         const int n = pl.lo[b + 1] - pl.lo[b];
         const int cls = 36 + b;
         c->cls_pq[cls] += pl.units[b];
         c->cls_flops[cls] += pl.flops[b];
-        // ZV_TUNE_ERI_STREAMS limits the streams (1: buckets one after another)
-        const int nst = c->tune[ZV_TUNE_ERI_STREAMS] > 0
-                            ? (int)std::min<int64_t>(c->tune[ZV_TUNE_ERI_STREAMS], NST)
-                            : NST;
         int s = 0;
         for (int q = 1; q < nst; q++)
             if (load[q] < load[s]) s = q;
@@ -1294,7 +1298,7 @@ int zv_shell_run(zv_context *c, const PP &pp, const std::vector<std::pair<int, i
                                 (double *)bpart.p, sts[s]});
         ZV_HIPCHECK(c, hipGetLastError());
     }
-    for (int k = 0; k < zv_context::NSIDE; k++) {
+    for (int k = 0; k < nst - 1; k++) {
         ZV_HIPCHECK(c, hipEventRecord(c->ev_join[k], c->side[k]));
         ZV_HIPCHECK(c, hipStreamWaitEvent(c->stream, c->ev_join[k], 0));
     }
