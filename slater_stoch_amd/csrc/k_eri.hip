@@ -50,36 +50,27 @@ struct BasisE {
     const int *npower, *itype, *ngauss;
 };
 
-// 1D Hermite coefficients E[a][b][t] (a <= A, b <= B), E[0][0][0] = 1.
-constexpr int kEA = 5, kET = 9; // per-axis power <= 4 (validated in zv_set_basis)
-__device__ void hermite_1d(double ip2, double xpa, double xpb, int A, int Bm,
-                           double (&E)[kEA][kEA][kET])
+// per-axis power <= 4 (validated in zv_set_basis), r^2 included, so the 1D
+// Hermite coefficients of a pair run over t <= 8
+constexpr int kET = 9;
+
+// One power more of (x - A): E'_t = x E_t + E_{t-1} / (2p) + (t+1) E_{t+1}
+__device__ inline void hermite_raise(double x, double ip2, double (&E)[kET])
 {
-    for (int a = 0; a <= A; a++)
-        for (int b = 0; b <= Bm; b++)
-            for (int t = 0; t < kET; t++) E[a][b][t] = 0.0;
-    E[0][0][0] = 1.0;
-    for (int a = 0; a <= A; a++) {
-        if (a > 0)
-            for (int t = 0; t <= a; t++) {
-                double v = xpa * E[a - 1][0][t];
-                if (t > 0) v += ip2 * E[a - 1][0][t - 1];
-                if (t + 1 <= a - 1) v += (t + 1) * E[a - 1][0][t + 1];
-                E[a][0][t] = v;
-            }
-        for (int b = 1; b <= Bm; b++)
-            for (int t = 0; t <= a + b; t++) {
-                double v = xpb * E[a][b - 1][t];
-                if (t > 0) v += ip2 * E[a][b - 1][t - 1];
-                if (t + 1 <= a + b - 1) v += (t + 1) * E[a][b - 1][t + 1];
-                E[a][b][t] = v;
-            }
+    double low = 0.0;
+#pragma unroll
+    for (int t = 0; t < kET; t++) {
+        const double v = E[t];
+        double r = x * v;
+        if (t > 0) r += ip2 * low;
+        if (t + 1 < kET) r += (t + 1) * E[t + 1];
+        low = v;
+        E[t] = r;
     }
 }
 
 // One wavefront per AO pair: all n_gauss(i) x n_gauss(k) primitive pairs,
-// cut as in the reference, compacted in order (ballot prefix), with their
-// Hermite coefficients summed over the r^2 variants of i_type 2 orbitals.
+// cut as in the reference, compacted in order (ballot prefix).
 __global__ __launch_bounds__(64) void k_primpairs(BasisE B, const int *pair_i, const int *pair_k,
                                                   PP pp)
 {
@@ -88,14 +79,11 @@ __global__ __launch_bounds__(64) void k_primpairs(BasisE B, const int *pair_i, c
     int i = pair_i[P] - 1, k = pair_k[P] - 1;
     int ngi = B.ngauss[i], ngk = B.ngauss[k];
     int cap = ngi * ngk;
-    int L = pp.L[P];
-    int H = hcount(L);
     const double *A = B.center + 3 * i, *Bc = B.center + 3 * k;
     int ti = B.itype[i], tk = B.itype[k];
-    const int *pa = B.npower + 3 * i, *pb = B.npower + 3 * k;
     const double *di = (ti == 1 ? B.c1 : B.c2) + (size_t)i * ZV_GMAX;
     const double *dk = (tk == 1 ? B.c1 : B.c2) + (size_t)k * ZV_GMAX;
-    int64_t off = pp.off[P], eoff = pp.eoff[P];
+    int64_t off = pp.off[P];
     int base = 0;
     for (int e0 = 0; e0 < cap; e0 += 64) {
         int e = e0 + lane;
@@ -136,35 +124,72 @@ __global__ __launch_bounds__(64) void k_primpairs(BasisE B, const int *pair_i, c
         pp.c[at] = coef;
         pp.al[at] = ea;
         pp.be[at] = eb;
-        // Hermite expansion, summed over the r^2 variants
-        double ip2 = 0.5 / p;
-        double E1[3][kEA][kEA][kET];
-        int Amax[3], Bmax[3];
-        for (int d = 0; d < 3; d++) {
-            Amax[d] = pa[d] + (ti == 2 ? 2 : 0);
-            Bmax[d] = pb[d] + (tk == 2 ? 2 : 0);
-            hermite_1d(ip2, Pc[d] - A[d], Pc[d] - Bc[d], Amax[d], Bmax[d], E1[d]);
-        }
-        double E3[165];
-        for (int h = 0; h < H; h++) E3[h] = 0.0;
-        int nvi = ti == 2 ? 3 : 1, nvk = tk == 2 ? 3 : 1;
-        for (int vi = 0; vi < nvi; vi++)
-            for (int vk = 0; vk < nvk; vk++) {
-                int ai[3], bk[3];
-                for (int d = 0; d < 3; d++) {
-                    ai[d] = pa[d] + ((ti == 2 && d == vi) ? 2 : 0);
-                    bk[d] = pb[d] + ((tk == 2 && d == vk) ? 2 : 0);
-                }
-                for (int t = 0; t <= ai[0] + bk[0]; t++)
-                    for (int u = 0; u <= ai[1] + bk[1]; u++)
-                        for (int v = 0; v <= ai[2] + bk[2]; v++)
-                            E3[hidx(t, u, v)] += E1[0][ai[0]][bk[0]][t] *
-                                                 E1[1][ai[1]][bk[1]][u] *
-                                                 E1[2][ai[2]][bk[2]][v];
-            }
-        for (int h = 0; h < H; h++) pp.E[eoff + (int64_t)h * cap + slot] = E3[h];
     }
     if (lane == 0) pp.cnt[P] = base;
+}
+
+// Hermite coefficients of the kept primitive pairs of one AO pair (a wavefront,
+// a lane per primitive pair), summed over the r^2 variants of i_type 2
+// orbitals.  Only the component kernels read them, so they are made when a list
+// or a pair of order above ZV_LMAX_T first asks.  The 1D recursion runs in
+// registers and the powers that the variants use (one per side, two where R2)
+// go to the lane's LDS column.  With whole [power][power][t] tables per lane in
+// scratch memory, inside k_primpairs, both took 739 us for the pairs of 110 AOs
+// and 335 us for 7; now 29 and 8 us without, 357 us with the coefficients.
+template <bool R2>
+__global__ __launch_bounds__(64) void k_pair_e(BasisE B, const int *pair_i, const int *pair_k,
+                                               PP pp)
+{
+    constexpr int NV = R2 ? 2 : 1;
+    __shared__ double E1[3][NV][NV][kET][64];
+    const int P = blockIdx.x, lane = threadIdx.x;
+    const int i = pair_i[P] - 1, k = pair_k[P] - 1;
+    const bool r2i = B.itype[i] == 2, r2k = B.itype[k] == 2;
+    if ((r2i || r2k) != R2) return;
+    const double *A = B.center + 3 * i, *C = B.center + 3 * k;
+    const int *pa = B.npower + 3 * i, *pb = B.npower + 3 * k;
+    const int nvi = r2i ? 3 : 1, nvk = r2k ? 3 : 1;
+    const int n = pp.cnt[P], cap = pp.cap[P], H = hcount(pp.L[P]);
+    const int64_t off = pp.off[P], eoff = pp.eoff[P];
+    for (int s = lane; s < n; s += 64) {
+        const double ip2 = 0.5 / pp.p[off + s];
+        const double Pc[3] = {pp.Px[off + s], pp.Py[off + s], pp.Pz[off + s]};
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const double xa = Pc[d] - A[d], xb = Pc[d] - C[d];
+            double ea[kET] = {1.0};
+            for (int a = 0;; a++) {
+                if (a == pa[d] || (r2i && a == pa[d] + 2)) {
+                    double eb[kET];
+#pragma unroll
+                    for (int t = 0; t < kET; t++) eb[t] = ea[t];
+                    for (int b = 0;; b++) {
+                        if (b == pb[d] || (r2k && b == pb[d] + 2)) {
+#pragma unroll
+                            for (int t = 0; t < kET; t++)
+                                E1[d][R2 && a > pa[d]][R2 && b > pb[d]][t][lane] = eb[t];
+                            if (!r2k || b > pb[d]) break;
+                        }
+                        hermite_raise(xb, ip2, eb);
+                    }
+                    if (!r2i || a > pa[d]) break;
+                }
+                hermite_raise(xa, ip2, ea);
+            }
+        }
+        for (int h = 0; h < H; h++) {
+            const int t = kH.t[h], u = kH.u[h], v = kH.v[h];
+            double sum = 0.0;
+            for (int vi = 0; vi < nvi; vi++)
+                for (int vk = 0; vk < nvk; vk++) {
+                    auto of = [&](int d, int x) {
+                        return E1[d][R2 && r2i && vi == d][R2 && r2k && vk == d][x][lane];
+                    };
+                    sum += of(0, t) * of(1, u) * of(2, v);
+                }
+            pp.E[eoff + (int64_t)h * cap + s] = sum;
+        }
+    }
 }
 
 // ------------------------------------------------------------------ classes
@@ -504,6 +529,22 @@ static int ensure_primpairs(zv_context *c, PP &pp)
     return ZV_OK;
 }
 
+// The Hermite coefficients for the component kernels (no allocation: b_ppE
+// comes with the pair tables).
+static int ensure_pair_e(zv_context *c, const PP &pp)
+{
+    if (c->ppE_ready) return ZV_OK;
+    BasisE B{c->d_center, c->d_c1, c->d_c2, c->d_g, c->d_npower, c->d_itype, c->d_ngauss};
+    PhaseTimer tm(c, PH_PRIM);
+    hipLaunchKernelGGL(k_pair_e<false>, dim3(c->npair), dim3(64), 0, c->stream, B, c->d_pair_i,
+                       c->d_pair_k, pp);
+    hipLaunchKernelGGL(k_pair_e<true>, dim3(c->npair), dim3(64), 0, c->stream, B, c->d_pair_i,
+                       c->d_pair_k, pp);
+    ZV_HIPCHECK(c, hipGetLastError());
+    c->ppE_ready = true;
+    return ZV_OK;
+}
+
 // FP64 flops per primitive quartet of the (LB, LK) component kernel: Boys
 // values (3 per order plus ~25 for erf/exp/sqrt/division), the Hermite R
 // recursion (2 FMA per entry over all levels), the ket-Hermite contraction
@@ -585,6 +626,7 @@ static int run_generic_pairs(zv_context *c, const PP &pp, const std::vector<int>
 {
     const int64_t nq = (int64_t)qb.size();
     if (!nq) return ZV_OK;
+    ZV_CHECK(ensure_pair_e(c, pp));
     double pq = 0.0, flops = 0.0;
     int nbra = 0;
     for (int64_t t = 0; t < nq; t++) {
@@ -763,6 +805,7 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
 {
     PP pp;
     ZV_CHECK(ensure_primpairs(c, pp));
+    ZV_CHECK(ensure_pair_e(c, pp));
     constexpr int ncls = ZV_LMAX_T + 2;
     auto order = [&](int P) {
         int L = c->h_pair_L[P];
@@ -940,6 +983,7 @@ int zv_run_gauss_list_noalloc(zv_context *c, int64_t nq, const int *qi, const in
                        "the primitive-pair tables of this basis are not built: call zv_gauss_eri "
                        "or zv_gauss_ijkl_list once after zv_set_basis");
     const PP pp = pp_view(c);
+    ZV_CHECK(ensure_pair_e(c, pp));
     constexpr int ncls = ZV_LMAX_T + 2;
     static int h_qb[kNaQ], h_qk[kNaQ], h_pos[kNaQ];
     static unsigned char h_bk[kNaQ];

@@ -388,7 +388,7 @@ static void free_basis(zv_context *c)
     c->d_pair_i = c->d_pair_k = nullptr;
     c->d_pair_f = c->d_pair_jf = c->d_pair_G = nullptr;
     c->d_kbase = nullptr;
-    c->pp_ready = false;
+    c->pp_ready = c->ppE_ready = false;
     c->sp_ready = false;
     c->grp_ready = false;
     for (bool &v : c->res_valid) v = false;

@@ -93,7 +93,7 @@ struct zv_context {
     DevBuf b_list;                     // class lists
     DevBuf b_part;                     // split partial sums
     DevBuf b_misc;
-    bool pp_ready = false;
+    bool pp_ready = false, ppE_ready = false; // pair tables; their E planes
     // shell-pair data
     DevBuf b_spmeta;                   // offsets, component tables (spd_of, k_eri_shell.hip)
     DevBuf b_spu, b_spe;               // primitive-pair rows; expansion tables of the components

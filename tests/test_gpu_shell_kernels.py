@@ -68,3 +68,22 @@ def test_list_classes_side_by_side(engine, nq, ng):
     np.testing.assert_array_equal(engine.gauss_ijkl(i, k, j, l), got)
     if nq <= 16384:
         np.testing.assert_array_equal(engine.gauss_ijkl_noalloc(i, k, j, l), got)
+
+
+def test_hermite_planes_on_first_use(engine):
+    """The component kernels' Hermite coefficients are made on first use: by
+    the allocation-free entry point after gauss_eri, by a list, and again for
+    a new basis, with the same values."""
+    geom = B.geometry_from_angstrom(["O", "H"], [[0.05, -0.1, 0.2], [0.7, 0.4, -0.5]])
+    basis = {"O": [("2S", 1.9), ("2P", 2.1), ("3P", 1.3)], "H": [("1S", 1.2), ("3D", 1.4)]}
+    bas = B.expand_basis(geom, basis, ng0=3)
+    rng = np.random.default_rng(3)
+    q = rng.integers(1, bas.n + 1, (4, 300))
+    engine.set_basis(bas)
+    engine.gauss_eri()
+    first = engine.gauss_ijkl_noalloc(*q)
+    engine.set_basis(B.expand_basis(geom, basis, ng0=2))
+    other = engine.gauss_ijkl(*q)
+    engine.set_basis(bas)
+    np.testing.assert_array_equal(engine.gauss_ijkl(*q), first)
+    assert np.abs(other - first).max() > 1e-6
