@@ -191,6 +191,20 @@ def roofline_eri(res):
             "heaviest_kernel_flop_share": heavy[1]["flops"] / flops}
 
 
+def mfma_fraction(res):
+    """Share of the analytic phase's counted flops that are row sums on the
+    matrix units: everything beyond the Boys values and the R table in the
+    classes whose uniform side is above order 0."""
+    st = res["eri_stats"]
+    on = 0.0
+    for key, v in st.items():
+        if key[0] == "shell" and key[1] > 0:
+            l = key[1] + key[2]
+            r = (l + 1) * (l + 2) * (l + 3) * (l + 4) / 24.0
+            on += v["flops"] - v["units"] * (25.0 + 3.0 * (l + 1) + 4.0 * (r - 1.0) + 12.0)
+    return on / sum(v["flops"] for v in st.values())
+
+
 def mfma_eligibility(bas):
     """Why the estimator stays on the vector unit, measured on this basis:
     the per-shell-pair-pair products that matrix cores would run
@@ -527,7 +541,7 @@ def main():
         "n_screened": int(last["n_screened"]),
         "host_copy_s": float(np.mean([r["host_copy"] for r in res64])),
         "with_host_copy_s": float(np.mean([r["total"] + r["host_copy"] for r in res64])),
-        "mfma_fraction": 0.0,
+        "mfma_fraction": mfma_fraction(last),
         "mfma_eligibility": mfma_eligibility(bas),
         "roofline": roofline_eri(last),
         "roofline_other_phase": roofline_estimator(last["pilot_timings"], bas, "fp64",

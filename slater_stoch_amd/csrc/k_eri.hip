@@ -529,13 +529,12 @@ static int ensure_primpairs(zv_context *c, PP &pp)
     return ZV_OK;
 }
 
-// The Hermite coefficients for the component kernels (no allocation: b_ppE
-// comes with the pair tables).
-static int ensure_pair_e(zv_context *c, const PP &pp)
+// The Hermite coefficients for the component kernels: no allocation (b_ppE
+// comes with the pair tables), no timing.
+static int pair_e_raw(zv_context *c, const PP &pp)
 {
     if (c->ppE_ready) return ZV_OK;
     BasisE B{c->d_center, c->d_c1, c->d_c2, c->d_g, c->d_npower, c->d_itype, c->d_ngauss};
-    PhaseTimer tm(c, PH_PRIM);
     hipLaunchKernelGGL(k_pair_e<false>, dim3(c->npair), dim3(64), 0, c->stream, B, c->d_pair_i,
                        c->d_pair_k, pp);
     hipLaunchKernelGGL(k_pair_e<true>, dim3(c->npair), dim3(64), 0, c->stream, B, c->d_pair_i,
@@ -543,6 +542,13 @@ static int ensure_pair_e(zv_context *c, const PP &pp)
     ZV_HIPCHECK(c, hipGetLastError());
     c->ppE_ready = true;
     return ZV_OK;
+}
+
+static int ensure_pair_e(zv_context *c, const PP &pp)
+{
+    if (c->ppE_ready) return ZV_OK;
+    PhaseTimer tm(c, PH_PRIM);
+    return pair_e_raw(c, pp);
 }
 
 // FP64 flops per primitive quartet of the (LB, LK) component kernel: Boys
@@ -983,7 +989,7 @@ int zv_run_gauss_list_noalloc(zv_context *c, int64_t nq, const int *qi, const in
                        "the primitive-pair tables of this basis are not built: call zv_gauss_eri "
                        "or zv_gauss_ijkl_list once after zv_set_basis");
     const PP pp = pp_view(c);
-    ZV_CHECK(ensure_pair_e(c, pp));
+    ZV_CHECK(pair_e_raw(c, pp));
     constexpr int ncls = ZV_LMAX_T + 2;
     static int h_qb[kNaQ], h_qk[kNaQ], h_pos[kNaQ];
     static unsigned char h_bk[kNaQ];
