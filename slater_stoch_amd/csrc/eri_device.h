@@ -52,51 +52,7 @@ struct PP {
 };
 
 // ------------------------------------------------------------------ Boys
-// F_n(T) = int_0^1 t^2n exp(-T t^2) dt for n = 0..L, as src/rint_sum.F90:
-// T < 1: Taylor series of F_L (20 terms) and downward recursion;
-// T >= 1: F_0 from erf and upward recursion, exp(-T) = 0 beyond T = 80.
-// From T = 36 on erf(sqrt T) = 1 - erfc(6) rounds to 1.0 (erfc(6) = 2.2e-17
-// is below half an ulp of 1), so the call is skipped there: same value,
-// and a wave whose lanes all have T >= 36 (distant pairs) skips the erf.
-template <int L> struct BoysCoef {
-    double c[20];
-    constexpr BoysCoef() : c()
-    {
-        double f = 1.0;
-        for (int k = 0; k < 20; k++) {
-            if (k > 0) f = f * k;
-            c[k] = ((k & 1) ? -1.0 : 1.0) / (f * (2 * L + 2 * k + 1));
-        }
-    }
-};
-
-template <int L> __device__ inline void boys(double T, double *F)
-{
-    if (T < 1.0) {
-        constexpr BoysCoef<L> bc{};
-        double s = bc.c[19];
-#pragma unroll
-        for (int k = 18; k >= 0; k--) s = fma(s, T, bc.c[k]);
-        F[L] = s;
-        if (L > 0) {
-            double e = exp(-T);
-#pragma unroll
-            for (int m = L - 1; m >= 0; m--) F[m] = (2.0 * T * F[m + 1] + e) * (1.0 / (2 * m + 1));
-        }
-    } else {
-        double u_inv = rsqrt(T);
-        double u = T * u_inv;
-        double ef = 1.0;
-        if (T < 36.0) ef = erf(u);
-        F[0] = ((0.5 * u_inv) * kSqrtPi) * ef;
-        if (L > 0) {
-            double e = T > 80.0 ? 0.0 : exp(-T);
-            double tri = (0.5 * u_inv) * u_inv;
-#pragma unroll
-            for (int m = 0; m < L; m++) F[m + 1] = (F[m] * (2 * m + 1) - e) * tri;
-        }
-    }
-}
+// F_n(T) = int_0^1 t^2n exp(-T t^2) dt for n = 0..L
 
 // Tabulated Boys function: polynomials in d = T - T_i about the nearest grid
 // point T_i = i h, |d| <= h/2.  The Taylor series
@@ -196,7 +152,9 @@ template <int L> __device__ inline void boys_table(double T, const double *lt, d
     }
 }
 
-// generic-L version (runtime loop)
+// Runtime order, as src/rint_sum.F90: T < 1: Taylor series of F_L and downward
+// recursion; T >= 1: F_0 from erf and upward recursion, exp(-T) = 0 beyond
+// T = 80.
 __device__ inline void boys_rt(int L, double T, double *F)
 {
     if (T < 1.0) {

@@ -20,8 +20,8 @@
 // the kept primitive pairs.  Primitive pairs whose Gaussian-product factor is
 // cut by the reference (exponent > 40, src/gaussian_product.F90:25, or factor
 // < 1e-15, src/give_explicit_poly_and_gaussian.F90:46) are dropped the same
-// way.  The Boys values follow src/rint_sum.F90: series for T < 1, erf plus
-// upward recursion for T >= 1.
+// way.  The Boys values come from the tabulated expansions (eri_device.h); at
+// run-time orders as in src/rint_sum.F90.
 //
 // Work layout: quartets are grouped by the Hermite orders (LB, LK) of their
 // two pairs (LB >= LK) and each class runs a kernel templated on (LB, LK) so
