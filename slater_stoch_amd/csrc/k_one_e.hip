@@ -21,7 +21,8 @@
 // run k_one_e with run-time orders, whose tables live in scratch memory.
 // Bound: FP64 issue (Boys and R per primitive pair and nucleus).  110-AO
 // random molecule, 12 nuclei: 15.3 ms with every pair on the run-time kernel,
-// 0.49 ms with the five register kernels.
+// 0.49 ms with the five register kernels one after another, 0.40 ms side by
+// side.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -372,16 +373,36 @@ int zv_run_one_e(zv_context *c, int nnuc, const double *charge, const double *nu
                c->d_ngauss, n, ZV_GMAX, nnuc, dq, dnuc, dS, dV, dK};
     {
         PhaseTimer tm(c, PH_ERI);
-        // the highest orders, whose workgroups run longest, first
+        // The orders write disjoint pairs, so from 256 pairs on they run side by
+        // side on the context's stream and its side streams, whose other orders
+        // fill the CUs that one order's last workgroups leave idle (whole call:
+        // 325 pairs 250 -> 205 us, 6105 pairs 563 -> 474 us; below, the fork and
+        // join cost more: 55 pairs 148 -> 158 us).  The run-time kernel stays on
+        // the context's stream, whose scratch memory it needs.  The longest
+        // launches come first.
+        static_assert(zv_context::NSIDE >= 4, "a stream per order");
+        const bool fork = pairs.size() >= 256;
+        hipStream_t sts[ZV_LMAX_T + 1];
+        for (int L = 0; L <= ZV_LMAX_T; L++)
+            sts[L] = fork && L != 3 ? c->side[L < 3 ? L : 3] : c->stream;
+        if (fork) {
+            ZV_HIPCHECK(c, hipEventRecord(c->ev_fork, c->stream));
+            for (int k = 0; k < 4; k++) ZV_HIPCHECK(c, hipStreamWaitEvent(c->side[k], c->ev_fork, 0));
+        }
         if (lo[ZV_LMAX_T + 2] > lo[ZV_LMAX_T + 1])
             hipLaunchKernelGGL(k_one_e, dim3((unsigned)(lo[ZV_LMAX_T + 2] - lo[ZV_LMAX_T + 1])),
                                dim3(256), 0, c->stream, a, (const int2 *)dp + lo[ZV_LMAX_T + 1]);
-        launch_pair<4>(a, dp + lo[4], lo[5] - lo[4], btab, c->stream);
-        launch_pair<3>(a, dp + lo[3], lo[4] - lo[3], btab, c->stream);
-        launch_pair<2>(a, dp + lo[2], lo[3] - lo[2], btab, c->stream);
-        launch_pair<1>(a, dp + lo[1], lo[2] - lo[1], btab, c->stream);
-        launch_pair<0>(a, dp + lo[0], lo[1] - lo[0], btab, c->stream);
+        launch_pair<3>(a, dp + lo[3], lo[4] - lo[3], btab, sts[3]);
+        launch_pair<4>(a, dp + lo[4], lo[5] - lo[4], btab, sts[4]);
+        launch_pair<2>(a, dp + lo[2], lo[3] - lo[2], btab, sts[2]);
+        launch_pair<1>(a, dp + lo[1], lo[2] - lo[1], btab, sts[1]);
+        launch_pair<0>(a, dp + lo[0], lo[1] - lo[0], btab, sts[0]);
         ZV_HIPCHECK(c, hipGetLastError());
+        if (fork)
+            for (int k = 0; k < 4; k++) {
+                ZV_HIPCHECK(c, hipEventRecord(c->ev_join[k], c->side[k]));
+                ZV_HIPCHECK(c, hipStreamWaitEvent(c->stream, c->ev_join[k], 0));
+            }
     }
     ZV_HIPCHECK(c, hipMemcpyAsync(S, dS, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
     ZV_HIPCHECK(c, hipMemcpyAsync(V, dV, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
