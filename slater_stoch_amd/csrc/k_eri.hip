@@ -132,23 +132,23 @@ __global__ __launch_bounds__(64) void k_primpairs(BasisE B, const int *pair_i, c
 // a lane per primitive pair), summed over the r^2 variants of i_type 2
 // orbitals.  Only the component kernels read them, so they are made when a list
 // or a pair of order above ZV_LMAX_T first asks.  The 1D recursion runs in
-// registers and the powers that the variants use (one per side, two where R2)
+// registers and the powers that the variants use (one per side, two where r^2)
 // go to the lane's LDS column.  With whole [power][power][t] tables per lane in
 // scratch memory, inside k_primpairs, both took 739 us for the pairs of 110 AOs
-// and 335 us for 7; now 29 and 8 us without, 357 us with the coefficients.
-template <bool R2>
+// and 335 us for 7; now 29 and 8 us without, 204 us with the coefficients (the
+// variants unrolled over twelve values in registers; looped, 357 us).
+template <bool R2I, bool R2K>
 __global__ __launch_bounds__(64) void k_pair_e(BasisE B, const int *pair_i, const int *pair_k,
                                                PP pp)
 {
-    constexpr int NV = R2 ? 2 : 1;
-    __shared__ double E1[3][NV][NV][kET][64];
+    constexpr int PI = R2I ? 2 : 1, PK = R2K ? 2 : 1; // powers per side
+    __shared__ double E1[3][PI][PK][kET][64];
     const int P = blockIdx.x, lane = threadIdx.x;
     const int i = pair_i[P] - 1, k = pair_k[P] - 1;
-    const bool r2i = B.itype[i] == 2, r2k = B.itype[k] == 2;
-    if ((r2i || r2k) != R2) return;
+    if ((B.itype[i] == 2) != R2I || (B.itype[k] == 2) != R2K) return;
     const double *A = B.center + 3 * i, *C = B.center + 3 * k;
     const int *pa = B.npower + 3 * i, *pb = B.npower + 3 * k;
-    const int nvi = r2i ? 3 : 1, nvk = r2k ? 3 : 1;
+    constexpr int NVI = R2I ? 3 : 1, NVK = R2K ? 3 : 1; // r^2 = x^2 + y^2 + z^2
     const int n = pp.cnt[P], cap = pp.cap[P], H = hcount(pp.L[P]);
     const int64_t off = pp.off[P], eoff = pp.eoff[P];
     for (int s = lane; s < n; s += 64) {
@@ -159,34 +159,42 @@ __global__ __launch_bounds__(64) void k_pair_e(BasisE B, const int *pair_i, cons
             const double xa = Pc[d] - A[d], xb = Pc[d] - C[d];
             double ea[kET] = {1.0};
             for (int a = 0;; a++) {
-                if (a == pa[d] || (r2i && a == pa[d] + 2)) {
+                if (a == pa[d] || (R2I && a == pa[d] + 2)) {
                     double eb[kET];
 #pragma unroll
                     for (int t = 0; t < kET; t++) eb[t] = ea[t];
                     for (int b = 0;; b++) {
-                        if (b == pb[d] || (r2k && b == pb[d] + 2)) {
+                        if (b == pb[d] || (R2K && b == pb[d] + 2)) {
 #pragma unroll
                             for (int t = 0; t < kET; t++)
-                                E1[d][R2 && a > pa[d]][R2 && b > pb[d]][t][lane] = eb[t];
-                            if (!r2k || b > pb[d]) break;
+                                E1[d][R2I && a > pa[d]][R2K && b > pb[d]][t][lane] = eb[t];
+                            if (!R2K || b > pb[d]) break;
                         }
                         hermite_raise(xb, ip2, eb);
                     }
-                    if (!r2i || a > pa[d]) break;
+                    if (!R2I || a > pa[d]) break;
                 }
                 hermite_raise(xa, ip2, ea);
             }
         }
         for (int h = 0; h < H; h++) {
             const int t = kH.t[h], u = kH.u[h], v = kH.v[h];
+            const int x[3] = {t, u, v};
+            double e[3][PI][PK];
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+                for (int a = 0; a < PI; a++)
+#pragma unroll
+                    for (int b = 0; b < PK; b++) e[d][a][b] = E1[d][a][b][x[d]][lane];
             double sum = 0.0;
-            for (int vi = 0; vi < nvi; vi++)
-                for (int vk = 0; vk < nvk; vk++) {
-                    auto of = [&](int d, int x) {
-                        return E1[d][R2 && r2i && vi == d][R2 && r2k && vk == d][x][lane];
-                    };
-                    sum += of(0, t) * of(1, u) * of(2, v);
-                }
+#pragma unroll
+            for (int vi = 0; vi < NVI; vi++)
+#pragma unroll
+                for (int vk = 0; vk < NVK; vk++)
+                    sum += e[0][R2I && vi == 0][R2K && vk == 0] *
+                           e[1][R2I && vi == 1][R2K && vk == 1] *
+                           e[2][R2I && vi == 2][R2K && vk == 2];
             pp.E[eoff + (int64_t)h * cap + s] = sum;
         }
     }
@@ -535,10 +543,11 @@ static int pair_e_raw(zv_context *c, const PP &pp)
 {
     if (c->ppE_ready) return ZV_OK;
     BasisE B{c->d_center, c->d_c1, c->d_c2, c->d_g, c->d_npower, c->d_itype, c->d_ngauss};
-    hipLaunchKernelGGL(k_pair_e<false>, dim3(c->npair), dim3(64), 0, c->stream, B, c->d_pair_i,
-                       c->d_pair_k, pp);
-    hipLaunchKernelGGL(k_pair_e<true>, dim3(c->npair), dim3(64), 0, c->stream, B, c->d_pair_i,
-                       c->d_pair_k, pp);
+    // a pair is done by the launch of its types, the others pass over it
+    for (auto kern : {k_pair_e<false, false>, k_pair_e<true, false>, k_pair_e<false, true>,
+                      k_pair_e<true, true>})
+        hipLaunchKernelGGL(kern, dim3(c->npair), dim3(64), 0, c->stream, B, c->d_pair_i,
+                           c->d_pair_k, pp);
     ZV_HIPCHECK(c, hipGetLastError());
     c->ppE_ready = true;
     return ZV_OK;
