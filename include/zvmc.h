@@ -141,7 +141,9 @@ int zv_gauss_ijkl_list_noalloc(zv_context *ctx, int64_t nq, const int *qi, const
  * mean(kcp) = block average of e_S - e_G, err(kcp) = the reference's
  * standard error sqrt|<x^2>-<x>^2|/sqrt(nbl), optional block_means(kcp,nbl)
  * (may be NULL).  A NULL mean or err keeps that array on the device only
- * (zv_get_result). */
+ * (zv_get_result).  The order in which a block's samples are added (rounding
+ * only) follows from the basis, nbl, npts, the precision and the tuning keys
+ * below; progress lines and block_means leave every bit alone. */
 int zv_mc_blocks(zv_context *ctx, int nbl, int64_t npts, int mode, uint64_t seed,
                  uint64_t stream, int precision, const double *r1, const double *r2,
                  const double *pi0, double *mean, double *err, double *block_means);
@@ -255,8 +257,10 @@ int zv_davidson_lowest(zv_context *ctx, int nev, double tol, int max_iter, int p
  * prints what the reference prints unconditionally in svd_clean ("Vectors
  * a -- b / N" per randomized pass, src/svd_clean.F90:153-154, and the
  * largest/smallest singular value of the pass, :285); level 2 adds one line
- * per finished zv_mc_blocks block (the call then waits for each block, so
- * the line reports work done); level 0 (the default) prints nothing.  From
+ * per finished zv_mc_blocks block (the call then waits for each round of
+ * blocks that runs together, so the lines report work done; a block too
+ * long for that is a round of its own); level 0 (the default) prints
+ * nothing.  From
  * level 1 on, zv_gauss_eri also writes the host time of its Schwarz
  * phases' planning to stderr (lines starting "[zvmc]").  No counterpart
  * in the reference, whose prints cannot be switched off. */

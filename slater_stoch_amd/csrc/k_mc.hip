@@ -827,7 +827,7 @@ __global__ void k_scatter_ref(int64_t ntri, const double *__restrict__ in, doubl
 // nsplit rows (in split order), x = sum / npts.  s1, s2 carry the sums of x
 // and x^2 between calls (first: none yet); the last call writes the mean and
 // the standard error (k_final_stats) to their reference positions.  blk (may
-// be null, nb = 1): the block's x.
+// be null): the x of block b at blk[b ntri + t].
 __global__ void k_block_rows(int64_t ntri, double f, const double *__restrict__ rows, int nb,
                              int nsplit, bool first, bool last, int nbl, double *s1, double *s2,
                              double *blk, double *mean, double *err, const int *pi, const int *pk,
@@ -843,7 +843,7 @@ __global__ void k_block_rows(int64_t ntri, double f, const double *__restrict__ 
         const double x = e * f;
         a1 += x;
         a2 += x * x;
-        if (blk) blk[t] = x;
+        if (blk) blk[(size_t)b * ntri + t] = x;
     }
     if (!last) {
         s1[t] = a1;
@@ -1050,6 +1050,9 @@ static int pick_chunk(zv_context *c, int64_t npts, int precision)
 // estimator launches and one statistics launch, so small molecules pay their
 // launches once instead of per block (10 AOs, 10 x 1000 samples FP32: 2.34 ms
 // block by block) and large ones their last, partly empty wave of tiles.
+// The count also sets the sample splits (pick_split) and so the order of the
+// sums: progress lines and block means take the blocks of a round as they
+// are, so that asking for either leaves every bit of the results alone.
 static int pick_blocks(zv_context *c, int nbl, int64_t npts, int64_t chunk)
 {
     const int64_t rows = std::max<int64_t>(1, ((int64_t)1 << 28) / std::max<int64_t>(1, c->nint));
@@ -1266,8 +1269,8 @@ static int run_group_estimator(zv_context *c, const T *comp, const T *grp, Group
     return ZV_OK;
 }
 
-// samples of blocks [b, b + nb) at offset m0 of each (nb > 1: m0 = 0) into
-// the chunk's sample buffers
+// samples g0 .. g0 + M - 1 of the call (block b starts at b npts) into the
+// chunk's sample buffers
 static int fill_samples(zv_context *c, int mode, uint64_t seed, uint64_t stream, uint64_t g0, int M,
                         const double *r1, const double *r2, const double *pi0)
 {
@@ -1382,7 +1385,7 @@ static int run_group_chunk(zv_context *c, int Mv, const GroupSpan &span, double 
 // The group estimator: the mean and the standard error go to the result
 // buffers in reference order.  Rounds of nb blocks when a block fits in a
 // chunk; otherwise block by block, the chunks of a block added up in its
-// rows.  Block means and the per-block progress lines take one block a round.
+// rows.  The per-block progress lines are printed when their round is done.
 static int run_mc_group(zv_context *c, int nbl, int64_t npts, int mode, uint64_t seed,
                         uint64_t stream, int precision, const double *r1, const double *r2,
                         const double *pi0, double *block_means)
@@ -1391,8 +1394,7 @@ static int run_mc_group(zv_context *c, int nbl, int64_t npts, int mode, uint64_t
     ZV_CHECK(group_ready(c));
     const bool single = precision != ZV_PREC_FP64;
     const int cap = pick_chunk(c, (int64_t)nbl * npts, precision);
-    int nb = cap >= npts ? pick_blocks(c, nbl, npts, cap) : 1;
-    if (block_means || c->verbose >= 2) nb = 1;
+    const int nb = cap >= npts ? pick_blocks(c, nbl, npts, cap) : 1;
     const int Mc = cap >= npts ? (int)(nb * npts) : cap;
     const size_t fields = (size_t)Mc * (4 * (size_t)c->npair + 6 * (size_t)c->nsp);
     ZV_CHECK(zv_ensure(c, c->b_r1, sizeof(double) * 3 * Mc));
@@ -1409,7 +1411,7 @@ static int run_mc_group(zv_context *c, int nbl, int64_t npts, int mode, uint64_t
         ZV_CHECK(zv_ensure(c, c->b_s1, sizeof(double) * ntri));
         ZV_CHECK(zv_ensure(c, c->b_s2, sizeof(double) * ntri));
     }
-    if (block_means) ZV_CHECK(zv_ensure(c, c->b_blk, sizeof(double) * ntri));
+    if (block_means) ZV_CHECK(zv_ensure(c, c->b_blk, sizeof(double) * nb * ntri));
     for (int which : {ZV_RESULT_MEAN, ZV_RESULT_STDERR}) {
         c->res_valid[which] = false;
         ZV_CHECK(zv_ensure(c, c->b_res[which], sizeof(double) * ntri));
@@ -1441,12 +1443,12 @@ static int run_mc_group(zv_context *c, int nbl, int64_t npts, int mode, uint64_t
                                c->d_kbase, c->n);
             ZV_HIPCHECK(c, hipGetLastError());
         }
-        if (block_means)
-            ZV_CHECK(zv_run_scatter_ref(c, (const double *)c->b_blk.p,
-                                        block_means + (size_t)b * ntri));
+        for (int k = 0; block_means && k < bn; k++)
+            ZV_CHECK(zv_run_scatter_ref(c, (const double *)c->b_blk.p + (size_t)k * ntri,
+                                        block_means + (size_t)(b + k) * ntri));
         if (c->verbose >= 2) {
             ZV_HIPCHECK(c, hipStreamSynchronize(c->stream));
-            block_line(c, b, nbl, npts);
+            for (int k = 0; k < bn; k++) block_line(c, b + k, nbl, npts);
         }
     }
     return ZV_OK;
