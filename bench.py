@@ -191,17 +191,47 @@ def roofline_eri(res):
             "heaviest_kernel_flop_share": heavy[1]["flops"] / flops}
 
 
+def quartet_macs(lu, ll, p):
+    """(matrix, vector) multiply-adds per primitive quartet of the row sums of
+    k_eri_quartet<lu, ll, p>, by the kernel's own rule (make_slots): a row of
+    order rho needs the scaled Hermite weights sigma with n >= rho - ll, and
+    each of the pass's groups of four of them is one matrix instruction, or a
+    plain vector multiply-add where a single sigma is needed."""
+    if lu == 4:
+        rho0, rho1, g0, g1 = ((0, 5, 0, 1), (0, 5, 1, 4), (6, 7, 0, 4), (8, 8, 0, 1))[p]
+    elif (lu, ll) == (3, 4):
+        rho0, rho1, g0, g1 = ((0, 7, 0, 1), (0, 5, 1, 3))[p]
+    else:
+        rho0, rho1, g0, g1 = 0, lu + ll, 0, ((lu + 1) * (lu + 2) // 2 + 3) // 4
+    matrix = vector = 0
+    for rho in range(rho0, rho1 + 1):
+        rows = (rho + 1) * (rho + 2) // 2
+        nmin = max(0, rho - ll)
+        need = (lu - nmin + 1) * (lu - nmin + 2) // 2
+        for g in range(g0, g1):
+            left = need - 4 * g
+            if left == 1:
+                vector += rows
+            elif left > 1:
+                matrix += rows * min(4, left)
+    return matrix, vector
+
+
+def boys_r_flops(l):
+    """Counted flops of the Boys values, the R table and the prefactor of one
+    primitive quartet of total order l."""
+    return 25.0 + 3.0 * (l + 1) + 4.0 * (math.comb(l + 4, 4) - 1.0) + 12.0
+
+
 def mfma_fraction(res):
-    """Share of the analytic phase's counted flops that are row sums on the
-    matrix units: everything beyond the Boys values and the R table in the
-    classes whose uniform side is above order 0."""
+    """Share of the analytic phase's counted flops that run on the matrix
+    units: the row sums of more than one scaled Hermite weight."""
     st = res["eri_stats"]
     on = 0.0
     for key, v in st.items():
-        if key[0] == "shell" and key[1] > 0:
-            l = key[1] + key[2]
-            r = (l + 1) * (l + 2) * (l + 3) * (l + 4) / 24.0
-            on += v["flops"] - v["units"] * (25.0 + 3.0 * (l + 1) + 4.0 * (r - 1.0) + 12.0)
+        if key[0] == "shell":
+            m, x = quartet_macs(key[1], key[2], key[3] - 1)
+            on += (v["flops"] - v["units"] * boys_r_flops(key[1] + key[2])) * m / (m + x)
     return on / sum(v["flops"] for v in st.values())
 
 
@@ -270,7 +300,7 @@ def eri_by_class(res):
             a[f] += d[f]
     total = sum(a["flops"] for a in agg.values()) or 1.0
     return [{"class": list(k), "flops": a["flops"], "flop_share": a["flops"] / total,
-             "prim_quartet_components": a["units"]}
+             "prim_quartets": a["units"]}
             for k, a in sorted(agg.items(), key=lambda kv: -kv[1]["flops"])]
 
 
