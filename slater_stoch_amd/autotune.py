@@ -12,7 +12,7 @@ size spends):
   small molecules)
 * ZV_TUNE_EST_SPLIT  sample splits per estimator tile (0 = automatic)
 * ZV_TUNE_MC_CHUNK   samples per estimator chunk (0 = automatic)
-* ZV_TUNE_ERI_ITEMS  work items per analytic Schwarz phase (0 = 40,000)
+* ZV_TUNE_ERI_ITEMS  work items per analytic Schwarz phase (0 = 20,000)
 
 A batch of molecules of uneven sizes is tuned per size class (by number of
 basis functions): the largest molecule of each class is tuned and its
@@ -32,7 +32,8 @@ KNOBS = {
     Z.TUNE_EST_TILES: [0, 1],
     Z.TUNE_EST_SPLIT: [0, 1, 2, 4, 8, 16, 32],
     Z.TUNE_MC_CHUNK: [0, 1600, 4000],
-    Z.TUNE_ERI_ITEMS: [0, 10000, 20000, 80000],
+    # 20000 repeats the automatic choice; its trial shows the noise of a timing
+    Z.TUNE_ERI_ITEMS: [0, 10000, 20000, 40000, 80000],
 }
 NAMES = {Z.TUNE_EST_TILES: "est_tiles", Z.TUNE_EST_SPLIT: "est_split",
          Z.TUNE_MC_CHUNK: "mc_chunk", Z.TUNE_ERI_ITEMS: "eri_items"}

@@ -75,3 +75,17 @@ def test_settings_for_falls_back_to_the_nearest_tuned_class():
     assert AT.settings_for(t, Bas(10))[Z.TUNE_EST_SPLIT] == 8       # below every tuned class
     assert AT.settings_for(t, Bas(200))[Z.TUNE_EST_SPLIT] == 2
     assert set(AT.settings_for(t, Bas(30))) == set(AT.KNOBS)
+
+
+def test_analytic_items_twice_the_default_are_tried():
+    """0 is the library's own 20000 items; an engine that is fastest with
+    twice as many is tuned to them."""
+    eng = FakeEngine()
+
+    def gauss_eri(device_only=False):
+        items = eng.knob[Z.TUNE_ERI_ITEMS] or 20000
+        eng._an = 10 + abs(items - 40000) / 1000
+
+    eng.gauss_eri = gauss_eri
+    best, _ = AT.tune(eng, Bas(50), npts=800, reps=1)
+    assert best[Z.TUNE_ERI_ITEMS] == 40000
