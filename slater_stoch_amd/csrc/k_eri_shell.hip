@@ -1087,64 +1087,11 @@ static SPD spd_of(zv_context *c)
                g + c->sp_g_total};
 }
 
-// The Boys tables of boys_table (eri_device.h), computed once per process in
-// extended precision (x87 long double on the host).
-// F_m(T) = exp(-T) sum_j (2T)^j / ((2m+1)(2m+3)...(2m+2j+1)), all terms
-// positive, summed until they fall below 1e-22 of the sum, for the highest m;
-// the others by the stable downward recursion.
-static const std::vector<double> &boys_table_host()
-{
-    static std::vector<double> tab;
-    if (!tab.empty()) return tab;
-    typedef long double LD;
-    constexpr int M = kBoysM, NM = kBoysLmax + M;
-    // Chebyshev polynomials T_k in powers of x
-    LD ch[M + 1][M + 1] = {};
-    ch[0][0] = ch[1][1] = 1.0L;
-    for (int k = 2; k <= M; k++)
-        for (int j = 0; j <= k; j++)
-            ch[k][j] = (j ? 2.0L * ch[k - 1][j - 1] : 0.0L) - ch[k - 2][j];
-    std::vector<double> t((size_t)boys_off(kBoysLmax + 1));
-    for (int L = 0; L <= kBoysLmax; L++)
-        for (int i = 0; i < boys_cols(L); i++) {
-            const LD T = (LD)i / boys_inv_h(L), delta = 0.5L / boys_inv_h(L), ex = expl(-T);
-            LD F[NM + 1], term = 1.0L / (2 * NM + 1), sum = term;
-            for (int j = 1; j < 2000; j++) {
-                term *= 2.0L * T / (2 * NM + 2 * j + 1);
-                sum += term;
-                if (term < 1e-22L * sum) break;
-            }
-            F[NM] = sum * ex;
-            for (int m = NM - 1; m >= 0; m--) F[m] = (2.0L * T * F[m + 1] + ex) / (2 * m + 1);
-            // q in powers of x = d / delta
-            const int D = boys_deg(L);
-            LD q[M + 1], s = 1.0L;
-            for (int k = 0; k <= M; k++) {
-                q[k] = F[L + k] * s;
-                s *= -delta / (k + 1);
-            }
-            for (int k = M; k > D; k--) {
-                const LD a = q[k] / ch[k][k];
-                for (int j = 0; j <= k; j++) q[j] -= a * ch[k][j];
-            }
-            double *o = t.data() + boys_off(L) + (size_t)i * boys_rows(L);
-            if (boys_pair(L)) o[0] = (double)F[L - 1];
-            s = 1.0L;
-            for (int k = 0; k <= D; k++) {
-                const LD v = q[k] * s;
-                s /= delta;
-                if (boys_pair(L)) o[k + 1] = (double)(-v / (k + 1));
-                else o[k] = (double)v;
-            }
-        }
-    tab.swap(t);
-    return tab;
-}
-
-// the table on the context's device (once per context)
+// the Boys tables, made once per process, on the context's device (once per
+// context)
 int zv_boys_table(zv_context *c, const double **tab)
 {
-    const std::vector<double> &t = boys_table_host();
+    static const std::vector<double> t = boys_table_host();
     ZV_CHECK(zv_ensure(c, c->b_btab, sizeof(double) * t.size()));
     *tab = (const double *)c->b_btab.p;
     if (c->btab_ready) return ZV_OK;
