@@ -388,12 +388,15 @@ __global__ __launch_bounds__(256) void k_reduce_parts(QSrc S, int nsplit, const 
     if (lane == 0) out[oidx] = s;
 }
 
-// the same over the classes of one list: class b holds list entries
-// lo[b] .. lo[b+1] - 1 and its partial sums start at poff[b] (ns[b] each; none
-// where ns[b] = 1)
+// the same over the split classes of one list, at most class_split's 16384
+// quartets each: of them all, class b holds numbers lo[b] .. lo[b+1] - 1 (none
+// if it is not split), in the list from first[b] on, and its partial sums start
+// at poff[b] (ns[b] each).  A wave per quartet of the whole list would launch
+// more than 2^32 threads, of which only the remainder runs, from 67,108,865
+// quartets on.
 constexpr int kListCls = (ZV_LMAX_T + 2) * (ZV_LMAX_T + 2);
 struct ListParts {
-    int64_t lo[kListCls + 1], poff[kListCls];
+    int64_t lo[kListCls + 1], first[kListCls], poff[kListCls];
     int ns[kListCls];
 };
 
@@ -403,10 +406,10 @@ __global__ __launch_bounds__(256) void k_reduce_list(ListParts lp, const double 
     if (x >= lp.lo[kListCls]) return;
     int b = 0;
     while (x >= lp.lo[b + 1]) b++;
-    if (lp.ns[b] <= 1) return;
     const int lane = threadIdx.x & 63;
-    const double s = wave_sum_parts(part + lp.poff[b] + (x - lp.lo[b]) * lp.ns[b], lp.ns[b], lane);
-    if (lane == 0) out[x] = s;
+    const int64_t q = x - lp.lo[b];
+    const double s = wave_sum_parts(part + lp.poff[b] + q * lp.ns[b], lp.ns[b], lane);
+    if (lane == 0) out[lp.first[b] + q] = s;
 }
 
 __global__ void k_diag_pre(int np, const double *tri, double *pre)
@@ -873,14 +876,18 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
     // stream, whose scratch memory they need.
     static_assert(ncls * ncls == kListCls, "list classes");
     ListParts lp;
-    int64_t npart = 0;
+    int64_t npart = 0, nred = 0;
     for (int b = 0; b < kListCls; b++) {
-        lp.lo[b] = lo[b];
-        lp.ns[b] = class_split(std::max<int64_t>(lo[b + 1] - lo[b], 1), bnb[b]);
+        const int64_t cnt = lo[b + 1] - lo[b];
+        lp.lo[b] = nred;
+        lp.first[b] = lo[b];
+        lp.ns[b] = class_split(std::max<int64_t>(cnt, 1), bnb[b]);
         lp.poff[b] = npart;
-        if (lp.ns[b] > 1) npart += (lo[b + 1] - lo[b]) * lp.ns[b];
+        if (lp.ns[b] <= 1) continue;
+        nred += cnt;
+        npart += cnt * lp.ns[b];
     }
-    lp.lo[kListCls] = nq;
+    lp.lo[kListCls] = nred;
     if (npart) ZV_CHECK(zv_ensure(c, c->b_part, sizeof(double) * npart));
     double *part = (double *)c->b_part.p;
     {
@@ -926,7 +933,7 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
                 ZV_HIPCHECK(c, hipStreamWaitEvent(c->stream, c->ev_join[k], 0));
             }
         if (npart) {
-            hipLaunchKernelGGL(k_reduce_list, dim3(nblk(nq, 4)), dim3(256), 0, c->stream, lp,
+            hipLaunchKernelGGL(k_reduce_list, dim3(nblk(nred, 4)), dim3(256), 0, c->stream, lp,
                                (const double *)part, dout);
             ZV_HIPCHECK(c, hipGetLastError());
         }
