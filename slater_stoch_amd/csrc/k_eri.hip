@@ -591,19 +591,25 @@ static int class_split(int64_t nq, int nbra)
                                   (target_waves + nq - 1) / nq);
 }
 
-// The class kernel of one list on stream st.
+// The class kernel of one list on stream st (a list of more than one launch is
+// never split: class_split).
 static int launch_class_on(zv_context *c, hipStream_t st, const PP &pp, QSrc S, int LB, int LK,
                            double *out, double *part, int nsplit)
 {
-    int64_t items = S.nq * nsplit;
-    if (LB <= ZV_LMAX_T && LK <= ZV_LMAX_T) {
-        if (!launch_class_t(LB, LK, nblk(items * 64, 256), st, pp, S, nsplit, out, part))
-            return zv_fail(c, ZV_ERR_STATE, "no ERI kernel for class (%d,%d)", LB, LK);
-    } else {
-        hipLaunchKernelGGL(k_eri_generic, dim3(nblk(items * 64, 64)), dim3(64), 0, st, pp, S,
-                           nsplit, out, part);
+    constexpr int64_t most = kLaunchThreads / 64;
+    for (int64_t x = 0; x < S.nq; x += most) {
+        const QSrc s{S.mode, S.qb + x, S.qk + x, std::min(S.nq - x, most)};
+        double *o = S.mode == Q_LIST ? out + x : out;
+        const int64_t items = s.nq * nsplit;
+        if (LB <= ZV_LMAX_T && LK <= ZV_LMAX_T) {
+            if (!launch_class_t(LB, LK, nblk(items * 64, 256), st, pp, s, nsplit, o, part))
+                return zv_fail(c, ZV_ERR_STATE, "no ERI kernel for class (%d,%d)", LB, LK);
+        } else {
+            hipLaunchKernelGGL(k_eri_generic, dim3(nblk(items * 64, 64)), dim3(64), 0, st, pp, s,
+                               nsplit, o, part);
+        }
+        ZV_HIPCHECK(c, hipGetLastError());
     }
-    ZV_HIPCHECK(c, hipGetLastError());
     return ZV_OK;
 }
 

@@ -749,10 +749,13 @@ struct LaunchArgs {
 
 template <int LU, int LL, int PASS> void launch_quartet(const LaunchArgs &a)
 {
-    constexpr int WPB = quartet_wpb(LU, LL, PASS);
-    hipLaunchKernelGGL((k_eri_quartet<LU, LL, PASS>), dim3((unsigned)((a.n + WPB - 1) / WPB)),
-                       dim3(64 * WPB), 0, a.st, a.sd, a.items, a.n, a.btab, a.ztab, a.sd.rows,
-                       a.sd.gu, a.sd.gl, a.part);
+    constexpr int WPB = quartet_wpb(LU, LL, PASS), most = (int)(kLaunchThreads / 64);
+    for (int i = 0, n; i < a.n; i += n) {
+        n = std::min(a.n - i, most);
+        hipLaunchKernelGGL((k_eri_quartet<LU, LL, PASS>), dim3((unsigned)((n + WPB - 1) / WPB)),
+                           dim3(64 * WPB), 0, a.st, a.sd, a.items + i, n, a.btab, a.ztab,
+                           a.sd.rows, a.sd.gu, a.sd.gl, a.part);
+    }
 }
 
 struct ClassInfo {
@@ -1255,11 +1258,13 @@ int zv_shell_run(zv_context *c, const PP &pp, const std::vector<std::pair<int, i
 int zv_shell_scatter(zv_context *c, const DevBuf &bgroup, const DevBuf &bpart, int64_t ngroups,
                      const double *pre, double *tri)
 {
-    if (ngroups <= 0) return ZV_OK;
-    hipLaunchKernelGGL(k_shell_scatter, dim3((unsigned)ngroups), dim3(256), 0, c->stream,
-                       (const ShellGroup *)bgroup.p, spd_of(c), (const double *)bpart.p, pre,
-                       tri);
-    ZV_HIPCHECK(c, hipGetLastError());
+    constexpr int64_t most = kLaunchThreads / 256;
+    for (int64_t g = 0; g < ngroups; g += most) {
+        hipLaunchKernelGGL(k_shell_scatter, dim3((unsigned)std::min(ngroups - g, most)), dim3(256),
+                           0, c->stream, (const ShellGroup *)bgroup.p + g, spd_of(c),
+                           (const double *)bpart.p, pre, tri);
+        ZV_HIPCHECK(c, hipGetLastError());
+    }
     return ZV_OK;
 }
 

@@ -154,6 +154,10 @@ int zv_ensure(zv_context *c, DevBuf &b, size_t bytes);
 // device -> host copy after the work on the context's stream; returns when done
 int zv_copy_out(zv_context *c, void *host, const void *dev, size_t bytes);
 
+// A launch of more than 2^32 - 1 threads runs only the remainder, without an
+// error: longer work lists go in slices of at most this many threads.
+constexpr int64_t kLaunchThreads = (int64_t)1 << 31;
+
 // triangle index of (P, Q), P >= Q (0-based pair indices)
 __host__ __device__ inline int64_t zv_tri(int64_t P, int64_t Q) { return P * (P + 1) / 2 + Q; }
 
