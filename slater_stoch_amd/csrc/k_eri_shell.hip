@@ -103,7 +103,6 @@ constexpr int kLaneC = 16, kStepA = 4;
 constexpr int kNgMax = 98;
 struct GTable {
     int n = 0;
-    int off[15] = {}, h0[15] = {}; // per sigma: first entry, first h
     int sig[kNgMax] = {}, h[kNgMax] = {};
 };
 constexpr GTable make_gtable(int L)
@@ -112,8 +111,6 @@ constexpr GTable make_gtable(int L)
     for (int s = 0; s < nsig(L); s++) {
         const int n = sig_n(L, s);
         const int lo = 2 * n - L > 0 ? 2 * n - L : 0;
-        g.off[s] = g.n;
-        g.h0[s] = hco(lo - 1);
         for (int h = hco(lo - 1); h < hco(n); h++) {
             g.sig[g.n] = s;
             g.h[g.n] = h;
