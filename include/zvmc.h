@@ -271,7 +271,8 @@ int zv_set_verbose(zv_context *ctx, int level);
  * the input deck); for autotuners and for tests that pin each code path.
  *  ZV_TUNE_EST_SPLIT  sample splits per estimator tile (1 = unsplit; capped
  *                     at 64, at 4 LDS stages per split and at 1 GiB of
- *                     partial sums)
+ *                     partial sums beyond the first of each block, which
+ *                     take up to 2 GiB over the blocks that run together)
  *  ZV_TUNE_MC_CHUNK   largest number of samples per estimator chunk (rounded
  *                     down to a multiple of 160, at least 160)
  *  ZV_TUNE_ERI_ITEMS  the analytic shell planner cuts a Schwarz phase into
@@ -283,9 +284,9 @@ int zv_set_verbose(zv_context *ctx, int level);
  *                     units per thread along the longer side (more, smaller
  *                     tiles for small molecules)
  * Values < 0 give ZV_ERR_ARG; the setting holds for the context's later
- * calls and changes only speed, except ZV_TUNE_EST_SPLIT and
- * ZV_TUNE_MC_CHUNK, which also change the estimator's summation order
- * (rounding only). */
+ * calls and changes speed and, by the order of sums, rounding:
+ * ZV_TUNE_EST_SPLIT, ZV_TUNE_MC_CHUNK and ZV_TUNE_EST_TILES the estimator's,
+ * ZV_TUNE_ERI_ITEMS the analytic integrals'. */
 #define ZV_TUNE_EST_SPLIT 0
 #define ZV_TUNE_MC_CHUNK 1
 #define ZV_TUNE_ERI_ITEMS 2
@@ -303,12 +304,15 @@ int zv_last_timings(const zv_context *ctx, double *ms, int64_t *launches);
 /* Per ERI kernel of the last zv_gauss_eri / zv_gauss_ijkl_list call, arrays
  * of 236.  Entries 0..35: component kernels, index 6*LB + LK (LB >= LK the
  * Hermite orders of the two AO pairs, 5 = the runtime-order kernel);
- * entries 36..235: shell kernels, index 36 + 25*v + 5*LU + LL (LU, LL the
- * orders of the uniform-side and lane-side shell pairs; v = 2*(lane batch-1)
- * + mode, lane batch 1..4, mode 0 direct, 1 wave-sum reduction).  ms: kernel milliseconds;
- * launches; units: primitive-quartet evaluations (times the lane-side
- * components for shell kernels); flops: algorithmic FP64 flops (Boys values
- * and R table once per primitive quartet, contractions per component).
+ * entries 36..235: shell kernels, index 36 + 50*pass + 5*LU + LL (LU <= LL
+ * the orders of the uniform-side and lane-side shell pairs; pass 0..3, of
+ * which only (3,4) and (4,4) have more than pass 0).  ms: kernel milliseconds;
+ * launches; units: primitive quartets (shell kernels: of shell pairs, however
+ * many components, counted with pass 0); flops: algorithmic FP64 flops.  Shell
+ * kernels: Boys values and R table once per primitive quartet (counted with
+ * pass 0) and two per multiply-add of the row sums of the pass (one per row
+ * and scaled Hermite weight that the row needs); component kernels: the
+ * contractions of each component quartet.
  * Diagnostic entry point with no counterpart in the reference (which prints
  * only a CPU time, src/two_e_slater.F90:286-287). */
 int zv_last_eri_stats(const zv_context *ctx, double *ms, int64_t *launches,

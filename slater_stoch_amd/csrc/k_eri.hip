@@ -20,7 +20,7 @@
 // the kept primitive pairs.  Primitive pairs whose Gaussian-product factor is
 // cut by the reference (exponent > 40, src/gaussian_product.F90:25, or factor
 // < 1e-15, src/give_explicit_poly_and_gaussian.F90:46) are dropped the same
-// way.  The Boys values come from the tabulated expansions (eri_device.h); at
+// way.  The Boys values come from the tabulated expansions (boys_table.h); at
 // run-time orders as in src/rint_sum.F90.
 //
 // Work layout: quartets are grouped by the Hermite orders (LB, LK) of their
@@ -575,9 +575,6 @@ static double component_flops(int LB, int LK)
     return 25.0 + 3.0 * (L + 1) + 4.0 * (HR4 - 1.0) + 2.0 * HB * HK + 2.0 * HB + 12.0;
 }
 
-// Launch one class over an explicit quartet list S, splitting bra primitive
-// pairs when there are too few quartets to fill the device.  pq and flops
-// (primitive quartets and algorithmic flops of the list) feed the statistics.
 // Split of a class launch over the bra primitive pairs, of which its longest
 // quartet has nbra: short lists are spread over up to 128 waves per quartet,
 // about 16384 waves in all (the longest waves decide: 2000 quartets 1.61 ms
@@ -626,6 +623,9 @@ static int launch_class_raw(zv_context *c, const PP &pp, QSrc S, int LB, int LK,
     return ZV_OK;
 }
 
+// Launch one class over an explicit quartet list S, splitting bra primitive
+// pairs when there are too few quartets to fill the device.  pq and flops
+// (primitive quartets and algorithmic flops of the list) feed the statistics.
 static int launch_class(zv_context *c, const PP &pp, QSrc S, int LB, int LK, double *out,
                         int nbra, double pq, double flops)
 {
@@ -877,9 +877,8 @@ int zv_run_gauss_list(zv_context *c, int64_t nq, const int *qi, const int *qk, c
     // the context's stream and its side streams, the costliest first, each on
     // the stream with the least work so far: a class of a few hundred quartets
     // ends on long waves that leave most of the chip idle (15 classes of 2000
-    // quartets: 3.25 ms one after another, 2.2 ms
-    // side by side).  Runtime orders stay on the context's
-    // stream, whose scratch memory they need.
+    // quartets: 3.25 ms one after another, 2.2 ms side by side).  Runtime orders
+    // stay on the context's stream, whose scratch memory they need.
     static_assert(ncls * ncls == kListCls, "list classes");
     ListParts lp;
     int64_t npart = 0, nred = 0;

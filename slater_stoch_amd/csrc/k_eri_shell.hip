@@ -44,8 +44,8 @@
 // the matrix form buys registers, not flops; there is no memory access in the
 // loop but the next step's rows.  Before, each lane contracted R with the E of
 // its components (passes of 1-4 components, Boys and R redone per pass, lane
-// data reloaded per uniform pair): kernel time of the 110-AO random molecule
-// 0.55 -> 0.27 s, of a 128-AO hydrocarbon 1.20 -> 0.42 s.
+// data reloaded per uniform pair): whole call on the 110-AO random molecule
+// 402 ms, now 130 ms; on a 128-AO hydrocarbon 1190 ms, now 383 ms.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -128,9 +128,10 @@ static_assert(kG.t[4].n == kNgMax, "expansion entries");
 
 // ------------------------------------------------------------------ passes
 // A class (LU, LL), LU <= LL, whose accumulators and R table do not fit in
-// the registers (256 of each kind per wave) runs in passes, each a kernel of its own over the same
-// primitive quartets: the rows r of order rho0..rho1 and the sigma groups
-// [g0, g1).  The passes of a quartet write partial sums that the scatter adds.
+// the registers (256 of each kind per wave) runs in passes, each a kernel of its
+// own over the same primitive quartets: the rows r of order rho0..rho1 and the
+// sigma groups [g0, g1).  The passes of a quartet write partial sums that the
+// scatter adds.
 struct Pass {
     int rho0, rho1, g0, g1;
 };
@@ -1202,8 +1203,9 @@ int zv_shell_run(zv_context *c, const PP &pp, const std::vector<std::pair<int, i
     // The buckets write disjoint partial sums, so they run side by side on
     // the context's stream and its side streams (a bucket's last items leave
     // CUs idle that the next bucket fills), joined back before the scatter.
-    // Largest planned cost first, each to the stream with the least planned
-    // cost so far.
+    // Most counted flops first, each to the stream with the fewest so far (the
+    // count of a later pass leaves out the Boys values and R rows that it
+    // repeats, so the passes of (3, 4) and (4, 4) come late).
     // bucket b = 50 pass + 5 LU + LL: statistics slot 36 + b
     static_assert(36 + kNB <= ZV_NSTAT, "statistics slots");
     constexpr int NST = 1 + zv_context::NSIDE;

@@ -1065,7 +1065,8 @@ static int pick_blocks(zv_context *c, int nbl, int64_t npts, int64_t chunk)
 // leave most CUs idle while each tile walks a whole block, so the block's
 // stages are split over up to 64 workgroups per tile, aiming at about 1024
 // workgroups in all (about one resident round: 4 per CU by LDS), with at
-// least 4 stages per split and at most 1 GiB of partial rows.
+// least 4 stages per split and at most 1 GiB of partial rows beyond the first
+// of each block (those are pick_blocks').
 static int pick_split(zv_context *c, int mblock, int precision, int64_t tiles, int nb)
 {
     if (tiles <= 0) return 1;

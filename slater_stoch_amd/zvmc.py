@@ -328,7 +328,8 @@ class Engine:
     def eri_stats(self):
         """Per ERI kernel of the last gauss_eri / gauss_ijkl: {key: dict(ms,
         launches, units, flops)} with key ("component", LB, LK) or ("shell",
-        LU, LL, pass + 1, False)."""
+        LU, LL, pass + 1, False), passes from 0; the last field is always
+        False."""
         n_stat = 236
         ms, un, fl = np.zeros(n_stat), np.zeros(n_stat), np.zeros(n_stat)
         n = np.zeros(n_stat, np.int64)
